@@ -15,8 +15,8 @@ LIBDIR = os.path.join(HERE, "lib")
 LIB = os.path.join(LIBDIR, "libstroemung_hip.so")
 BUILD = os.path.join(HERE, "_build")
 
-SOURCES = ["api.hip", "kernels_step.hip", "kernels_pressure.hip", "kernels_rbtb.hip",
-           "kernels_learn.hip", "nn_kernels.hip", "nn_net.hip", "kernels_view.hip",
+SOURCES = ["api.hip", "kernels_step.hip", "kernels_pressure.hip", "kernels_lex.hip",
+           "kernels_rbtb.hip", "kernels_learn.hip", "nn_kernels.hip", "nn_net.hip", "kernels_view.hip",
            "kernels_sync.hip"]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")

@@ -68,6 +68,8 @@ struct stm_ctx {
     bool any_rb = false, any_lex = false;
     double *u = nullptr, *v = nullptr, *p = nullptr, *f = nullptr, *g = nullptr, *rhs = nullptr;
     double* scratch = nullptr;
+    double* lexwork = nullptr;     // pipelined lexicographic solve: its channels' scratch
+    int64_t* d_lexoff = nullptr;   // ... and each channel's offset in it
     double* p2 = nullptr;          // second pressure buffer of the blocked solver
     uint8_t* flags = nullptr;
     ChanDesc* d_cd = nullptr;
@@ -267,6 +269,7 @@ ChanDesc make_desc(const HostChan& c) {
     d.check_every = q.check_every > 0 ? q.check_every : 1;
     d.tb0 = c.tb0;
     d.ntb = c.ntb;
+    d.lex_class = lex_class(d.nx, d.ny);
     d.delx = q.delx;
     d.dely = q.dely;
     d.gamma = q.gamma;
@@ -1071,6 +1074,45 @@ int check_net(stm_ctx* ctx, stm_net* net, uint32_t f) {
     return STM_OK;
 }
 
+// Scratch of the pipelined lexicographic solve, made at the first solve that
+// has a lexicographic channel: every channel that fits an instance has its
+// part (a channel may switch solvers later).
+int lex_buffers(stm_ctx* ctx) {
+    if (ctx->lexwork) return STM_OK;
+    std::vector<int64_t> off;
+    int64_t n = 0;
+    for (const HostChan& c : ctx->chans) {
+        off.push_back(n);
+        n += round_up(lex_work_doubles(lex_class((int)c.nx, (int)c.ny), (int)c.nx, (int)c.ny), 16);
+    }
+    if (n == 0) return STM_OK;
+    if (!ctx->d_lexoff) HIPCHK(ctx, hipMalloc(&ctx->d_lexoff, sizeof(int64_t) * off.size()));
+    HIPCHK(ctx, hipMemcpyAsync(ctx->d_lexoff, off.data(), sizeof(int64_t) * off.size(),
+                               hipMemcpyHostToDevice, ctx->stream));
+    HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
+    HIPCHK(ctx, hipMalloc(&ctx->lexwork, sizeof(double) * (size_t)n));
+    return STM_OK;
+}
+
+// The lexicographic channels: a launch per class in use.
+int stage_lex(stm_ctx* ctx) {
+    int rc = lex_buffers(ctx);
+    if (rc) return rc;
+    std::vector<bool> used(N_LEX_CLASSES + 1, false);
+    for (const HostChan& c : ctx->chans)
+        if (c.prm.solver == STM_SOLVER_LEX) used[1 + lex_class((int)c.nx, (int)c.ny)] = true;
+    for (int k = 0; k < N_LEX_CLASSES; k++)
+        if (used[1 + k])
+            LAUNCH("lex_solve", launch_lex_pipe(ctx->stream, k, nch(ctx), ctx->d_cd, ctx->d_cs,
+                                                ctx->d_lexoff, ctx->flags, ctx->rhs, ctx->p,
+                                                ctx->lexwork));
+    if (used[0])
+        LAUNCH("lex_solve", launch_lex_solve(ctx->stream, nch(ctx), ctx->d_cd, ctx->d_cs,
+                                             ctx->d_be, ctx->flags, ctx->rhs, ctx->p,
+                                             ctx->scratch));
+    return STM_OK;
+}
+
 // POISSON: the rhs statistics, tol2 and the per-channel flags, then each
 // channel's solver.
 int stage_solve(stm_ctx* ctx) {
@@ -1078,10 +1120,7 @@ int stage_solve(stm_ctx* ctx) {
     if (rc) return rc;
     LAUNCH("solve_begin", launch_solve_begin(ctx->stream, nch(ctx), ctx->d_cd, ctx->d_cs,
                                              ctx->d_part, ctx->d_active));
-    if (ctx->any_lex)
-        LAUNCH("lex_solve", launch_lex_solve(ctx->stream, nch(ctx), ctx->d_cd, ctx->d_cs,
-                                             ctx->d_be, ctx->flags, ctx->rhs, ctx->p,
-                                             ctx->scratch));
+    if (ctx->any_lex && (rc = stage_lex(ctx))) return rc;
     if (!ctx->any_rb) return STM_OK;
     if (ctx->cnet || (ctx->lnet && ctx->lcycles > 0)) return phased_solve(ctx);
     return blocked_solve(ctx, 1);
@@ -1205,7 +1244,7 @@ void stm_destroy(stm_ctx* ctx) {
     drain(ctx);
     for (hipEvent_t e : ctx->free_events) hipEventDestroy(e);
     void* bufs[] = {ctx->u, ctx->v, ctx->p, ctx->f, ctx->g, ctx->rhs, ctx->scratch, ctx->p2,
-                    ctx->flags, ctx->d_cd, ctx->d_cs, ctx->d_be, ctx->d_restore, ctx->d_tiles,
+                    ctx->lexwork, ctx->d_lexoff, ctx->flags, ctx->d_cd, ctx->d_cs, ctx->d_be, ctx->d_restore, ctx->d_tiles,
                     ctx->d_part, ctx->d_active, ctx->d_tbpart, ctx->d_tb, ctx->d_codes, ctx->d_tbc, ctx->d_lc, ctx->lres,
                     ctx->lcf, ctx->lprev, ctx->lprev2, ctx->lsnap, ctx->lrc, ctx->lmc, ctx->d_cpart, ctx->d_map,
                     ctx->d_inv, ctx->d_live, ctx->d_rgba};

@@ -47,6 +47,21 @@ void launch_initial_norm(hipStream_t, int nchan, const ChanDesc*, ChanState*, co
 void launch_lex_solve(hipStream_t, int nchan, const ChanDesc*, ChanState*, const BEntry*,
                       const uint8_t* flags, const double* rhs, double* p, double* scratch);
 
+// kernels_lex.hip: the lexicographic solve with several sweeps in flight
+struct LexClass {
+    int row;        // most rows (ring included) a channel of the class has
+    int full;       // sweeps whose squares are kept at once
+    int codes;      // bytes of a diagonal's codes
+};
+extern const LexClass LEX_CLASSES[];
+extern const int N_LEX_CLASSES;
+int lex_class(int nx, int ny);
+int64_t lex_work_doubles(int cls, int nx, int ny);   // scratch of one channel
+// The channels of class `cls`; work_off: each channel's element offset in work.
+void launch_lex_pipe(hipStream_t, int cls, int nchan, const ChanDesc*, ChanState*,
+                     const int64_t* work_off, const uint8_t* flags, const double* rhs, double* p,
+                     double* work);
+
 // kernels_rbtb.hip: temporally blocked red-black SOR
 struct TbVariant {
     int k;          // sweeps per launch

@@ -1,0 +1,674 @@
+// The reference's lexicographic SOR (src/simulation.rs:239-285) with many
+// sweeps in flight, bit-exact.
+//
+// A sweep visits the interior cells x-major in place, so cell (x, y) reads the
+// new W and N and the old E and S values: the anti-diagonals x + y = d, taken
+// in increasing d, give exactly those reads.  One sweep is a chain of nx + ny
+// dependent diagonals, and on one diagonal at a time a workgroup waits for
+// latency with most lanes idle.  But sweep k + 1 may follow sweep k a few
+// diagonals behind, so a workgroup runs NSLOT sweeps at once: slot s does
+// sweeps s, s + NSLOT, ..., each LAG diagonals behind the slot before it.
+//
+// A slot is LW lanes; lane l owns the RPL rows y = RPL * l .. + RPL - 1 (ring
+// rows included), and takes cell (d - y, y) of each of them on diagonal d:
+// independent cells.  Everything a cell needs is in registers: W is the row's
+// own last result, N the last result of the row above, E and S the row's own
+// and the row below's value on the next diagonal before the sweep (a DPP shift
+// where the row belongs to the next lane).  A slot hands its results to the
+// next through a three-diagonal LDS ring, so a step is one barrier.  Slot 0
+// reads the solve's input (A) and later the last slot's results (C, a round of
+// steps behind); the batch's last sweep writes B.  A ghost's pressure is the
+// copy of its fluid neighbours before the sweep (src/grid/mod.rs:343-412);
+// those are the slot's inputs of the two neighbouring diagonals, so each slot
+// forms the ghosts of its own sweep while its input passes.
+//
+// The stopping rule is tested after every sweep, so sweeps in flight are
+// speculative: A stays as it was until the batch is accepted.  Two ways:
+//   LIGHT  The squares of the residual are added in order, so the sum is at
+//          least as large as any one of them (rounding is monotone): a sweep
+//          in which one square alone reaches the bound has not met the rule.
+//          A quarter of the diagonals are looked at; when every sweep of the
+//          batch shows such a square, all of them count.  The norm the solve
+//          returns, its last sweep's, is formed from the final field.
+//   FULL   Every sweep leaves all its squares (T), the norms are summed in the
+//          reference's order and tested one after another; if sweep r of the
+//          batch meets the rule, the batch is repeated from A with r + 1 sweeps.
+// A solve starts LIGHT when the channel's last one ran to its limit (or there
+// was none) and goes on FULL from the first batch that cannot be shown; batch
+// lengths start at the last solve's and double, so little is swept for nothing.
+//
+// Fields are kept diagonal-major (row d + LEX_PAD of ROW = LW * RPL values,
+// entry y), so a diagonal is one contiguous access.  LEX_PAD rows before the
+// first and after the last diagonal hold no cells: they are 0 with code 0, a
+// slot whose diagonal is outside the grid reads them and passes zeros on.
+#include <hip/hip_runtime.h>
+
+#include "kernels.h"
+#include "stm_internal.h"
+
+namespace stm {
+
+namespace {
+
+constexpr int LAG = 3;
+
+// Codes of the diagonal-major flags: the fluid neighbours a ghost copies (one
+// bit, or a vertical and a horizontal one whose mean it takes), whether the
+// sweep updates the cell, and whether it is an interior cell.
+enum : uint32_t { G_N = 1, G_S = 2, G_E = 4, G_W = 8, C_UPD = 16, C_IN = 32 };
+
+__device__ __forceinline__ uint32_t lex_code(uint8_t flag, bool inner) {
+    const uint32_t in = inner ? C_IN : 0u;
+    if (flag_fluid(flag)) return inner ? in | C_UPD : 0u;
+    switch (flag_edge(flag)) {
+    case E_N: return in | G_N;
+    case E_NE: return in | G_N | G_E;
+    case E_E: return in | G_E;
+    case E_SE: return in | G_S | G_E;
+    case E_S: return in | G_S;
+    case E_SW: return in | G_S | G_W;
+    case E_W: return in | G_W;
+    case E_NW: return in | G_N | G_W;
+    default: return in;
+    }
+}
+
+// Lane i takes lane i - 1's value (UP) or lane i + 1's: a DPP wave shift.
+// The lane at the wave's end gets 0.0.
+template <bool UP>
+__device__ __forceinline__ double lane_shift(double v) {
+    constexpr int CTRL = UP ? 0x138 : 0x130;
+    const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), CTRL, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), CTRL, 0xf, 0xf, true);
+    return __hiloint2double(hi, lo);
+}
+
+// a / b, correctly rounded, for a divisor that stays the same: with y = RN(1/b)
+// and yl = RN(1/b - y), q = a y + a yl is within one ulp of a / b, and one
+// fused correction rounds it correctly (Markstein, IBM J. Res. Dev. 34 (1990);
+// Brisebarre, Muller, Raina, IEEE Trans. Comput. 53 (2004)): four dependent
+// operations instead of the general divide's two scalings, reciprocal, four
+// Newton steps and fix-up.  It holds while nothing over- or underflows, which
+// the bounds below secure (divisible), and while b's significand is not all
+// ones; EXACT takes the general divide.  The sign is a's (b > 0), so a zero
+// keeps its sign.
+struct Divisor {
+    double b, y, yl;
+};
+__device__ __forceinline__ Divisor make_divisor(double b) {
+    Divisor v;
+    v.b = b;
+    v.y = 1.0 / b;
+    v.yl = __builtin_fma(-b, v.y, 1.0) * v.y;
+    return v;
+}
+__device__ __forceinline__ bool divisible(double b) {
+    const uint64_t m = (uint64_t)__double_as_longlong(b) & 0xfffffffffffffull;
+    return b >= 0x1p-30 && b <= 0x1p30 && m != 0xfffffffffffffull;
+}
+template <bool EXACT>
+__device__ __forceinline__ double quotient(double a, const Divisor& v) {
+    if constexpr (EXACT) return a / v.b;
+    double q = __builtin_fma(a, v.y, a * v.yl);
+    q = __builtin_fma(__builtin_fma(-v.b, q, a), v.y, q);
+    return __hiloint2double((__double2hiint(q) & 0x7fffffff) |
+                                (__double2hiint(a) & (int)0x80000000), __double2loint(q));
+}
+// A nonzero pressure (or right-hand side) below 2^-840 sends its batch to the
+// general divide.  Without one every sum and difference of two pressures is a
+// multiple of 2^-893, so no dividend but 0 is below that and no product or
+// remainder of the quotient is subnormal; and a result of the update is 0 or
+// at least 2^-1019 (omega in 2^-10 .. 2^10), so the upper word alone tells a
+// tiny one from 0: `tiny_word` is below TINY_WORD for tiny results only.
+// Towards infinity the quotient is right until something overflows; then it is
+// NaN where the divide may be infinite, and a pressure that is not finite
+// stays so (it is tested at the end of a batch, and so are the norms).
+__device__ __forceinline__ bool tiny(double p) { return (fabs(p) < 0x1p-840) & (p != 0.0); }
+constexpr uint32_t TINY_WORD = ((uint32_t)(1023 - 840) << 21) - 1u;
+__device__ __forceinline__ uint32_t tiny_word(double p) {
+    return ((uint32_t)__double2hiint(p) << 1) - 1u;
+}
+__device__ __forceinline__ bool finite(double p) { return fabs(p) < __builtin_inf(); }
+
+// A lane's RPL values, and its codes (CODES bytes).
+typedef double double2u __attribute__((ext_vector_type(2), aligned(8)));
+template <int RPL>
+__device__ __forceinline__ void load_row(const void* p, double (&v)[RPL]) {
+    const double* q = static_cast<const double*>(p);
+#pragma unroll
+    for (int i = 0; i + 1 < RPL; i += 2) {
+        const double2u t = *reinterpret_cast<const double2u*>(q + i);
+        v[i] = t.x;
+        v[i + 1] = t.y;
+    }
+    if constexpr (RPL % 2 != 0) v[RPL - 1] = q[RPL - 1];
+}
+template <int RPL>
+__device__ __forceinline__ void store_row(void* p, const double (&v)[RPL]) {
+    double* q = static_cast<double*>(p);
+#pragma unroll
+    for (int i = 0; i + 1 < RPL; i += 2)
+        *reinterpret_cast<double2u*>(q + i) = double2u{v[i], v[i + 1]};
+    if constexpr (RPL % 2 != 0) q[RPL - 1] = v[RPL - 1];
+}
+constexpr int code_bytes(int rpl) { return rpl <= 4 ? 4 : 8; }
+template <int RPL>
+__device__ __forceinline__ uint64_t load_codes(const void* p) {
+    if constexpr (code_bytes(RPL) == 4) return *static_cast<const uint32_t*>(p);
+    else return *static_cast<const uint64_t*>(p);
+}
+
+// Sum of acc and t of the row's lanes 0 .. 15, added one after another in that
+// order by every lane of the row of 16 (a broadcast within the row and a fused
+// multiply by one, which rounds as the addition does).
+__device__ __forceinline__ double add_row(double acc, double t) {
+#define STM_ADD_LANE(k) "v_fmac_f64_dpp %0, %1, %2 row_newbcast:" #k " row_mask:0xf bank_mask:0xf\n\t"
+    asm volatile("s_nop 1\n\t"
+                 STM_ADD_LANE(0) STM_ADD_LANE(1) STM_ADD_LANE(2) STM_ADD_LANE(3)
+                 STM_ADD_LANE(4) STM_ADD_LANE(5) STM_ADD_LANE(6) STM_ADD_LANE(7)
+                 STM_ADD_LANE(8) STM_ADD_LANE(9) STM_ADD_LANE(10) STM_ADD_LANE(11)
+                 STM_ADD_LANE(12) STM_ADD_LANE(13) STM_ADD_LANE(14) STM_ADD_LANE(15)
+                 : "+v"(acc) : "v"(t), "v"(1.0));
+#undef STM_ADD_LANE
+    return acc;
+}
+
+// One workgroup's view of its channel: its buffers as byte offsets from `base`
+// (32 bits: lex_class keeps a channel's scratch below 4 GB).
+struct LexWork {
+    char* base;
+    uint32_t a, b, c, rhs, t, codes;   // codes: code_bytes per lane, the others 8 per entry
+    uint32_t bytes;           // of one diagonal-major field
+    int dmax;                 // the last diagonal, nx + ny - 2
+    int ny;
+    double omw, mid;
+    Divisor dx2, dy2;
+};
+
+enum : int { LIGHT = 0, FULL = 1, FULL_DIV = 2 };   // FULL_DIV: FULL with the general divide
+
+template <int LW, int RPL, int NSLOT, int TS>
+struct Pipe {
+    static constexpr int ROW = LW * RPL, NT = LW * NSLOT;
+    static constexpr uint32_t ROWB = ROW * 8, ROWC = LW * code_bytes(RPL);   // bytes of a row
+    static constexpr int Q = 3;              // steps of a group; loads are a group ahead
+    static constexpr int RING = NSLOT * ROW;
+    static_assert(LAG == Q && TS <= NSLOT, "slots change sweeps between groups");
+    // rows of the pads a slot reads and writes: -2 - 6 - 1 and up to
+    // -2 + 3 * last() + 2 + 2 <= dmax + 7
+    static_assert(LEX_PAD >= 10, "pads");
+
+    // Groups of a sweep, and of a round: a slot starts its next sweep a round
+    // after this one.  Slot 0 uses row q of C in step q of its round and loads
+    // it a group earlier; the last slot stores row q in step 3 (NSLOT - 1) + 2
+    // + q of the round before: at least 13 steps earlier, and it waits for its
+    // stores once a group.
+    __device__ static __forceinline__ int last(const LexWork& w) { return (w.dmax + 3 + Q - 1) / Q; }
+    __device__ static __forceinline__ int round(const LexWork& w) { return max(last(w) + 1, NSLOT + 5); }
+
+    struct Result {
+        int mode;
+        bool bad;      // a pressure the fixed quotient is not right for
+        bool open;     // LIGHT: a sweep that may have met the stopping rule
+    };
+
+    // Sweeps 0 .. n - 1 from A; the last one's result in B.  LIGHT: sweeps
+    // below `need` are shown not to have met the rule by a square of `bound`
+    // or more.  FULL: n <= TS, the squares of sweep k in T, field k.
+    template <int MODE>
+    __device__ static __forceinline__ Result sweeps(const LexWork& w, int n, int need,
+                                                    double bound, double* ring) {
+        constexpr bool EXACT = MODE == FULL_DIV;
+        // (a wave's slot is uniform when a slot is a wave)
+        const int slot = LW == 64 ? __builtin_amdgcn_readfirstlane(threadIdx.x / LW)
+                                  : threadIdx.x / LW;
+        const int y0 = (threadIdx.x % LW) * RPL;
+        const int glast = last(w), ground = round(w);
+        const int groups = (n - 1) / NSLOT * ground + (n - 1) % NSLOT + glast;
+        Result res{MODE, false, false};
+#pragma unroll
+        for (int i = 0; i < 3 * RPL; i++) ring[i * NT + threadIdx.x] = 0.0;
+        __syncthreads();
+        // waves without a slot of the batch only keep the barriers
+        if ((int)(threadIdx.x & ~63u) / LW >= n) {
+            for (int e = 0; e < groups * Q; e++) asm volatile("s_barrier" ::: "memory");
+            return res;
+        }
+        const bool rows_in = y0 < w.ny;      // lanes below the last row: zeros with code 0
+        const bool first = slot == 0;
+        const uint32_t yb = (uint32_t)y0 * 8u;
+        const double* in = ring + (slot > 0 ? slot - 1 : 0) * ROW + y0;
+        double* out = ring + slot * ROW + y0;
+        // the slot's group g of its sweep k: diagonals d = -2 + 3 g .. + 2.
+        // Before its first and after its last group a slot is on the pads.
+        int g = -slot, k = slot;
+        auto row0 = [&](int gg) -> uint32_t {   // row -2 + 3 gg of a field
+            return (uint32_t)(min(max(gg, -2), glast) * Q + (LEX_PAD - 2));
+        };
+        // this lane's codes of row r
+        auto code_at = [&](uint32_t r) -> uint32_t {
+            return w.codes + r * ROWC + (threadIdx.x % LW) * code_bytes(RPL);
+        };
+        // what slot 0 reads in sweep kk
+        auto from = [&](int kk, uint32_t r0) -> uint32_t {
+            return (kk == 0 ? w.a : w.c) + (r0 + 2) * ROWB + yb;
+        };
+        const bool wave0 = __builtin_amdgcn_readfirstlane(threadIdx.x) < 64;   // holds slot 0
+        double raw0[RPL], raw1[RPL];         // inputs of diagonals d, d + 1
+        double in0[RPL];                     // diagonal d with its ghosts formed
+        double o1[RPL], dxp[RPL], dvp[RPL], rp[RPL];   // diagonal d - 1: result, its differences
+                                                       // to W and N, rhs
+        uint64_t code0 = 0, codep = 0;       // codes of diagonals d, d - 1
+        double aq[Q][RPL], rq[Q][RPL];       // slot 0's input of d + 2, rhs of d
+        uint64_t cq[Q];                      // codes of d + 1
+#pragma unroll
+        for (int i = 0; i < RPL; i++)
+            raw0[i] = raw1[i] = in0[i] = o1[i] = dxp[i] = dvp[i] = rp[i] = 0.0;
+        {
+            const uint32_t r0 = row0(g), f0 = from(k, r0);
+#pragma unroll
+            for (int j = 0; j < Q; j++) {
+                if (wave0) load_row<RPL>(w.base + (f0 + j * ROWB), aq[j]);
+                load_row<RPL>(w.base + (w.rhs + r0 * ROWB + yb + j * ROWB), rq[j]);
+                cq[j] = load_codes<RPL>(w.base + (code_at(r0) + (j + 1) * ROWC));
+            }
+        }
+        uint32_t small = ~0u;                // the least tiny_word
+        bool shown = false;                  // LIGHT: this lane's square for sweep k
+        auto slot_any = [&](bool v) -> bool {   // some lane of the slot
+            const uint64_t m = __ballot(v);
+            const int base = (threadIdx.x & 63) / LW * LW;
+            return LW == 64 ? m != 0 : ((m >> base) & ((1ull << (LW & 63)) - 1ull)) != 0;
+        };
+        for (int e = 0; e < groups; e++) {
+            const uint32_t r0 = row0(g);
+            int gn = g + 1, kn = k;
+            if (gn == ground) {
+                gn = 0;
+                kn = k + NSLOT;
+            }
+            const uint32_t rn0 = row0(gn), fn0 = from(kn, rn0);
+            const bool final_sweep = k == n - 1;
+            const bool keep = rows_in & (final_sweep | ((slot == NSLOT - 1) & (k < n)));
+            const uint32_t ob = (final_sweep ? w.b : w.c) + r0 * ROWB + yb;
+            const uint32_t tb = w.t + (uint32_t)min(slot, TS - 1) * w.bytes + (r0 - 1) * ROWB + yb;
+            const uint32_t rb = w.rhs + rn0 * ROWB + yb, cb = code_at(rn0) + ROWC;
+            const bool keep_t = rows_in & (k < n);
+#pragma unroll
+            for (int j = 0; j < Q; j++) {
+                // the input of diagonal d + 2: the previous slot's result of the
+                // last step
+                double raw2[RPL];
+                load_row<RPL>(in + j * RING, raw2);
+                if (wave0)
+#pragma unroll
+                    for (int i = 0; i < RPL; i++) raw2[i] = first ? aq[j][i] : raw2[i];
+                // ghosts of diagonal d + 1
+                double in1[RPL];
+                const uint64_t code1 = cq[j];
+                {
+                    const double un = lane_shift<true>(raw0[RPL - 1]);
+                    const double dn = lane_shift<false>(raw2[0]);
+                    constexpr uint64_t HORZ = 0x0101010101010101ull * (G_E | G_W);
+                    const bool full = __ballot((code1 & HORZ) != 0) != 0;   // uniform
+#pragma unroll
+                    for (int i = 0; i < RPL; i++) {
+                        const uint32_t c = (uint32_t)(code1 >> (8 * i));
+                        const double vn = i > 0 ? raw0[i > 0 ? i - 1 : 0] : un;
+                        const double vs = i + 1 < RPL ? raw2[i + 1 < RPL ? i + 1 : i] : dn;
+                        const double v = (c & G_N) ? vn : ((c & G_S) ? vs : raw1[i]);
+                        in1[i] = v;
+                        if (full) {   // copies across, and means
+                            const double h = (c & G_E) ? raw2[i] : raw0[i];
+                            const bool vert = (c & (G_N | G_S)) != 0;
+                            const double m = vert ? (v + h) * 0.5 : h;
+                            in1[i] = (c & (G_E | G_W)) ? m : v;
+                        }
+                    }
+                }
+                // the update of diagonal d (src/simulation.rs:266-270)
+                double o[RPL], nb[RPL];
+                {
+                    const double un = lane_shift<true>(o1[RPL - 1]);
+                    const double dn = lane_shift<false>(in1[0]);
+#pragma unroll
+                    for (int i = 0; i < RPL; i++) {
+                        nb[i] = i > 0 ? o1[i > 0 ? i - 1 : 0] : un;
+                        const double s = i + 1 < RPL ? in1[i + 1 < RPL ? i + 1 : i] : dn;
+                        const double lap = quotient<EXACT>(in1[i] + o1[i], w.dx2) +
+                                           quotient<EXACT>(s + nb[i], w.dy2);
+                        const double v = (w.omw * in0[i]) + (w.mid * (lap - rq[j][i]));
+                        o[i] = ((uint32_t)(code0 >> (8 * i)) & C_UPD) ? v : in0[i];
+                        if constexpr (!EXACT) small = min(small, tiny_word(o[i]));
+                    }
+                }
+                store_row<RPL>(out + (j + 1) % 3 * RING, o);
+                // the residual of diagonal d - 1 (src/math.rs:176-186): c - W of
+                // a cell is E - c of the cell before it, c - N is S - c of the
+                // cell above
+                if (MODE != LIGHT || j == 0 || j == Q - 1) {
+                    double dx[RPL], dv[RPL];
+#pragma unroll
+                    for (int i = 0; i < RPL; i++) {
+                        dx[i] = o[i] - o1[i];
+                        dv[i] = o[i] - nb[i];
+                    }
+                    if (MODE != LIGHT || j == 0) {
+                        double tt[RPL];
+                        const double dn = lane_shift<false>(dv[0]);
+#pragma unroll
+                        for (int i = 0; i < RPL; i++) {
+                            const double sc = i + 1 < RPL ? dv[i + 1 < RPL ? i + 1 : i] : dn;
+                            const double r = (quotient<EXACT>(dx[i] - dxp[i], w.dx2) +
+                                              quotient<EXACT>(sc - dvp[i], w.dy2)) - rp[i];
+                            tt[i] = r * r;
+                            if (MODE == LIGHT)
+                                shown |= (((uint32_t)(codep >> (8 * i)) & C_IN) != 0) &
+                                         (tt[i] >= bound);
+                        }
+                        if (MODE != LIGHT && keep_t)
+                            store_row<RPL>(w.base + (tb + j * ROWB), tt);
+                    }
+#pragma unroll
+                    for (int i = 0; i < RPL; i++) {
+                        dxp[i] = dx[i];
+                        dvp[i] = dv[i];
+                        rp[i] = rq[j][i];
+                    }
+                }
+                if (keep) {
+                    store_row<RPL>(w.base + (ob + j * ROWB), o);
+                    if (!EXACT && final_sweep)
+#pragma unroll
+                        for (int i = 0; i < RPL; i++) res.bad |= !finite(o[i]);
+                }
+                // the stores before this group's last step are done (the loads
+                // this also waits for are nearly a group old)
+                if (MODE == LIGHT && j == Q - 1) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+                // on to the next diagonal
+#pragma unroll
+                for (int i = 0; i < RPL; i++) {
+                    raw0[i] = raw1[i];
+                    raw1[i] = raw2[i];
+                    in0[i] = in1[i];
+                    o1[i] = o[i];
+                }
+                codep = code0;
+                code0 = code1;
+                if (wave0) load_row<RPL>(w.base + (fn0 + j * ROWB), aq[j]);
+                load_row<RPL>(w.base + (rb + j * ROWB), rq[j]);
+                cq[j] = load_codes<RPL>(w.base + (cb + j * ROWC));
+                // the ring's writes are done before the others read them; global
+                // loads and stores stay in flight
+                asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            }
+            if (MODE == LIGHT && __ballot(kn != k) != 0) {   // a slot of the wave ends its sweep
+                const bool any = slot_any(shown);
+                res.open |= (kn != k) & (k < need) & !any;
+                shown = shown & (kn == k);
+            }
+            g = gn;
+            k = kn;
+        }
+        res.bad |= small < TINY_WORD;
+        if (MODE == LIGHT) {
+            const bool any = slot_any(shown);
+            // a slot that has gone round waits for a sweep past the batch's last
+            res.open |= (k < need) & !any;
+        }
+        return res;
+    }
+
+    // The sum from 0.0 of a field's squares over the interior, x-major, by a
+    // row of 16 lanes: U * 16 terms are loaded (that many ahead) and added one
+    // by one.  Places past the end add +0.0, which changes no sum of squares.
+    // `linear`: the squares are in that order in memory (as `squares` leaves
+    // them), else diagonal-major.
+    static constexpr int U = 8;
+    __device__ static __forceinline__ double norm_sum(const char* t, int nxi, int nyi,
+                                                      bool linear) {
+        constexpr int CHUNK = U * 16;
+        const int lane = threadIdx.x & 15;
+        const int n = nxi * nyi;
+        const int sx = CHUNK / nyi, sy = CHUNK - sx * nyi;
+        int x[U], y[U];
+        double v[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int k = u * 16 + lane;
+            x[u] = 1 + k / nyi;
+            y[u] = 1 + k - (k / nyi) * nyi;
+        }
+        auto gather = [&]() {
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const int xc = min(x[u], nxi);
+                const uint32_t at = linear ? (uint32_t)((xc - 1) * nyi + y[u] - 1) * 8u
+                                           : (uint32_t)(xc + y[u] + LEX_PAD) * ROWB + y[u] * 8u;
+                const double q = *reinterpret_cast<const double*>(t + at);
+                v[u] = x[u] <= nxi ? q : 0.0;
+                x[u] += sx;
+                y[u] += sy;
+                if (y[u] > nyi) {
+                    y[u] -= nyi;
+                    x[u]++;
+                }
+            }
+        };
+        double acc = 0.0;
+        gather();
+        for (int k = 0; k < n; k += CHUNK) {
+            double c[U];
+#pragma unroll
+            for (int u = 0; u < U; u++) c[u] = v[u];
+            gather();
+#pragma unroll
+            for (int u = 0; u < U; u++) acc = add_row(acc, c[u]);
+        }
+        return acc;
+    }
+
+    // The squares of the residual of the field at `p` (every interior cell;
+    // the general divide) to the start of T in the norm's order.
+    __device__ static __forceinline__ void squares(const LexWork& w, uint32_t p, int nxi, int nyi) {
+        const int n = (nxi + nyi - 1) * ROW;   // diagonals 2 .. nxi + nyi
+        for (int k = threadIdx.x; k < n; k += NT) {
+            const int y = k % ROW, x = 2 + k / ROW - y;
+            if (x < 1 || x > nxi || y < 1 || y > nyi) continue;
+            const uint32_t at = (uint32_t)(x + y + LEX_PAD) * ROWB + y * 8u;
+            const double* q = reinterpret_cast<const double*>(w.base + (p + at));
+            const double c = q[0];
+            const double a = ((q[ROW] - c) - (c - q[-ROW])) / w.dx2.b;
+            const double b = ((q[ROW + 1] - c) - (c - q[-ROW - 1])) / w.dy2.b;
+            const double r = (a + b) - *reinterpret_cast<const double*>(w.base + (w.rhs + at));
+            *reinterpret_cast<double*>(w.base + (w.t + (uint32_t)((x - 1) * nyi + y - 1) * 8u)) = r * r;
+        }
+    }
+};
+
+}  // namespace
+
+// Class of a channel: which instance solves it; -1 (k_lex_solve) with more
+// rows than a wave can own, or beyond the 32-bit offsets.
+int lex_class(int nx, int ny) {
+    for (int c = 0; c < N_LEX_CLASSES; c++)
+        if (ny <= LEX_CLASSES[c].row) return lex_work_doubles(c, nx, ny) < (1ll << 29) ? c : -1;
+    return -1;
+}
+
+// A, B, C, rhs, the squares of the FULL sweeps, the codes.
+int64_t lex_work_doubles(int cls, int nx, int ny) {
+    if (cls < 0) return 0;
+    const int64_t rows = (int64_t)nx + ny - 1 + 2 * LEX_PAD, cells = rows * LEX_CLASSES[cls].row;
+    return cells * (4 + LEX_CLASSES[cls].full) + rows * LEX_CLASSES[cls].codes / 8;
+}
+
+constexpr int LIGHT_MOST = 256;   // sweeps of a LIGHT batch
+
+template <int CLASS, int LW, int RPL, int NSLOT, int TS>
+__global__ void __launch_bounds__(LW * NSLOT)
+k_lex_pipe(const ChanDesc* __restrict__ cd, ChanState* __restrict__ cs,
+           const int64_t* __restrict__ work_off, const uint8_t* __restrict__ flags,
+           const double* __restrict__ rhs, double* __restrict__ p, double* work)
+{
+    using P = Pipe<LW, RPL, NSLOT, TS>;
+    constexpr int ROW = P::ROW, NT = P::NT;
+    __shared__ __attribute__((aligned(16))) double ring[3 * P::RING];
+    __shared__ double snorm[TS];
+    const ChanDesc d = cd[blockIdx.x];
+    if (d.solver != SOLVER_LEX || d.lex_class != CLASS) return;
+    ChanState& s = cs[blockIdx.x];
+    const int tid = threadIdx.x;
+    const int nxi = d.nx - 2, nyi = d.ny - 2;
+    LexWork w;
+    w.dmax = d.nx + d.ny - 2;
+    w.ny = d.ny;
+    w.omw = d.omw;
+    w.mid = d.mid;
+    w.dx2 = make_divisor(d.delx2);
+    w.dy2 = make_divisor(d.dely2);
+    const uint32_t cells = (uint32_t)(w.dmax + 1 + 2 * LEX_PAD) * ROW;
+    w.bytes = cells * 8;
+    w.base = reinterpret_cast<char*>(work + work_off[blockIdx.x]);
+    w.a = 0;
+    w.b = w.bytes;
+    w.c = 2 * w.bytes;
+    w.rhs = 3 * w.bytes;
+    w.t = 4 * w.bytes;
+    w.codes = (4 + TS) * w.bytes;
+
+    // the fields, diagonal-major; entries that are no cell hold 0 and code 0
+    bool odd = !divisible(d.delx2) || !divisible(d.dely2) ||
+               !(d.omega >= 0x1p-10 && d.omega <= 0x1p10);
+#pragma unroll 4
+    for (uint32_t k = tid; k < cells; k += NT) {
+        const int y = (int)(k % ROW), x = (int)(k / ROW) - LEX_PAD - y;
+        double pv = 0.0, rv = 0.0;
+        uint32_t c = 0;
+        if (x >= 0 && x < d.nx && y < d.ny) {
+            const int64_t g = d.off + x * (int64_t)d.pitch + y;
+            pv = p[g];
+            rv = rhs[g];
+            c = lex_code(flags[g], x >= 1 && x <= nxi && y >= 1 && y <= nyi);
+        }
+        double* e = reinterpret_cast<double*>(w.base) + k;
+        e[0] = pv;
+        e[cells] = 0.0;
+        e[2 * (int64_t)cells] = 0.0;
+        e[3 * (int64_t)cells] = rv;
+        const uint32_t row = k / ROW, lane = (uint32_t)y / RPL;
+        char* cp = w.base + (w.codes + row * P::ROWC + lane * code_bytes(RPL) + (uint32_t)y % RPL);
+        cp[0] = (char)c;
+        if (RPL == 3 && (uint32_t)y % RPL == RPL - 1) cp[1] = 0;   // the lane's pad
+        odd |= tiny(pv) | !finite(pv) | tiny(rv);
+    }
+    __syncthreads();
+    bool exact = __syncthreads_or(odd) != 0;
+
+    const double init = s.init_norm2, fluid = d.fluid_cells;
+    // a square of `bound` or more makes the norm neither < init nor < eps2
+    // (the factor covers the roundings of this product and of the norm's division)
+    const double bound = (init > d.eps2 ? init : d.eps2) * fluid * (1.0 + 0x1p-48);
+    double norm2 = 0.0;
+    int iters = d.itermax, exhausted = 1, done = 0;
+    const int before = (int)min(s.sor_iters, (uint32_t)LIGHT_MOST);
+    bool light = before == 0 || s.exhausted;
+    int len = before > 0 ? before : NSLOT;
+    int replay = 0;   // sweeps of the batch to be repeated, ending with the one that met the rule
+    while (done < d.itermax) {
+        const bool lt = light && !exact && replay == 0;
+        const int n = replay > 0 ? replay : min(lt ? len : min(len, TS), d.itermax - done);
+        const bool end = done + n == d.itermax;
+        typename P::Result r;
+        if (lt) r = P::template sweeps<LIGHT>(w, n, end ? n - 1 : n, bound, ring);
+        else if (!exact) r = P::template sweeps<FULL>(w, n, 0, 0.0, ring);
+        else r = P::template sweeps<FULL_DIV>(w, n, 0, 0.0, ring);
+        __syncthreads();
+        exact = exact || __syncthreads_or(r.bad) != 0;
+        if (lt) light = __syncthreads_or(r.open) == 0;
+        if ((lt && !light) || (exact && r.mode != FULL_DIV)) continue;   // again from A
+        if (lt && end) {   // the final field's norm
+            P::squares(w, w.b, nxi, nyi);
+            __syncthreads();
+        }
+        int stop = -1;
+        if (!lt || end) {
+            // the first norm in T that meets the rule
+            const int nt = lt ? 1 : n;
+            if (tid / 16 < nt) {
+                const double acc = P::norm_sum(w.base + (w.t + (tid / 16) * w.bytes), nxi, nyi,
+                                                 lt);
+                if (tid % 16 == 0) snorm[tid / 16] = acc / fluid;
+            }
+            __syncthreads();
+            for (int k = 0; k < nt && stop < 0; k++) {
+                norm2 = snorm[k];
+                if ((norm2 < init) || (norm2 < d.eps2)) stop = k;
+            }
+            __syncthreads();   // snorm is written again
+            if (r.mode == FULL && !finite(norm2)) {   // an overflow the quotient may have made a NaN
+                exact = true;
+                continue;
+            }
+            if (stop >= 0 && !lt && stop + 1 < n) {
+                replay = stop + 1;
+                continue;
+            }
+        }
+        const uint32_t old = w.a;
+        w.a = w.b;
+        w.b = old;
+        done += n;
+        len = min(2 * len, LIGHT_MOST);
+        if (stop >= 0) {
+            iters = done;
+            exhausted = 0;
+            break;
+        }
+    }
+    for (int k = tid; k < d.nx * d.ny; k += NT) {
+        const int x = k / d.ny, y = k - x * d.ny;
+        p[d.off + x * (int64_t)d.pitch + y] = *reinterpret_cast<const double*>(
+            w.base + (w.a + (uint32_t)(x + y + LEX_PAD) * P::ROWB + y * 8u));
+    }
+    if (tid == 0) {
+        s.sor_iters = (uint32_t)iters;
+        s.norm2 = norm2;
+        s.exhausted = exhausted;
+        s.active = 0;
+    }
+}
+
+// (class, lanes per slot, rows per lane, slots, slots of a FULL batch): rows
+// up to LW * RPL
+#define STM_LEX_CLASSES(V) \
+    V(0, 16, 2, 32, 16)    \
+    V(1, 16, 3, 32, 16)    \
+    V(2, 16, 4, 32, 16)    \
+    V(3, 32, 3, 16, 16)    \
+    V(4, 32, 4, 16, 16)    \
+    V(5, 64, 3, 8, 8)      \
+    V(6, 64, 4, 8, 8)      \
+    V(7, 64, 8, 4, 4)
+
+#define L_ENTRY(c, LW, RPL, NSLOT, TS) {LW * RPL, TS, LW * code_bytes(RPL)},
+const LexClass LEX_CLASSES[] = {STM_LEX_CLASSES(L_ENTRY)};
+#undef L_ENTRY
+const int N_LEX_CLASSES = sizeof(LEX_CLASSES) / sizeof(LEX_CLASSES[0]);
+
+void launch_lex_pipe(hipStream_t st, int cls, int nchan, const ChanDesc* cd, ChanState* cs,
+                     const int64_t* work_off, const uint8_t* flags, const double* rhs, double* p,
+                     double* work) {
+#define L_CASE(c, LW, RPL, NSLOT, TS)                                                             \
+    case c:                                                                                   \
+        k_lex_pipe<c, LW, RPL, NSLOT, TS><<<nchan, LW * NSLOT, 0, st>>>(cd, cs, work_off, flags, rhs, \
+                                                                    p, work);                 \
+        break;
+    switch (cls) {
+        STM_LEX_CLASSES(L_CASE)
+    default: break;
+    }
+#undef L_CASE
+}
+
+}  // namespace stm

@@ -33,6 +33,7 @@ struct ChanDesc {
     int32_t tile0, ntiles;       // slice of the tile list
     int32_t itermax, check_every;
     int32_t tb0, ntb;            // slice of the blocked-solver tile list
+    int32_t lex_class, pad;      // instance of the pipelined lexicographic solve, -1: none
     double delx, dely, gamma, reynolds, omega, eps, tau;
     double fluid_cells;
     double n_inner;              // interior fluid cells, x in [1, nx-2], y in [1, ny-2]
@@ -113,6 +114,9 @@ static_assert(sizeof(TbTile) == 64, "one 64-byte scalar load per tile");
 constexpr int TILE_X = 4;        // x-rows per tile
 constexpr int TILE_Y = 64;       // y-cells per tile (one wavefront)
 constexpr int TILE_THREADS = TILE_X * TILE_Y;
+
+// Rows of a diagonal-major field before its first and after its last diagonal.
+constexpr int LEX_PAD = 16;
 
 // Partial-sum slots per tile.
 constexpr int NPART = 16;
