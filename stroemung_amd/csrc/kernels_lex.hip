@@ -15,12 +15,14 @@
 // own last result, N the last result of the row above, E and S the row's own
 // and the row below's value on the next diagonal before the sweep (a DPP shift
 // where the row belongs to the next lane).  A slot hands its results to the
-// next through a three-diagonal LDS ring, so a step is one barrier.  Slot 0
-// reads the solve's input (A) and later the last slot's results (C, a round of
-// steps behind); the batch's last sweep writes B.  A ghost's pressure is the
-// copy of its fluid neighbours before the sweep (src/grid/mod.rs:343-412);
-// those are the slot's inputs of the two neighbouring diagonals, so each slot
-// forms the ghosts of its own sweep while its input passes.
+// next through a ring of four diagonals in LDS, so a step is one barrier.
+// Slot 0's ring is filled from the solve's input (A) and later from the last
+// slot's results (C, a round of steps behind); the batch's last sweep writes B.
+// A ghost's pressure is the copy of its fluid neighbours before the sweep
+// (src/grid/mod.rs:343-412); those are inputs of the two neighbouring
+// diagonals, still in the ring.  So a cell's code is the place its input is
+// read from, relative to its own: itself, or the neighbour a ghost copies --
+// one LDS read and no selection; only a ghost of two neighbours reads twice.
 //
 // The stopping rule is tested after every sweep, so sweeps in flight are
 // speculative: A stays as it was until the batch is accepted.  Two ways:
@@ -39,8 +41,8 @@
 //
 // Fields are kept diagonal-major (row d + LEX_PAD of ROW = LW * RPL values,
 // entry y), so a diagonal is one contiguous access.  LEX_PAD rows before the
-// first and after the last diagonal hold no cells: they are 0 with code 0, a
-// slot whose diagonal is outside the grid reads them and passes zeros on.
+// first and after the last diagonal hold no cells: they are 0 and their own
+// inputs, and a slot whose diagonal is outside the grid passes zeros on.
 #include <hip/hip_runtime.h>
 
 #include "kernels.h"
@@ -52,26 +54,12 @@ namespace {
 
 constexpr int LAG = 3;
 
-// Codes of the diagonal-major flags: the fluid neighbours a ghost copies (one
-// bit, or a vertical and a horizontal one whose mean it takes), whether the
-// sweep updates the cell, and whether it is an interior cell.
-enum : uint32_t { G_N = 1, G_S = 2, G_E = 4, G_W = 8, C_UPD = 16, C_IN = 32 };
-
-__device__ __forceinline__ uint32_t lex_code(uint8_t flag, bool inner) {
-    const uint32_t in = inner ? C_IN : 0u;
-    if (flag_fluid(flag)) return inner ? in | C_UPD : 0u;
-    switch (flag_edge(flag)) {
-    case E_N: return in | G_N;
-    case E_NE: return in | G_N | G_E;
-    case E_E: return in | G_E;
-    case E_SE: return in | G_S | G_E;
-    case E_S: return in | G_S;
-    case E_SW: return in | G_S | G_W;
-    case E_W: return in | G_W;
-    case E_NW: return in | G_N | G_W;
-    default: return in;
-    }
-}
+// A cell's code, 16 bits: the byte offset of its input in its slot's ring (a
+// multiple of 8 below 2^14, see Pipe), and in the other bits whether the sweep
+// updates the cell, whether it is an interior cell, whether it is a ghost of
+// two neighbours (whose vertical one the offset names), and whether the other
+// one is its E neighbour (else W).
+enum : uint32_t { C_UPD = 1, C_IN = 2, C_CORNER = 4, C_EAST = 0x8000, C_OFFSET = 0x3ff8 };
 
 // Lane i takes lane i - 1's value (UP) or lane i + 1's: a DPP wave shift.
 // The lane at the wave's end gets 0.0.
@@ -130,7 +118,7 @@ __device__ __forceinline__ uint32_t tiny_word(double p) {
 }
 __device__ __forceinline__ bool finite(double p) { return fabs(p) < __builtin_inf(); }
 
-// A lane's RPL values, and its codes (CODES bytes).
+// A lane's RPL values, and its codes.
 typedef double double2u __attribute__((ext_vector_type(2), aligned(8)));
 template <int RPL>
 __device__ __forceinline__ void load_row(const void* p, double (&v)[RPL]) {
@@ -151,11 +139,32 @@ __device__ __forceinline__ void store_row(void* p, const double (&v)[RPL]) {
         *reinterpret_cast<double2u*>(q + i) = double2u{v[i], v[i + 1]};
     if constexpr (RPL % 2 != 0) q[RPL - 1] = v[RPL - 1];
 }
-constexpr int code_bytes(int rpl) { return rpl <= 4 ? 4 : 8; }
+constexpr int code_words(int rpl) { return rpl <= 2 ? 1 : rpl <= 4 ? 2 : 4; }
 template <int RPL>
-__device__ __forceinline__ uint64_t load_codes(const void* p) {
-    if constexpr (code_bytes(RPL) == 4) return *static_cast<const uint32_t*>(p);
-    else return *static_cast<const uint64_t*>(p);
+struct Codes {
+    uint32_t w[code_words(RPL)];
+    __device__ __forceinline__ uint32_t raw(int i) const { return w[i / 2] >> (16 * (i & 1)); }
+    __device__ __forceinline__ bool is(int i, uint32_t bit) const {
+        return (w[i / 2] & (bit << (16 * (i & 1)))) != 0;
+    }
+};
+template <int RPL>
+__device__ __forceinline__ Codes<RPL> load_codes(const void* p) {
+    Codes<RPL> c;
+    if constexpr (code_words(RPL) == 1) {
+        c.w[0] = *static_cast<const uint32_t*>(p);
+    } else if constexpr (code_words(RPL) == 2) {
+        const uint2 t = *static_cast<const uint2*>(p);
+        c.w[0] = t.x;
+        c.w[1] = t.y;
+    } else {
+        const uint4 t = *static_cast<const uint4*>(p);
+        c.w[0] = t.x;
+        c.w[1] = t.y;
+        c.w[2] = t.z;
+        c.w[3] = t.w;
+    }
+    return c;
 }
 
 // Sum of acc and t of the row's lanes 0 .. 15, added one after another in that
@@ -177,7 +186,7 @@ __device__ __forceinline__ double add_row(double acc, double t) {
 // (32 bits: lex_class keeps a channel's scratch below 4 GB).
 struct LexWork {
     char* base;
-    uint32_t a, b, c, rhs, t, codes;   // codes: code_bytes per lane, the others 8 per entry
+    uint32_t a, b, c, rhs, t, codes;   // codes: code_words per lane, the others 8 bytes per entry
     uint32_t bytes;           // of one diagonal-major field
     int dmax;                 // the last diagonal, nx + ny - 2
     int ny;
@@ -190,20 +199,46 @@ enum : int { LIGHT = 0, FULL = 1, FULL_DIV = 2 };   // FULL_DIV: FULL with the g
 template <int LW, int RPL, int NSLOT, int TS>
 struct Pipe {
     static constexpr int ROW = LW * RPL, NT = LW * NSLOT;
-    static constexpr uint32_t ROWB = ROW * 8, ROWC = LW * code_bytes(RPL);   // bytes of a row
+    static constexpr uint32_t ROWB = ROW * 8, ROWC = LW * 4 * code_words(RPL);   // bytes of a row
     static constexpr int Q = 3;              // steps of a group; loads are a group ahead
-    static constexpr int RING = NSLOT * ROW;
     static_assert(LAG == Q && TS <= NSLOT, "slots change sweeps between groups");
-    // rows of the pads a slot reads and writes: -2 - 6 - 1 and up to
-    // -2 + 3 * last() + 2 + 2 <= dmax + 7
+    // rows of the pads a slot reads and writes: -3 - 6 - 1 and up to
+    // -3 + 3 * last() + 2 + 3 <= dmax + 8
     static_assert(LEX_PAD >= 10, "pads");
 
+    // A slot's ring: four diagonals of ROWP places (a power of two).  In step
+    // e the slot before it writes place e & 3; diagonals d, d + 1, d + 2 are
+    // the results of its steps e - 3, e - 2, e - 1.
+    static constexpr uint32_t pow2(uint32_t n) { return n <= 1 ? 1 : 2 * pow2((n + 1) / 2); }
+    static constexpr uint32_t ROWP = pow2(ROW) * 8, RINGB = 4 * ROWP;        // bytes
+    static constexpr uint32_t SHARED = (NSLOT + 1) * RINGB / 8;              // doubles
+    static_assert(RINGB <= 0x4000, "offsets of codes");
+    // The code of cell (x, y) with flag f: the offset is relative to the
+    // lane's first row on diagonal d, the cell being on d + 1.
+    __device__ static __forceinline__ uint32_t code(uint8_t f, int y, bool inner) {
+        int dd = 1, dy = 0;
+        uint32_t c = inner ? C_IN : 0u;
+        if (flag_fluid(f)) {
+            if (inner) c |= C_UPD;
+        } else {
+            const uint8_t e = flag_edge(f);
+            if (e == E_N || e == E_NE || e == E_NW) { dd = 0; dy = -1; }
+            else if (e == E_S || e == E_SE || e == E_SW) { dd = 2; dy = 1; }
+            else if (e == E_E) dd = 2;
+            else if (e == E_W) dd = 0;
+            if (e == E_NE || e == E_SE) c |= C_CORNER | C_EAST;
+            if (e == E_NW || e == E_SW) c |= C_CORNER;
+        }
+        return c | ((uint32_t)(dd * (int)ROWP + (y % RPL + dy) * 8) & (RINGB - 8));
+    }
+
     // Groups of a sweep, and of a round: a slot starts its next sweep a round
-    // after this one.  Slot 0 uses row q of C in step q of its round and loads
-    // it a group earlier; the last slot stores row q in step 3 (NSLOT - 1) + 2
-    // + q of the round before: at least 13 steps earlier, and it waits for its
-    // stores once a group.
-    __device__ static __forceinline__ int last(const LexWork& w) { return (w.dmax + 3 + Q - 1) / Q; }
+    // after this one.  Slot 0's ring takes row q of C in step q of its round,
+    // loaded a group earlier; the last slot stores row q in step 3 NSLOT + q of
+    // the round before: at least 12 steps earlier.  A wave's global loads and
+    // stores complete in order, and in every step it uses loads issued a group
+    // (3 steps) before, so that store has long been complete.
+    __device__ static __forceinline__ int last(const LexWork& w) { return (w.dmax + 4 + Q - 1) / Q; }
     __device__ static __forceinline__ int round(const LexWork& w) { return max(last(w) + 1, NSLOT + 5); }
 
     struct Result {
@@ -226,44 +261,42 @@ struct Pipe {
         const int glast = last(w), ground = round(w);
         const int groups = (n - 1) / NSLOT * ground + (n - 1) % NSLOT + glast;
         Result res{MODE, false, false};
-#pragma unroll
-        for (int i = 0; i < 3 * RPL; i++) ring[i * NT + threadIdx.x] = 0.0;
+        for (uint32_t i = threadIdx.x; i < SHARED; i += NT) ring[i] = 0.0;
         __syncthreads();
         // waves without a slot of the batch only keep the barriers
         if ((int)(threadIdx.x & ~63u) / LW >= n) {
             for (int e = 0; e < groups * Q; e++) asm volatile("s_barrier" ::: "memory");
             return res;
         }
-        const bool rows_in = y0 < w.ny;      // lanes below the last row: zeros with code 0
+        const bool rows_in = y0 < w.ny;      // lanes below the last row: zeros, inputs themselves
         const bool first = slot == 0;
         const uint32_t yb = (uint32_t)y0 * 8u;
-        const double* in = ring + (slot > 0 ? slot - 1 : 0) * ROW + y0;
-        double* out = ring + slot * ROW + y0;
-        // the slot's group g of its sweep k: diagonals d = -2 + 3 g .. + 2.
+        // this lane's first row in its slot's ring, and in the next slot's
+        char* const lds = reinterpret_cast<char*>(ring);
+        const uint32_t ring_in = (uint32_t)slot * RINGB, ring_out = ring_in + RINGB + yb;
+        // the slot's group g of its sweep k: diagonals d = -3 + 3 g .. + 2.
         // Before its first and after its last group a slot is on the pads.
         int g = -slot, k = slot;
-        auto row0 = [&](int gg) -> uint32_t {   // row -2 + 3 gg of a field
-            return (uint32_t)(min(max(gg, -2), glast) * Q + (LEX_PAD - 2));
+        auto row0 = [&](int gg) -> uint32_t {   // row -3 + 3 gg of a field
+            return (uint32_t)(min(max(gg, -2), glast) * Q + (LEX_PAD - 3));
         };
         // this lane's codes of row r
         auto code_at = [&](uint32_t r) -> uint32_t {
-            return w.codes + r * ROWC + (threadIdx.x % LW) * code_bytes(RPL);
+            return w.codes + r * ROWC + (threadIdx.x % LW) * (4u * code_words(RPL));
         };
-        // what slot 0 reads in sweep kk
+        // what slot 0's ring takes in sweep kk: rows from d + 3 on
         auto from = [&](int kk, uint32_t r0) -> uint32_t {
-            return (kk == 0 ? w.a : w.c) + (r0 + 2) * ROWB + yb;
+            return (kk == 0 ? w.a : w.c) + (r0 + 3) * ROWB + yb;
         };
         const bool wave0 = __builtin_amdgcn_readfirstlane(threadIdx.x) < 64;   // holds slot 0
-        double raw0[RPL], raw1[RPL];         // inputs of diagonals d, d + 1
-        double in0[RPL];                     // diagonal d with its ghosts formed
+        double in0[RPL];                     // the input of diagonal d (ghosts formed)
         double o1[RPL], dxp[RPL], dvp[RPL], rp[RPL];   // diagonal d - 1: result, its differences
                                                        // to W and N, rhs
-        uint64_t code0 = 0, codep = 0;       // codes of diagonals d, d - 1
-        double aq[Q][RPL], rq[Q][RPL];       // slot 0's input of d + 2, rhs of d
-        uint64_t cq[Q];                      // codes of d + 1
+        Codes<RPL> code0{}, codep{};         // codes of diagonals d, d - 1
+        double aq[Q][RPL], rq[Q][RPL];       // slot 0's input of d + 3, rhs of d
+        Codes<RPL> cq[Q];                    // codes of d + 1
 #pragma unroll
-        for (int i = 0; i < RPL; i++)
-            raw0[i] = raw1[i] = in0[i] = o1[i] = dxp[i] = dvp[i] = rp[i] = 0.0;
+        for (int i = 0; i < RPL; i++) in0[i] = o1[i] = dxp[i] = dvp[i] = rp[i] = 0.0;
         {
             const uint32_t r0 = row0(g), f0 = from(k, r0);
 #pragma unroll
@@ -273,6 +306,7 @@ struct Pipe {
                 cq[j] = load_codes<RPL>(w.base + (code_at(r0) + (j + 1) * ROWC));
             }
         }
+        uint32_t cur = ROWP;                 // byte offset of diagonal d in the rings: (e + 1) & 3
         uint32_t small = ~0u;                // the least tiny_word
         bool shown = false;                  // LIGHT: this lane's square for sweep k
         auto slot_any = [&](bool v) -> bool {   // some lane of the slot
@@ -296,34 +330,26 @@ struct Pipe {
             const bool keep_t = rows_in & (k < n);
 #pragma unroll
             for (int j = 0; j < Q; j++) {
-                // the input of diagonal d + 2: the previous slot's result of the
-                // last step
-                double raw2[RPL];
-                load_row<RPL>(in + j * RING, raw2);
-                if (wave0)
-#pragma unroll
-                    for (int i = 0; i < RPL; i++) raw2[i] = first ? aq[j][i] : raw2[i];
-                // ghosts of diagonal d + 1
+                // the inputs of diagonal d + 1, ghosts' from their neighbours
                 double in1[RPL];
-                const uint64_t code1 = cq[j];
-                {
-                    const double un = lane_shift<true>(raw0[RPL - 1]);
-                    const double dn = lane_shift<false>(raw2[0]);
-                    constexpr uint64_t HORZ = 0x0101010101010101ull * (G_E | G_W);
-                    const bool full = __ballot((code1 & HORZ) != 0) != 0;   // uniform
+                const Codes<RPL> code1 = cq[j];
+                const uint32_t at = yb + cur;
+#pragma unroll
+                for (int i = 0; i < RPL; i++)
+                    in1[i] = *reinterpret_cast<const double*>(
+                        lds + (((code1.raw(i) + at) & (RINGB - 8)) | ring_in));
+                // slot 0's ring takes diagonal d + 3
+                if (wave0 && first) store_row<RPL>(lds + (((cur + 3 * ROWP) & (RINGB - 8)) + yb), aq[j]);
+                bool corner = false;
+#pragma unroll
+                for (int i = 0; i < RPL; i++) corner |= code1.is(i, C_CORNER);
+                if (__ballot(corner) != 0) {   // uniform
 #pragma unroll
                     for (int i = 0; i < RPL; i++) {
-                        const uint32_t c = (uint32_t)(code1 >> (8 * i));
-                        const double vn = i > 0 ? raw0[i > 0 ? i - 1 : 0] : un;
-                        const double vs = i + 1 < RPL ? raw2[i + 1 < RPL ? i + 1 : i] : dn;
-                        const double v = (c & G_N) ? vn : ((c & G_S) ? vs : raw1[i]);
-                        in1[i] = v;
-                        if (full) {   // copies across, and means
-                            const double h = (c & G_E) ? raw2[i] : raw0[i];
-                            const bool vert = (c & (G_N | G_S)) != 0;
-                            const double m = vert ? (v + h) * 0.5 : h;
-                            in1[i] = (c & (G_E | G_W)) ? m : v;
-                        }
+                        const uint32_t q = at + (code1.is(i, C_EAST) ? 2 * ROWP : 0u) + i * 8;
+                        const double h = *reinterpret_cast<const double*>(
+                            lds + ((q & (RINGB - 8)) | ring_in));
+                        in1[i] = code1.is(i, C_CORNER) ? (in1[i] + h) * 0.5 : in1[i];
                     }
                 }
                 // the update of diagonal d (src/simulation.rs:266-270)
@@ -338,11 +364,11 @@ struct Pipe {
                         const double lap = quotient<EXACT>(in1[i] + o1[i], w.dx2) +
                                            quotient<EXACT>(s + nb[i], w.dy2);
                         const double v = (w.omw * in0[i]) + (w.mid * (lap - rq[j][i]));
-                        o[i] = ((uint32_t)(code0 >> (8 * i)) & C_UPD) ? v : in0[i];
+                        o[i] = code0.is(i, C_UPD) ? v : in0[i];
                         if constexpr (!EXACT) small = min(small, tiny_word(o[i]));
                     }
                 }
-                store_row<RPL>(out + (j + 1) % 3 * RING, o);
+                store_row<RPL>(lds + (((cur + 3 * ROWP) & (RINGB - 8)) + ring_out), o);
                 // the residual of diagonal d - 1 (src/math.rs:176-186): c - W of
                 // a cell is E - c of the cell before it, c - N is S - c of the
                 // cell above
@@ -363,8 +389,7 @@ struct Pipe {
                                               quotient<EXACT>(sc - dvp[i], w.dy2)) - rp[i];
                             tt[i] = r * r;
                             if (MODE == LIGHT)
-                                shown |= (((uint32_t)(codep >> (8 * i)) & C_IN) != 0) &
-                                         (tt[i] >= bound);
+                                shown |= codep.is(i, C_IN) & (tt[i] >= bound);
                         }
                         if (MODE != LIGHT && keep_t)
                             store_row<RPL>(w.base + (tb + j * ROWB), tt);
@@ -382,19 +407,15 @@ struct Pipe {
 #pragma unroll
                         for (int i = 0; i < RPL; i++) res.bad |= !finite(o[i]);
                 }
-                // the stores before this group's last step are done (the loads
-                // this also waits for are nearly a group old)
-                if (MODE == LIGHT && j == Q - 1) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
                 // on to the next diagonal
 #pragma unroll
                 for (int i = 0; i < RPL; i++) {
-                    raw0[i] = raw1[i];
-                    raw1[i] = raw2[i];
                     in0[i] = in1[i];
                     o1[i] = o[i];
                 }
                 codep = code0;
                 code0 = code1;
+                cur = (cur + ROWP) & (RINGB - 8);
                 if (wave0) load_row<RPL>(w.base + (fn0 + j * ROWB), aq[j]);
                 load_row<RPL>(w.base + (rb + j * ROWB), rq[j]);
                 cq[j] = load_codes<RPL>(w.base + (cb + j * ROWC));
@@ -419,15 +440,12 @@ struct Pipe {
         return res;
     }
 
-    // The sum from 0.0 of a field's squares over the interior, x-major, by a
-    // row of 16 lanes: U * 16 terms are loaded (that many ahead) and added one
-    // by one.  Places past the end add +0.0, which changes no sum of squares.
-    // `linear`: the squares are in that order in memory (as `squares` leaves
-    // them), else diagonal-major.
-    static constexpr int U = 8;
-    __device__ static __forceinline__ double norm_sum(const char* t, int nxi, int nyi,
-                                                      bool linear) {
-        constexpr int CHUNK = U * 16;
+    // The sum from 0.0 of a diagonal-major field's squares over the interior,
+    // x-major, by a row of 16 lanes: U * 16 terms are gathered (that many
+    // ahead) and added one by one.  Places past the end add +0.0, which
+    // changes no sum of squares.
+    static constexpr int U = 8, CHUNK = U * 16;
+    __device__ static __forceinline__ double norm_sum(const char* t, int nxi, int nyi) {
         const int lane = threadIdx.x & 15;
         const int n = nxi * nyi;
         const int sx = CHUNK / nyi, sy = CHUNK - sx * nyi;
@@ -442,9 +460,7 @@ struct Pipe {
         auto gather = [&]() {
 #pragma unroll
             for (int u = 0; u < U; u++) {
-                const int xc = min(x[u], nxi);
-                const uint32_t at = linear ? (uint32_t)((xc - 1) * nyi + y[u] - 1) * 8u
-                                           : (uint32_t)(xc + y[u] + LEX_PAD) * ROWB + y[u] * 8u;
+                const uint32_t at = (uint32_t)(min(x[u], nxi) + y[u] + LEX_PAD) * ROWB + y[u] * 8u;
                 const double q = *reinterpret_cast<const double*>(t + at);
                 v[u] = x[u] <= nxi ? q : 0.0;
                 x[u] += sx;
@@ -465,6 +481,31 @@ struct Pipe {
 #pragma unroll
             for (int u = 0; u < U; u++) acc = add_row(acc, c[u]);
         }
+        return acc;
+    }
+
+    // The same for n squares in the norm's order in memory (T, which is longer
+    // than they are by more than two chunks).
+    __device__ static __forceinline__ double norm_sum_linear(const char* t, int n) {
+        const double* q = reinterpret_cast<const double*>(t) + (threadIdx.x & 15);
+        double v[U], acc = 0.0;
+#pragma unroll
+        for (int u = 0; u < U; u++) v[u] = q[u * 16];
+        int k = 0;
+        for (; k + CHUNK <= n; k += CHUNK) {
+            double c[U];
+            q += CHUNK;
+#pragma unroll
+            for (int u = 0; u < U; u++) c[u] = v[u];
+#pragma unroll
+            for (int u = 0; u < U; u++) v[u] = q[u * 16];
+            __builtin_amdgcn_sched_barrier(0);   // the loads go first
+#pragma unroll
+            for (int u = 0; u < U; u++) acc = add_row(acc, c[u]);
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++)
+            acc = add_row(acc, k + u * 16 + (int)(threadIdx.x & 15) < n ? v[u] : 0.0);
         return acc;
     }
 
@@ -513,7 +554,7 @@ k_lex_pipe(const ChanDesc* __restrict__ cd, ChanState* __restrict__ cs,
 {
     using P = Pipe<LW, RPL, NSLOT, TS>;
     constexpr int ROW = P::ROW, NT = P::NT;
-    __shared__ __attribute__((aligned(16))) double ring[3 * P::RING];
+    __shared__ __attribute__((aligned(16))) double ring[P::SHARED];
     __shared__ double snorm[TS];
     const ChanDesc d = cd[blockIdx.x];
     if (d.solver != SOLVER_LEX || d.lex_class != CLASS) return;
@@ -540,26 +581,25 @@ k_lex_pipe(const ChanDesc* __restrict__ cd, ChanState* __restrict__ cs,
     // the fields, diagonal-major; entries that are no cell hold 0 and code 0
     bool odd = !divisible(d.delx2) || !divisible(d.dely2) ||
                !(d.omega >= 0x1p-10 && d.omega <= 0x1p10);
-#pragma unroll 4
+    // (every load from a clamped place: a batch of them is in flight at once)
+#pragma unroll 8
     for (uint32_t k = tid; k < cells; k += NT) {
-        const int y = (int)(k % ROW), x = (int)(k / ROW) - LEX_PAD - y;
-        double pv = 0.0, rv = 0.0;
-        uint32_t c = 0;
-        if (x >= 0 && x < d.nx && y < d.ny) {
-            const int64_t g = d.off + x * (int64_t)d.pitch + y;
-            pv = p[g];
-            rv = rhs[g];
-            c = lex_code(flags[g], x >= 1 && x <= nxi && y >= 1 && y <= nyi);
-        }
+        const int row = (int)(k / ROW), y = (int)(k % ROW), x = row - LEX_PAD - y;
+        const bool in = x >= 0 && x < d.nx && y < d.ny;
+        const int64_t g = d.off + min(max(x, 0), d.nx - 1) * (int64_t)d.pitch + min(y, d.ny - 1);
+        const double pg = p[g], rg = rhs[g];
+        const uint8_t fg = flags[g];
+        const double pv = in ? pg : 0.0, rv = in ? rg : 0.0;
+        const uint8_t f = in ? fg : make_flag(T_NOSLIP, E_NONE);
         double* e = reinterpret_cast<double*>(w.base) + k;
         e[0] = pv;
         e[cells] = 0.0;
         e[2 * (int64_t)cells] = 0.0;
         e[3 * (int64_t)cells] = rv;
-        const uint32_t row = k / ROW, lane = (uint32_t)y / RPL;
-        char* cp = w.base + (w.codes + row * P::ROWC + lane * code_bytes(RPL) + (uint32_t)y % RPL);
-        cp[0] = (char)c;
-        if (RPL == 3 && (uint32_t)y % RPL == RPL - 1) cp[1] = 0;   // the lane's pad
+        // (a lane of three rows leaves its fourth code unread)
+        reinterpret_cast<uint16_t*>(w.base + w.codes)[row * (P::ROWC / 2) + y / RPL * 2 * code_words(RPL) +
+                                                      y % RPL] =
+            (uint16_t)P::code(f, y, x >= 1 && x <= nxi && y >= 1 && y <= nyi);
         odd |= tiny(pv) | !finite(pv) | tiny(rv);
     }
     __syncthreads();
@@ -576,28 +616,31 @@ k_lex_pipe(const ChanDesc* __restrict__ cd, ChanState* __restrict__ cs,
     int len = before > 0 ? before : NSLOT;
     int replay = 0;   // sweeps of the batch to be repeated, ending with the one that met the rule
     while (done < d.itermax) {
-        const bool lt = light && !exact && replay == 0;
-        const int n = replay > 0 ? replay : min(lt ? len : min(len, TS), d.itermax - done);
+        const int most = light && !exact ? len : min(len, TS);
+        const int n = replay > 0 ? replay : min(most, d.itermax - done);
         const bool end = done + n == d.itermax;
+        // a single sweep's norm is the final field's: no need of T
+        const bool lt = !exact && ((light && replay == 0) || n == 1), field = lt && (end || n == 1);
         typename P::Result r;
-        if (lt) r = P::template sweeps<LIGHT>(w, n, end ? n - 1 : n, bound, ring);
+        if (lt) r = P::template sweeps<LIGHT>(w, n, field ? n - 1 : n, bound, ring);
         else if (!exact) r = P::template sweeps<FULL>(w, n, 0, 0.0, ring);
         else r = P::template sweeps<FULL_DIV>(w, n, 0, 0.0, ring);
         __syncthreads();
         exact = exact || __syncthreads_or(r.bad) != 0;
-        if (lt) light = __syncthreads_or(r.open) == 0;
-        if ((lt && !light) || (exact && r.mode != FULL_DIV)) continue;   // again from A
-        if (lt && end) {   // the final field's norm
+        const bool open = lt && __syncthreads_or(r.open) != 0;
+        light = light && !open;
+        if (open || (exact && r.mode != FULL_DIV)) continue;   // again from A
+        if (field) {
             P::squares(w, w.b, nxi, nyi);
             __syncthreads();
         }
         int stop = -1;
-        if (!lt || end) {
+        if (!lt || field) {
             // the first norm in T that meets the rule
             const int nt = lt ? 1 : n;
             if (tid / 16 < nt) {
-                const double acc = P::norm_sum(w.base + (w.t + (tid / 16) * w.bytes), nxi, nyi,
-                                                 lt);
+                const char* t = w.base + (w.t + (tid / 16) * w.bytes);
+                const double acc = lt ? P::norm_sum_linear(t, nxi * nyi) : P::norm_sum(t, nxi, nyi);
                 if (tid % 16 == 0) snorm[tid / 16] = acc / fluid;
             }
             __syncthreads();
@@ -610,7 +653,7 @@ k_lex_pipe(const ChanDesc* __restrict__ cd, ChanState* __restrict__ cs,
                 exact = true;
                 continue;
             }
-            if (stop >= 0 && !lt && stop + 1 < n) {
+            if (stop >= 0 && stop + 1 < n && !lt) {
                 replay = stop + 1;
                 continue;
             }
@@ -651,7 +694,7 @@ k_lex_pipe(const ChanDesc* __restrict__ cd, ChanState* __restrict__ cs,
     V(6, 64, 4, 8, 8)      \
     V(7, 64, 8, 4, 4)
 
-#define L_ENTRY(c, LW, RPL, NSLOT, TS) {LW * RPL, TS, LW * code_bytes(RPL)},
+#define L_ENTRY(c, LW, RPL, NSLOT, TS) {LW * RPL, TS, LW * 4 * code_words(RPL)},
 const LexClass LEX_CLASSES[] = {STM_LEX_CLASSES(L_ENTRY)};
 #undef L_ENTRY
 const int N_LEX_CLASSES = sizeof(LEX_CLASSES) / sizeof(LEX_CLASSES[0]);
