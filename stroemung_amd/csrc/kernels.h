@@ -32,6 +32,15 @@ void launch_advance_time(hipStream_t, int nchan, ChanState*);
 void launch_fill(hipStream_t, int64_t n, double* a, double val);
 void launch_zero_cells(hipStream_t, int n, const int64_t* idx, double* u, double* v,
                        double* p);
+// Rows of several fields of a channel against dense arrays (dense[f] holds the
+// rows [x0, x0 + rows) of field f, y contiguous without padding).
+struct FieldRows {
+    double* dev[6];
+    double* dense[6];
+    int64_t off, pitch;
+    int32_t x0, rows, ny;
+};
+void launch_rows(hipStream_t, const FieldRows&, int nfields, bool pack);
 void launch_copy(hipStream_t, int64_t bytes, const double* src, double* dst);
 
 // kernels_pressure.hip
