@@ -90,8 +90,9 @@ struct stm_ctx {
     double* d_tbpart = nullptr;    // blocked solver: residual partials, two launches
     TbTile* d_tb = nullptr;
     int ntb = 0, tb_capacity = 0, part_capacity = 0;
-    uint32_t* d_codes = nullptr;   // blocked solver: per-thread cell codes of every tile
-    size_t codes_capacity = 0;     // bytes
+    TbWave* d_waves = nullptr;     // blocked solver: what each wave of a tile holds
+    uint32_t* d_words = nullptr;   // and its cells' codes
+    size_t waves_capacity = 0, words_capacity = 0;   // bytes
     std::vector<TbTile> h_tb;      // host copy of the full list
     // the list launches use: d_tb, or during a polled solve the tiles of the
     // channels still running (d_tbc, staged through pinned h_tbc)
@@ -372,10 +373,10 @@ int upload_descs(stm_ctx* ctx) {
 
 int count_tb(stm_ctx* ctx, int variant) {
     const TbVariant& v = TB_VARIANTS[variant];
-    const int H = 2 * v.k + 4;
+    const int H = tb_halo(v.k);
     int n = 0;
     for (auto& c : ctx->chans)
-        n += (int)(plan_axis((int)c.nx, v.ex, H, 1).size() *
+        n += (int)(plan_axis((int)c.nx, v.ex, H, 2).size() *
                    plan_axis((int)c.ny, v.ey, H, 2).size());
     return n;
 }
@@ -408,18 +409,30 @@ void order_for_xcds(TbTile* t, int p0, int n, int nyt) {
         for (int p = p0 + c; p < p0 + n; p += NXCD) t[p - p0] = z[k++];
 }
 
+// A device buffer of at least `bytes` (its content is not kept).
+template <typename T>
+int grow(stm_ctx* ctx, T** buf, size_t* capacity, size_t bytes) {
+    if (bytes <= *capacity) return STM_OK;
+    if (*buf) HIPCHK(ctx, hipFree(*buf));
+    *buf = nullptr;
+    *capacity = 0;
+    HIPCHK(ctx, hipMalloc(buf, bytes));
+    *capacity = bytes;
+    return STM_OK;
+}
+
 // Output tiles of the blocked solver for `variant`, channel by channel
 // (canonical idx: x-major over the channel's tile grid; launch order from
 // order_for_xcds).
 int plan_tb(stm_ctx* ctx, int variant) {
     invalidate_graphs(ctx);   // blocked launches capture d_tb and its length
     const TbVariant& v = TB_VARIANTS[variant];
-    const int H = 2 * v.k + 4;
+    const int H = tb_halo(v.k);
     std::vector<TbTile> tl;
     for (size_t k = 0; k < ctx->chans.size(); k++) {
         HostChan& c = ctx->chans[k];
         c.tb0 = (int32_t)tl.size();
-        const auto ax = plan_axis((int)c.nx, v.ex, H, 1), ay = plan_axis((int)c.ny, v.ey, H, 2);
+        const auto ax = plan_axis((int)c.nx, v.ex, H, 2), ay = plan_axis((int)c.ny, v.ey, H, 2);
         for (auto xs : ax)
             for (auto ys : ay)
                 tl.push_back(TbTile{(int32_t)k, xs.start, ys.start, xs.len, ys.len,
@@ -438,14 +451,14 @@ int plan_tb(stm_ctx* ctx, int variant) {
     }
     HIPCHK(ctx, hipMemcpyAsync(ctx->d_tb, tl.data(), sizeof(TbTile) * tl.size(),
                                hipMemcpyHostToDevice, ctx->stream));
-    // the codes table (graphs holding the old one were dropped above)
-    const size_t cbytes = v.codes ? (size_t)tl.size() * v.nt * TB_CODE_BYTES : 0;
-    if (cbytes > ctx->codes_capacity) {
-        if (ctx->d_codes) HIPCHK(ctx, hipFree(ctx->d_codes));
-        ctx->d_codes = nullptr;
-        HIPCHK(ctx, hipMalloc(&ctx->d_codes, cbytes));
-        ctx->codes_capacity = cbytes;
-    }
+    // the cells' tables (graphs holding the old ones were dropped above)
+    const size_t nwaves = tl.size() * (size_t)(v.nt / 64);
+    int rc = grow(ctx, &ctx->d_waves, &ctx->waves_capacity, nwaves * sizeof(TbWave));
+    if (!rc) rc = grow(ctx, &ctx->d_words, &ctx->words_capacity,
+                       nwaves * (size_t)(v.rows + 1) * 64 * sizeof(uint32_t));
+    if (rc) return rc;
+    launch_rb_codes(ctx->stream, variant, (int)tl.size(), ctx->d_tb, ctx->flags, ctx->d_waves,
+                    ctx->d_words);
     ctx->ntb = (int)tl.size();
     ctx->h_tb = tl;
     ctx->tb_cur = ctx->d_tb;
@@ -690,16 +703,16 @@ int compact_tiles(stm_ctx* ctx, const int32_t* active) {
 }
 
 // Launch L of the blocked solver on the current variant.  Every sequence
-// of launches starts at L = 0, which computes the cell codes of every
-// running tile and stores them; launches L > 0 of the sequence load them
-// (variants whose codes fit the table).
+// of launches starts at L = 0, on fresh ghosts of the channels it runs.
 void launch_blocked(stm_ctx* ctx, int variant, int L, int mode) {
     const int cap = ctx->part_capacity;
     double* prev = ctx->d_tbpart + (size_t)((L + 1) & 1) * cap;
     double* cur = ctx->d_tbpart + (size_t)(L & 1) * cap;
-    if (TB_VARIANTS[variant].codes) mode |= L == 0 ? TB_CODES_PUT : TB_CODES_GET;
-    launch_rb_tb(ctx->stream, variant, ctx->ntb_cur, ctx->d_cd, ctx->d_cs, ctx->tb_cur, ctx->flags,
-                 ctx->rhs, ctx->p, ctx->p2, prev, cur, ctx->d_active, ctx->d_codes, L, mode);
+    if (L == 0)
+        launch_ghost(ctx->stream, ctx->nbtot, ctx->d_be, ctx->d_cs, ctx->p, -1, 1);
+    launch_rb_tb(ctx->stream, variant, ctx->ntb_cur, ctx->d_cd, ctx->d_cs, ctx->tb_cur,
+                 ctx->d_waves, ctx->d_words, ctx->rhs, ctx->p, ctx->p2, prev, cur, ctx->d_active,
+                 L, mode);
 }
 
 // Blocked red-black launches until no channel is running.  Launch L also
@@ -1251,7 +1264,7 @@ void stm_destroy(stm_ctx* ctx) {
     for (hipEvent_t e : ctx->free_events) hipEventDestroy(e);
     void* bufs[] = {ctx->u, ctx->v, ctx->p, ctx->f, ctx->g, ctx->rhs, ctx->scratch, ctx->p2,
                     ctx->lexwork, ctx->d_lexoff, ctx->flags, ctx->d_cd, ctx->d_cs, ctx->d_be, ctx->d_restore, ctx->d_tiles,
-                    ctx->d_part, ctx->d_active, ctx->d_tbpart, ctx->d_tb, ctx->d_codes, ctx->d_tbc, ctx->d_lc, ctx->lres,
+                    ctx->d_part, ctx->d_active, ctx->d_tbpart, ctx->d_tb, ctx->d_waves, ctx->d_words, ctx->d_tbc, ctx->d_lc, ctx->lres,
                     ctx->lcf, ctx->lprev, ctx->lprev2, ctx->lsnap, ctx->lrc, ctx->lmc, ctx->d_cpart, ctx->d_map,
                     ctx->d_inv, ctx->d_live, ctx->d_rgba};
     for (void* b : bufs)
@@ -1338,6 +1351,8 @@ int stm_set_cells(stm_ctx* ctx, uint32_t ch, const uint8_t* cell_type,
     if ((rc = ready(ctx))) return rc;
     if ((rc = upload_boundaries(ctx))) return rc;
     if ((rc = upload_flags(ctx, c))) return rc;
+    launch_rb_codes(ctx->stream, ctx->variant, ctx->ntb, ctx->d_tb, ctx->flags, ctx->d_waves,
+                    ctx->d_words);
     if ((rc = upload_descs(ctx))) return rc;
     if (!changed.empty()) {
         int64_t* d_idx = nullptr;
@@ -2022,12 +2037,12 @@ int stm_solver_bytes(stm_ctx* ctx, double* unique_bytes, double* loaded_bytes) {
     if (rc) return rc;
     const TbVariant& v = TB_VARIANTS[ctx->variant];
     double unique = 0.0, loaded = 0.0;
-    for (const auto& c : ctx->chans) unique += 25.0 * (double)c.nx * (double)c.ny;
+    for (const auto& c : ctx->chans) unique += 24.0 * (double)c.nx * (double)c.ny;
     for (const TbTile& t : ctx->h_tb) {
         const HostChan& c = ctx->chans[t.chan];
         const int64_t rx = std::min<int64_t>(t.rx0 + v.ex, c.nx) - std::max(t.rx0, 0);
         const int64_t ry = std::min<int64_t>(t.ry0 + v.ey, c.ny) - std::max(t.ry0, 0);
-        loaded += 17.0 * (double)(rx * ry) + 8.0 * (double)t.xn * (double)t.yn;
+        loaded += 16.0 * (double)(rx * ry) + 8.0 * (double)t.xn * (double)t.yn;
     }
     if (unique_bytes) *unique_bytes = unique;
     if (loaded_bytes) *loaded_bytes = loaded;

@@ -75,24 +75,34 @@ void launch_lex_pipe(hipStream_t, int cls, int nchan, const ChanDesc*, ChanState
 struct TbVariant {
     int k;          // sweeps per launch
     int oxm, oym;   // largest output tile away from a channel's edges
-    int ex, ey;     // loaded region; the halo is (ex - oxm) / 2 = 2k + 4
+    int ex, ey;     // loaded region; the halo is (ex - oxm) / 2 = tb_halo(k)
     int nt;         // threads per workgroup
-    int codes;      // 1: keeps its per-thread cell codes in the codes table
+    int rows;       // rows per strip (a wave each)
 };
 extern const TbVariant TB_VARIANTS[];
 extern const int N_TB_VARIANTS;
-// mode bits: TB_CHECK, form the residual after the sweeps and stop on it;
-// TB_CODES_PUT / TB_CODES_GET, compute the cell codes from the flags and
-// store them in the codes table / load them from it (variants with codes).
-enum : int { TB_CHECK = 1, TB_CODES_PUT = 2, TB_CODES_GET = 4 };
-// codes table: 32 bytes per thread of every tile, at (tile idx * nt + thread)
-constexpr int TB_CODE_BYTES = 32;
+constexpr int tb_halo(int k) { return 2 * k + 2; }
+// What a wave of a tile holds (k_rb_codes): masks of its rows, and its form.
+struct TbWave {
+    uint32_t special;   // rows whose half-sweeps take the cells' codes
+    uint32_t rest;      // rows with output cells that no sweep changes
+    uint32_t form;      // TBW_GHOSTS: ghosts its lanes' words give; TBW_CODED
+    uint32_t pad;
+};
+static_assert(sizeof(TbWave) == 16, "one 16-byte scalar load per wave");
+enum : uint32_t { TBW_GHOSTS = 15, TBW_CODED = 16 };   // CODED: not all inner cells are updated
+// The waves' table has one entry per wave of every tile (by tile idx), the
+// words' table (rows + 1) * 64 words for each of them.
+void launch_rb_codes(hipStream_t, int variant, int ntb, const TbTile*, const uint8_t* flags,
+                     TbWave* waves, uint32_t* words);
+enum : int { TB_CHECK = 1 };   // mode: form the residual after the sweeps and stop on it
 // Launch L of a blocked solve: reads the partials of launch L - 1 from
-// part_prev, writes its own to part_cur (one double per tile).
+// part_prev, writes its own to part_cur (one double per tile).  The ghosts of
+// the input are fresh.
 void launch_rb_tb(hipStream_t, int variant, int ntb, const ChanDesc*, ChanState*, const TbTile*,
-                  const uint8_t* flags, const double* rhs, double* pa, double* pb,
-                  const double* part_prev, double* part_cur, int32_t* active,
-                  uint32_t* codes, int L, int mode);
+                  const TbWave* waves, const uint32_t* words, const double* rhs, double* pa,
+                  double* pb, const double* part_prev, double* part_cur, int32_t* active, int L,
+                  int mode);
 void launch_pbuf_fix(hipStream_t, int ntiles, int nchan, const ChanDesc*, ChanState*,
                      const Tile*, const double* pb, double* pa);
 
