@@ -638,7 +638,7 @@ __global__ void k_pbuf_reset(int nchan, ChanState* __restrict__ cs) {
 
 // Wide tiles of ten rows a strip suit grids of several rounds of workgroups;
 // the others are faster where a launch is one round (us per launch: 133 x 69
-// cells, K = 4: 24 x 128 regions 7.7, 48 x 128 8.8, 80 x 128 12.5; 1026 x 1026,
+// cells, K = 4: 32 x 128 regions 7.9, 48 x 128 8.8, 80 x 128 12.5; 1026 x 1026,
 // K = 6: 72 x 128 13.9, 80 x 128 14.5, 96 x 96 16.9; K = 8: 96 x 128 17.7, 80 x
 // 128 18.2, but at 4002 x 3002 178 and 136).
 //
@@ -649,7 +649,7 @@ __global__ void k_pbuf_reset(int nchan, ChanState* __restrict__ cs) {
     V(0, 1, 4, 64, 8)        \
     V(1, 2, 4, 64, 8)        \
     V(2, 4, 6, 64, 8)        \
-    V(3, 4, 4, 64, 6)        \
+    V(3, 4, 4, 64, 8)        \
     V(4, 4, 10, 64, 8)       \
     V(5, 6, 10, 64, 8)       \
     V(6, 8, 10, 64, 8)       \

@@ -15,7 +15,7 @@ from tests.refdata import assert_bits_equal
 pytestmark = pytest.mark.gpu
 
 # variant: (sweeps per launch, region's rows, region's pairs * 2)
-REGIONS = [(1, 32, 128), (2, 32, 128), (4, 48, 128), (4, 24, 128), (4, 80, 128), (6, 80, 128),
+REGIONS = [(1, 32, 128), (2, 32, 128), (4, 48, 128), (4, 32, 128), (4, 80, 128), (6, 80, 128),
            (8, 80, 128), (6, 72, 128), (8, 96, 128), (6, 96, 96)]
 
 
