@@ -41,34 +41,38 @@ void conv3x3(hipStream_t, const bf16* in, int cin, const bf16* w, const float* b
 bool conv_tiles_fit(int H, int W);
 void conv3x3_in(hipStream_t, const ConvIn& src, const bf16* w, const float* bias, bf16* out,
                 float* out32, int cout, int nb, int H, int W, int flags);
-// w'[ci][8 - tap][co] = w[co][tap][ci]: the backward-input weights
-void weight_flip(hipStream_t, const bf16* w, bf16* wt, int cin, int cout);
+// w'[ci][8 - tap][co] = w[co][tap][ci]: the backward-input weights of each layer
+// of the list, at the offset of its weights
+struct FlipList {
+    int n = 0;
+    int cin[16], cout[16];
+    int64_t off[16];
+    unsigned block[16];   // first workgroup of each layer (filled by weight_flip)
+};
+void weight_flip(hipStream_t, FlipList& layers, const bf16* w, bf16* wt);
 // The gradient and loss reductions leave per-block partial sums in `part`
 // (device scratch, reused launch after launch on one stream) and add them in
 // a fixed order, so a gradient is the same from run to run.  Sizes in floats:
 // grad_partials and loss_partials (nn_sizes.h).
-// dw32[co][tap][ci] += sum_pix gz[pix][co] * in[pix + off(tap)][ci]
-void conv3x3_dw(hipStream_t, const bf16* gz, int cout, const bf16* in, int cin, float* dw32, int nb,
-                int H, int W, float* part);
-void relu_bwd(hipStream_t, int64_t n, const bf16* y, bf16* g);
-// db[c] += sum_pix g[pix][c]
-void bias_grad(hipStream_t, const bf16* g, int c, int64_t npix, float* db, float* part);
+// Through a ReLU and a convolution's parameters: g = g * (y > 0);
+// db[c] += sum_pix g[pix][c]; dw32[co][tap][ci] += sum_pix g[pix][co] * in[pix + off(tap)][ci]
+// (bpart: the bias' partials, bias_partials floats).
+void conv_grads(hipStream_t, const bf16* y, bf16* g, int cout, const bf16* in, int cin,
+                float* dw32, float* db, int nb, int H, int W, float* part, float* bpart);
 void maxpool(hipStream_t, const bf16* x, bf16* y, int nb, int H, int W, int c,
              const int* live = nullptr);
 // accumulates into gx
 void maxpool_bwd(hipStream_t, const bf16* x, const bf16* y, const bf16* gy, bf16* gx, int nb,
                  int H, int W, int c);
-// x (nb, H/2, W/2, c) -> channels [c0, c0 + c) of y (nb, H, W, cy)
-void upsample(hipStream_t, const bf16* x, bf16* y, int nb, int H, int W, int c, int cy, int c0,
-              const int* live = nullptr);
-void upsample_bwd(hipStream_t, const bf16* gy, bf16* gx, int nb, int H, int W, int c, int cy,
-                  int c0);
-void channel_copy(hipStream_t, const bf16* src, int cs, int s0, bf16* dst, int cd, int d0, int c,
-                  int64_t npix, int add, const int* live = nullptr, int64_t hw = 1);
+// y (nb, H, W, ca + cb) = [x (nb, H/2, W/2, ca) upsampled, s (nb, H, W, cb)]
+void join(hipStream_t, const bf16* x, int ca, const bf16* s, int cb, bf16* y, int nb, int H, int W,
+          const int* live = nullptr);
+void join_bwd(hipStream_t, const bf16* gy, bf16* gx, int ca, bf16* gs, int cb, int nb, int H,
+              int W);
 void head(hipStream_t, const bf16* x, int c, const float* w, const float* b, float* y,
           int64_t npix, const int* live = nullptr, int64_t hw = 1);
-// gx = gy w; dw += sum gy x; db += sum gy
-void head_bwd(hipStream_t, const bf16* x, int c, const float* w, const float* gy, bf16* gx,
+// gx = gy w; dw += sum gy x; db += sum gy (32 channels)
+void head_bwd(hipStream_t, const bf16* x, const float* w, const float* gy, bf16* gx,
               float* dw, float* db, int64_t npix, float* part);
 // denom[s] = sum m t^2 of sample s; loss_out += the masked, normalised MSE; gy its gradient
 void loss(hipStream_t, const float* y, const float* t, const float* m, float* denom, float* gy,

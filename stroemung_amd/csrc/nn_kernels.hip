@@ -115,6 +115,81 @@ k_conv3x3(const bf16* __restrict__ in, int cin, const bf16* __restrict__ w,
     }
 }
 
+// The same product, term by term in the same order (taps outermost), for images
+// of at most 64 pixels whose sides the tiles below do not divide: the deep
+// levels of a small frame.  A workgroup holds one whole image with its border of
+// zeros in LDS (all its channels), and each of its four waves one 16-pixel by
+// 16-channel tile.  A channel's weights are contiguous in the order they are
+// used, so a lane streams its own from L2, nine steps ahead.  The kernel above
+// waits for two loads from memory at every step, with a workgroup on a few CUs:
+// 31 us for 32 images of 8 x 4 pixels and 256 to 256 channels, 13.8 here.
+constexpr int SMALL_PIXELS = 64, SMALL_LDS = 64 * 1024;
+static inline int small_patch_bytes(int cin, int H, int W) {
+    return (H + 2) * (W + 2) * (cin + 8) * (int)sizeof(bf16);
+}
+__global__ void __launch_bounds__(256)
+k_conv3x3_small(const bf16* __restrict__ in, int cin, const bf16* __restrict__ w,
+                const float* __restrict__ bias, bf16* __restrict__ out, float* __restrict__ out32,
+                int cout, int H, int W, int mt, int flags, const int* __restrict__ live)
+{
+    extern __shared__ __attribute__((aligned(16))) bf16 patch[];   // [(H + 2) (W + 2)][cin + 8]
+    const int img = blockIdx.x, HW = H * W, PW = W + 2, cs = cin + 8;
+    if (live && img >= *live) return;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int row = lane & 15, kq = (lane >> 4) * 8;
+    const int nv = cin / 8;
+    for (int v = tid; v < (H + 2) * PW * nv; v += 256) {
+        const int px = v / nv, c = (v - px * nv) * 8, y = px / PW - 1, x = px - px / PW * PW - 1;
+        const bool inside = y >= 0 && y < H && x >= 0 && x < W;
+        const int64_t from = ((int64_t)img * HW + (inside ? y * W + x : 0)) * cin + c;
+        const bf16x8 q = load8(in + from);
+        *reinterpret_cast<bf16x8*>(&patch[px * cs + c]) = inside ? q : zero8();
+    }
+    __syncthreads();
+    const int tile = wave & (mt - 1), n0 = (blockIdx.y * (4 / mt) + wave / mt) * 16;
+    if (n0 >= cout || tile * 16 >= HW) return;
+    const int pix = min(tile * 16 + row, HW - 1), py = pix / W, px = pix - py * W;
+    const bf16* pa = &patch[(py * PW + px) * cs + kq];   // tap 0: one row up, one left
+    const bf16* pw = w + (int64_t)(n0 + row) * 9 * cin + kq;
+    // steps of 32 k's: tap-major, then the channels; nine at a time
+    const int per = cin / 32, batches = per;             // 9 * per steps
+    bf16x8 cur[9], nxt[9];
+#pragma unroll
+    for (int j = 0; j < 9; j++) cur[j] = load8(pw + j * 32);
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    int tap = 0, c = 0;
+    for (int b = 0; b < batches; b++) {
+        const bf16* ahead = pw + (int64_t)min(b + 1, batches - 1) * 9 * 32;
+#pragma unroll
+        for (int j = 0; j < 9; j++) nxt[j] = load8(ahead + j * 32);
+        __builtin_amdgcn_sched_barrier(0);   // the loads issue before the MFMAs
+#pragma unroll
+        for (int j = 0; j < 9; j++) {
+            const bf16x8 a = load8(pa + (tap / 3 * PW + tap % 3) * cs + c * 32);
+            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, cur[j], acc, 0, 0, 0);
+            if (++c == per) {
+                c = 0;
+                tap++;
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int j = 0; j < 9; j++) cur[j] = nxt[j];
+    }
+    const int n = n0 + row;
+    const float bv = (flags & 1) ? bias[n] : 0.f;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const int p = tile * 16 + (lane >> 4) * 4 + i;
+        if (p >= HW) continue;
+        float v = acc[i] + bv;
+        if (flags & 2) v = v > 0.f ? v : 0.f;
+        const int64_t o = ((int64_t)img * HW + p) * cout + n;
+        if (out) out[o] = (bf16)v;
+        if (out32) out32[o] = v;
+    }
+}
+
 // LDS-tiled variant.  A workgroup owns a TH x TW pixel tile of one image
 // (TH * TW = 64 or 128) and NW = 32 * WN output channels; for every
 // 32-channel slice of the input it stages in LDS the (TH + 2) x (TW + 2)
@@ -444,134 +519,235 @@ k_conv_finish(const float* __restrict__ acc32, int ks, const float* __restrict__
     if (out32) *reinterpret_cast<float4*>(out32 + k) = v;
 }
 
-// w'[ci][8 - tap][co] = w[co][tap][ci]
-__global__ void k_weight_flip(const bf16* __restrict__ w, bf16* __restrict__ wt, int cin, int cout)
+// w'[ci][8 - tap][co] = w[co][tap][ci] for every layer of the list, each at the
+// offset of its own weights: one launch in front of the backward pass (3.7 us
+// for each layer by itself before, 12.6 for all now)
+__global__ void __launch_bounds__(256)
+k_weight_flip(FlipList l, const bf16* __restrict__ w, bf16* __restrict__ wt)
 {
-    const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int64_t n = (int64_t)cin * 9 * cout;
-    if (k >= n) return;
-    const int ci = (int)(k % cin);
-    const int tap = (int)((k / cin) % 9);
-    const int co = (int)(k / ((int64_t)cin * 9));
-    wt[((int64_t)ci * 9 + (8 - tap)) * cout + co] = w[k];
+    int k = 0;
+    while (k + 1 < l.n && blockIdx.x >= l.block[k + 1]) k++;
+    const int cin = l.cin[k], cout = l.cout[k];
+    // consecutive threads take consecutive co: the stores are contiguous
+    const int i = (blockIdx.x - l.block[k]) * 256 + threadIdx.x;
+    if (i >= cin * 9 * cout) return;
+    const int co = i % cout, t = i / cout, tap = t % 9, ci = t / 9;
+    wt[l.off[k] + i] = w[l.off[k] + ((int64_t)co * 9 + 8 - tap) * cin + ci];
 }
 
 // dw[co][tap][ci] over a pixel chunk: sum of gz[pix][co] * in[pix+off][ci].
-// Block: 256 threads, a tile of up to 64 co x 64 ci for one tap; chunks of
-// 128 pixels are staged transposed in LDS ([channel][pixel]) so each lane's 8
-// consecutive pixels (the MFMA's k) are one 16-byte read.  The four waves
-// cover the tile in 32 x 32 pieces and split the chunk's four 32-pixel k
-// steps among themselves when the tile is narrower than 64 x 64, so no wave
+// Block: 256 threads, a tile of up to 64 co x 64 ci for the three taps of one
+// dy.  The MFMAs' k is the pixel, so both operands are read transposed: 128
+// pixels at a time are staged as they lie in memory (gz's rows, and of `in` the
+// 130 pixels that the three dx reach, whatever the width), and
+// ds_read_b64_tr_b16 hands lane c of 16 the channel c of four pixels; a lane
+// whose pixel has no neighbour there reads a row of zeros instead.  The next
+// 128 pixels are loaded while these are multiplied.  Transposing with 2-byte
+// LDS stores, for each tap by itself, was what bounded the pass before: 29.7 us
+// on average over the 14 layers of 32 frames of 64 x 64, 16.0
+// now.  What bounds a round is the transposed reads (16 for 12 MFMAs): eight
+// waves with 32 x 16 pieces, loads two and three rounds ahead and a pixel padded
+// to 160 bytes measured 15.7 to 16.6.
+//
+// The four waves cover the tile in 32 x 32 pieces and split the four 32-pixel
+// k steps among themselves when the tile is narrower than 64 x 64, so no wave
 // multiplies padding; those waves then add their sums in LDS in wave order.
 // With one pixel chunk (chunk_stride 0) the block adds its sums into dw; with
 // several, chunk z writes its own slice out[z * chunk_stride + ...] and
 // k_chunk_sum adds the slices in chunk order, so the result does not depend
 // on the order in which blocks finish.
+template <int CO, int CI>   // the tile: 32 or 64 of each
 __global__ void __launch_bounds__(256)
 k_conv3x3_dw(const bf16* __restrict__ gz, int cout, const bf16* __restrict__ in, int cin,
-             float* __restrict__ out, int64_t chunk_stride, int nb, int H, int W,
+             int ci_first, float* __restrict__ out, int64_t chunk_stride, int nb, int H, int W,
              int pix_per_block)
 {
-    constexpr int KP = 128, LS = KP + 8;
-    __shared__ __attribute__((aligned(16))) bf16 smem[2][64][LS];
-    bf16 (*sa)[LS] = smem[0];   // [co][pix]
-    bf16 (*sb)[LS] = smem[1];   // [ci][pix]
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int tap = blockIdx.z % 9;
-    const int dy = tap / 3 - 1, dx = tap % 3 - 1;
-    const int co0 = blockIdx.y * 64;
-    const int ci0 = blockIdx.x * 64;
+    // KP pixels at once; a staged pixel takes LS channels (144 bytes: the 16
+    // rows of a read then cover the banks evenly)
+    constexpr int KP = 128, WP = KP + 2, LS = 72;
+    constexpr int GV = CO / 8, IV = CI / 8;                       // 16-byte vectors of a pixel
+    constexpr int NG = KP * GV / 256, NI = (WP * IV + 255) / 256; // of them per thread
+    constexpr int WO = CO / 32, WI = CI / 32, KS = 4 / (WO * WI);
+    __shared__ __attribute__((aligned(16))) bf16 smem[(KP + WP + 1) * LS];
+    __shared__ uint8_t near[KP];   // bit dx + 1: the pixel has that neighbour in row h + dy
+    bf16* sg = smem;               // [pixel][co]
+    bf16* si = smem + KP * LS;     // [pixel + dx + 1][ci], then a row of zeros
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int dy = (int)(blockIdx.z % 3) - 1;
+    const int co0 = blockIdx.y * CO;
+    const int ci0 = ci_first + blockIdx.x * CI;
     const int npix = nb * H * W;
-    const int p_begin = (blockIdx.z / 9) * pix_per_block;
+    const int p_begin = (blockIdx.z / 3) * pix_per_block;
     const int p_end = min(npix, p_begin + pix_per_block);
-    const int ci_n = cin - ci0 < 64 ? cin - ci0 : 64;    // 32 or 64
-    const int co_n = cout - co0 < 64 ? cout - co0 : 64;
-    const int wo = co_n / 32, wi = ci_n / 32, ks = 4 / (wo * wi);
-    const int mo = wave % wo, ni = (wave / wo) % wi, kg = wave / (wo * wi);
-    f32x4 acc[2][2];
-    for (int t = 0; t < 2; t++)
-        for (int u = 0; u < 2; u++) acc[t][u] = f32x4{0.f, 0.f, 0.f, 0.f};
-    const int row = lane & 15, kq = (lane >> 4) * 8;
-    // staging: thread -> pixel j = tid / 2, channels [32 h, 32 h + 32), h = tid % 2
-    const int sj = threadIdx.x >> 1, sh = (threadIdx.x & 1) * 32;
+    const int mo = wave % WO, ni = wave / WO % WI, kg = wave / (WO * WI);
+    f32x4 acc[3][2][2];
+    for (int x = 0; x < 3; x++)
+        for (int t = 0; t < 2; t++)
+            for (int u = 0; u < 2; u++) acc[x][t][u] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const int row = lane & 15;
+
+    // a thread's vectors of the next 128 pixels: loaded from addresses clamped
+    // into the batch, without branches, and zeroed when stored if they lie
+    // outside the chunk
+    bf16x8 vg[NG], vi[NI];
+    uint32_t edge = 0;
+    auto fetch = [&](int p0) {
+#pragma unroll
+        for (int k = 0; k < NG; k++) {
+            const int v = tid + k * 256, pix = min(p0 + v / GV, npix - 1);
+            vg[k] = load8(gz + (int64_t)pix * cout + co0 + v % GV * 8);
+        }
+#pragma unroll
+        for (int k = 0; k < NI; k++) {
+            const int v = min(tid + k * 256, WP * IV - 1);
+            const int pix = min(max(p0 + dy * W - 1 + v / IV, 0), npix - 1);
+            vi[k] = load8(in + (int64_t)pix * cin + ci0 + v % IV * 8);
+        }
+        const int pix = p0 + (tid & (KP - 1)), w = pix % W, hh = pix / W % H + dy;
+        const bool inside = pix < p_end && hh >= 0 && hh < H;
+        edge = inside ? (w > 0 ? 1u : 0u) | 2u | (w + 1 < W ? 4u : 0u) : 0u;
+    };
+    if (tid < LS / 8) *reinterpret_cast<bf16x8*>(&si[WP * LS + tid * 8]) = zero8();
+
+    // a transposed read's source: pixel 8 (lane / 16) + row / 4 (+ 4), four channels
+    const int src = (8 * (lane >> 4) + row / 4) * LS + 4 * (row % 4);
+    typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+    typedef __attribute__((address_space(3))) bf16x4 lds4;
+    auto pair = [](const bf16* lo, const bf16* hi) -> bf16x8 {
+        const bf16x4 a = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds4*)lo);
+        const bf16x4 b = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds4*)hi);
+        return __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7);
+    };
+    fetch(p_begin);
     for (int p0 = p_begin; p0 < p_end; p0 += KP) {
-        const int pix = p0 + sj;
-        bf16x8 va[4], vb[4];
-        for (int q = 0; q < 4; q++) {
-            va[q] = zero8();
-            vb[q] = zero8();
-        }
-        if (pix < p_end) {
-            const int b = pix / (H * W), r = pix - b * H * W;
-            const int hh = r / W + dy, ww = r % W + dx;
-            const bool inside = hh >= 0 && hh < H && ww >= 0 && ww < W;
-            for (int q = 0; q < 4; q++) {
-                const int c = sh + q * 8;
-                if (c < co_n) va[q] = load8(gz + (int64_t)pix * cout + co0 + c);
-                if (inside && c < ci_n)
-                    vb[q] = load8(in + ((int64_t)(b * H + hh) * W + ww) * cin + ci0 + c);
-            }
-        }
         __syncthreads();
-        for (int q = 0; q < 4; q++)
-            for (int i = 0; i < 8; i++) {
-                sa[sh + q * 8 + i][sj] = va[q][i];
-                sb[sh + q * 8 + i][sj] = vb[q][i];
-            }
+#pragma unroll
+        for (int k = 0; k < NG; k++) {
+            const int v = tid + k * 256;
+            *reinterpret_cast<bf16x8*>(&sg[v / GV * LS + v % GV * 8]) =
+                p0 + v / GV < p_end ? vg[k] : zero8();
+        }
+#pragma unroll
+        for (int k = 0; k < NI; k++) {   // (a pixel that is no neighbour is not read)
+            const int v = tid + k * 256;
+            if (v < WP * IV) *reinterpret_cast<bf16x8*>(&si[v / IV * LS + v % IV * 8]) = vi[k];
+        }
+        if (tid < KP) near[tid] = (uint8_t)edge;
         __syncthreads();
-        for (int k = kg; k < 4; k += ks) {
-            bf16x8 a[2], bb[2];
-            for (int t = 0; t < 2; t++) a[t] = load8(&sa[mo * 32 + t * 16 + row][k * 32 + kq]);
-            for (int u = 0; u < 2; u++) bb[u] = load8(&sb[ni * 32 + u * 16 + row][k * 32 + kq]);
-            for (int t = 0; t < 2; t++)
-                for (int u = 0; u < 2; u++)
-                    acc[t][u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[t], bb[u], acc[t][u], 0, 0, 0);
+        fetch(p0 + KP);   // (past the chunk's end: loaded, not used)
+        __builtin_amdgcn_sched_barrier(0);   // the loads issue before the MFMAs
+        uint32_t n0[4 / KS], n1[4 / KS];
+#pragma unroll
+        for (int j = 0; j < 4 / KS; j++) {
+            const int px = (kg + j * KS) * 32 + 8 * (lane >> 4) + row / 4;
+            n0[j] = near[px];
+            n1[j] = near[px + 4];
+        }
+#pragma unroll
+        for (int j = 0; j < 4 / KS; j++) {
+            const int k = kg + j * KS;
+            const bf16* ga = sg + k * 32 * LS + src + mo * 32;
+            bf16x8 a[2];
+#pragma unroll
+            for (int t = 0; t < 2; t++) a[t] = pair(ga + t * 16, ga + t * 16 + 4 * LS);
+#pragma unroll
+            for (int x = 0; x < 3; x++) {
+                const bf16* ib = si + (k * 32 + x) * LS + src;
+                const bf16* zero = si + WP * LS;
+                const bf16* lo = ((n0[j] >> x) & 1u ? ib : zero) + ni * 32;
+                const bf16* hi = ((n1[j] >> x) & 1u ? ib + 4 * LS : zero) + ni * 32;
+#pragma unroll
+                for (int u = 0; u < 2; u++) {
+                    const bf16x8 b = pair(lo + u * 16, hi + u * 16);
+#pragma unroll
+                    for (int t = 0; t < 2; t++)
+                        acc[x][t][u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[t], b, acc[x][t][u],
+                                                                              0, 0, 0);
+                }
+            }
         }
     }
-    if (ks > 1) {
-        // wave w + g * wo * wi holds k group g of wave w's piece: 16 floats a
-        // lane, 4 KB a wave, in the staging memory (34 KB) once every wave is
-        // past its last MFMA read
-        float* red = reinterpret_cast<float*>(&smem[0][0][0]);
-        __syncthreads();
-        if (kg > 0)
-            for (int t = 0; t < 2; t++)
-                for (int u = 0; u < 2; u++)
-                    for (int i = 0; i < 4; i++)
-                        red[(wave * 16 + (t * 2 + u) * 4 + i) * 64 + lane] = acc[t][u][i];
-        __syncthreads();
-        if (kg == 0)
-            for (int g = 1; g < ks; g++) {
-                const int w2 = wave + g * wo * wi;
+    if (KS > 1) {
+#pragma unroll
+        for (int x = 0; x < 3; x++) {
+            // wave w + g * WO * WI holds k group g of wave w's piece: 16 floats a
+            // lane, 4 KB a wave, in the staging memory once every wave is past
+            // its last read of it
+            float* red = reinterpret_cast<float*>(smem);
+            __syncthreads();
+            if (kg > 0)
                 for (int t = 0; t < 2; t++)
                     for (int u = 0; u < 2; u++)
                         for (int i = 0; i < 4; i++)
-                            acc[t][u][i] += red[(w2 * 16 + (t * 2 + u) * 4 + i) * 64 + lane];
-            }
-    }
-    if (kg != 0) return;
-    float* dst = out + (int64_t)(blockIdx.z / 9) * chunk_stride;
-    for (int t = 0; t < 2; t++)
-        for (int u = 0; u < 2; u++) {
-            const int ci = ci0 + ni * 32 + u * 16 + row;
-            for (int i = 0; i < 4; i++) {
-                const int co = co0 + mo * 32 + t * 16 + (lane >> 4) * 4 + i;
-                const int64_t o = ((int64_t)co * 9 + tap) * cin + ci;
-                dst[o] = chunk_stride ? acc[t][u][i] : dst[o] + acc[t][u][i];
-            }
+                            red[(wave * 16 + (t * 2 + u) * 4 + i) * 64 + lane] = acc[x][t][u][i];
+            __syncthreads();
+            if (kg == 0)
+                for (int g = 1; g < KS; g++) {
+                    const int w2 = wave + g * WO * WI;
+                    for (int t = 0; t < 2; t++)
+                        for (int u = 0; u < 2; u++)
+                            for (int i = 0; i < 4; i++)
+                                acc[x][t][u][i] += red[(w2 * 16 + (t * 2 + u) * 4 + i) * 64 + lane];
+                }
         }
+        if (kg != 0) return;
+    }
+    // the wave's piece: lane l % 16 is a ci, so each store writes four runs of 64 bytes
+    const int cr = co0 + mo * 32 + (lane >> 4) * 4, cc = ci0 + ni * 32 + row;
+    float* dst = out + (int64_t)(blockIdx.z / 3) * chunk_stride + ((int64_t)cr * 9 + (dy + 1) * 3) * cin + cc;
+    auto at = [&](int x, int t, int u, int i) -> float& {
+        return dst[((t * 16 + i) * 9 + x) * cin + u * 16];
+    };
+    if (chunk_stride == 0) {   // the loads together, before any store
+        float old[3][2][2][4];
+#pragma unroll
+        for (int k = 0; k < 48; k++)
+            old[k / 16][k / 8 % 2][k / 4 % 2][k % 4] = at(k / 16, k / 8 % 2, k / 4 % 2, k % 4);
+#pragma unroll
+        for (int k = 0; k < 48; k++)
+            acc[k / 16][k / 8 % 2][k / 4 % 2][k % 4] =
+                old[k / 16][k / 8 % 2][k / 4 % 2][k % 4] + acc[k / 16][k / 8 % 2][k / 4 % 2][k % 4];
+    }
+#pragma unroll
+    for (int k = 0; k < 48; k++)
+        at(k / 16, k / 8 % 2, k / 4 % 2, k % 4) = acc[k / 16][k / 8 % 2][k / 4 % 2][k % 4];
 }
 
-// dst[i] += part[i] + part[n + i] + ... + part[(chunks - 1) n + i], in that order
-__global__ void k_chunk_sum(const float* __restrict__ part, int chunks, int64_t n,
-                            float* __restrict__ dst)
+// The sum of a block's 256 values in a fixed LDS tree; for thread 0.
+__device__ __forceinline__ float tree256(float s, float* red) {
+    red[threadIdx.x] = s;
+    __syncthreads();
+    for (int st = 128; st > 0; st >>= 1) {
+        if (threadIdx.x < st) red[threadIdx.x] += red[threadIdx.x + st];
+        __syncthreads();
+    }
+    return red[0];
+}
+
+// A layer's partial gradients into its gradients, in one launch.  Weights (the
+// blocks from `c` on, none if there was one chunk): dw[i] += part[i] + part[n +
+// i] + ... + part[(chunks - 1) n + i], in that order.  Bias channel j (block j):
+// db[j] += the sum over k of bpart[k * c + j], thread t adding k = t, t + 256,
+// ... in order, then a fixed LDS tree.
+__global__ void __launch_bounds__(256)
+k_grad_finish(const float* __restrict__ part, int chunks, int64_t n, float* __restrict__ dw,
+              const float* __restrict__ bpart, int nparts, int c, float* __restrict__ db)
 {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    __shared__ float red[256];
+    const int j = blockIdx.x;
+    if (j < c) {
+        float s = 0.f;
+        for (int k = threadIdx.x; k < nparts; k += 256) s += bpart[(int64_t)k * c + j];
+        s = tree256(s, red);
+        if (threadIdx.x == 0) db[j] = db[j] + s;
+        return;
+    }
+    const int64_t i = (int64_t)(j - c) * 256 + threadIdx.x;
     if (i >= n) return;
     float s = part[i];
 #pragma unroll 8
-    for (int c = 1; c < chunks; c++) s += part[(int64_t)c * n + i];
-    dst[i] += s;
+    for (int k = 1; k < chunks; k++) s += part[(int64_t)k * n + i];
+    dw[i] += s;
 }
 
 // Block j: the sum over k of part[k * stride + col0 + j], k in [0, nparts):
@@ -585,42 +761,48 @@ k_block_sum(const float* __restrict__ part, int nparts, int stride, int col0,
     const int j = blockIdx.x;
     float s = 0.f;
     for (int k = threadIdx.x; k < nparts; k += 256) s += part[(int64_t)k * stride + col0 + j];
-    red[threadIdx.x] = s;
-    __syncthreads();
-    for (int st = 128; st > 0; st >>= 1) {
-        if (threadIdx.x < st) red[threadIdx.x] += red[threadIdx.x + st];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) dst[j] = add ? dst[j] + red[0] : red[0];
+    s = tree256(s, red);
+    if (threadIdx.x == 0) dst[j] = add ? dst[j] + s : s;
 }
 
 // ------------------------------------------------------------ elementwise
 
-// g = g * (y > 0): gradient through a ReLU whose output is y
-__global__ void k_relu_bwd(int64_t n, const bf16* __restrict__ y, bf16* __restrict__ g)
-{
-    const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (k < n && !((float)y[k] > 0.f)) g[k] = (bf16)0.f;
-}
-
-// part[block][c] = sum over the block's pixels of g[pix][c].  c is 32, 64,
-// 128 or 256: thread t takes the 8 channels of vector v = t % (c / 8) (one
-// 16-byte load per pixel) for pixels j, j + lanes, ... of the block's chunk
-// (j = t / (c / 8), lanes = 256 / (c / 8)), each channel added in pixel
-// order; then the lanes' partials of each channel are added in LDS in lane
-// order.  The loads of several pixels are in flight at once.
+// The gradient through a ReLU whose output is y, g = g * (y > 0), and its sums
+// for the bias: part[block][c] = sum over the block's pixels of g[pix][c].  c is
+// 32, 64, 128 or 256: thread t takes the 8 channels of vector v = t % (c / 8)
+// (one 16-byte load per pixel) for pixels j, j + lanes, ... of the block's chunk
+// (j = t / (c / 8), lanes = 256 / (c / 8)), each channel added in pixel order;
+// then the lanes' partials of each channel are added in LDS in lane order.  The
+// loads of several pixels are in flight at once.  (Bound by memory; in two
+// passes, the first a value per thread, 9.4 us a layer on average at 32 frames
+// of 64 x 64, 5.4 now.)
 __global__ void __launch_bounds__(256)
-k_bias_grad(const bf16* __restrict__ g, int c, int npix, int per, float* __restrict__ part)
+k_relu_bias_bwd(const bf16* __restrict__ y, bf16* __restrict__ g, int c, int npix, int per,
+                float* __restrict__ part)
 {
     __shared__ float red[256 * 8];
     const int nv = c / 8, v = threadIdx.x % nv, j = threadIdx.x / nv, lanes = 256 / nv;
     const int p0 = blockIdx.x * per, p1 = min(npix, p0 + per);
     float s[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-#pragma unroll 4
-    for (int p = p0 + j; p < p1; p += lanes) {
-        const bf16x8 x = load8(g + (int64_t)p * c + v * 8);
+    constexpr int U = 4;
+    for (int p = p0 + j; p < p1; p += U * lanes) {
+        bf16x8 x[U], o[U];
 #pragma unroll
-        for (int e = 0; e < 8; e++) s[e] += (float)x[e];
+        for (int u = 0; u < U; u++) {
+            const int64_t at = (int64_t)min(p + u * lanes, p1 - 1) * c + v * 8;
+            x[u] = load8(g + at);
+            o[u] = load8(y + at);
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            if (p + u * lanes >= p1) break;
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                if (!((float)o[u][e] > 0.f)) x[u][e] = (bf16)0.f;
+                s[e] += (float)x[u][e];
+            }
+            *reinterpret_cast<bf16x8*>(g + (int64_t)(p + u * lanes) * c + v * 8) = x[u];
+        }
     }
 #pragma unroll
     for (int e = 0; e < 8; e++) red[threadIdx.x * 8 + e] = s[e];
@@ -633,93 +815,120 @@ k_bias_grad(const bf16* __restrict__ g, int c, int npix, int per, float* __restr
     }
 }
 
+// The elementwise passes take eight channels a thread, one 16-byte access each:
+// they are bound by memory (upsampling to 64 x 64 x 64 of 32 frames 17.7 us and
+// 6.1 for the skip's copy with a channel a thread, 6.1 together now).
+__device__ __forceinline__ void store8(bf16* p, bf16x8 v) { *reinterpret_cast<bf16x8*>(p) = v; }
+
 // 2x2 max pooling, H and W even
-__global__ void k_maxpool(const bf16* __restrict__ x, bf16* __restrict__ y, int nb, int H, int W, int c,
-                          const int* __restrict__ live)
+__global__ void __launch_bounds__(256)
+k_maxpool(const bf16* __restrict__ x, bf16* __restrict__ y, int nb, int H, int W, int c,
+          const int* __restrict__ live)
 {
     const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int Ho = H / 2, Wo = W / 2;
-    const int64_t n = (int64_t)(live ? min(nb, *live) : nb) * Ho * Wo * c;
+    const int Ho = H / 2, Wo = W / 2, nv = c / 8;
+    const int64_t n = (int64_t)(live ? min(nb, *live) : nb) * Ho * Wo * nv;
     if (k >= n) return;
-    const int ch = (int)(k % c);
-    const int64_t q = k / c;
+    const int ch = (int)(k % nv) * 8;
+    const int64_t q = k / nv;
     const int wo = (int)(q % Wo), ho = (int)((q / Wo) % Ho), b = (int)(q / ((int64_t)Wo * Ho));
-    const int64_t base = ((int64_t)(b * H + 2 * ho) * W + 2 * wo) * c + ch;
-    float m = (float)x[base];
-    m = fmaxf(m, (float)x[base + c]);
-    m = fmaxf(m, (float)x[base + (int64_t)W * c]);
-    m = fmaxf(m, (float)x[base + (int64_t)W * c + c]);
-    y[k] = (bf16)m;
+    const int64_t base = ((int64_t)(b * H + 2 * ho) * W + 2 * wo) * c + ch, down = (int64_t)W * c;
+    const bf16x8 v[4] = {load8(x + base), load8(x + base + c), load8(x + base + down),
+                         load8(x + base + down + c)};
+    bf16x8 r;
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+        float m = fmaxf((float)v[0][e], (float)v[1][e]);
+        m = fmaxf(m, (float)v[2][e]);
+        r[e] = (bf16)fmaxf(m, (float)v[3][e]);
+    }
+    store8(y + k * 8, r);
 }
 
 // gradient of max pooling: to the first maximal input of each window
-__global__ void k_maxpool_bwd(const bf16* __restrict__ x, const bf16* __restrict__ y,
-                              const bf16* __restrict__ gy, bf16* __restrict__ gx, int nb, int H,
-                              int W, int c)
+__global__ void __launch_bounds__(256)
+k_maxpool_bwd(const bf16* __restrict__ x, const bf16* __restrict__ y, const bf16* __restrict__ gy,
+              bf16* __restrict__ gx, int nb, int H, int W, int c)
 {
     const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int Ho = H / 2, Wo = W / 2;
-    const int64_t n = (int64_t)nb * Ho * Wo * c;
+    const int Ho = H / 2, Wo = W / 2, nv = c / 8;
+    const int64_t n = (int64_t)nb * Ho * Wo * nv;
     if (k >= n) return;
-    const int ch = (int)(k % c);
-    const int64_t q = k / c;
+    const int ch = (int)(k % nv) * 8;
+    const int64_t q = k / nv;
     const int wo = (int)(q % Wo), ho = (int)((q / Wo) % Ho), b = (int)(q / ((int64_t)Wo * Ho));
     const int64_t base = ((int64_t)(b * H + 2 * ho) * W + 2 * wo) * c + ch;
     const int64_t off[4] = {0, c, (int64_t)W * c, (int64_t)W * c + c};
-    const float m = (float)y[k];
-    int hit = 0;
+    bf16x8 v[4], g[4];
+#pragma unroll
     for (int i = 0; i < 4; i++) {
-        const bool take = !hit && (float)x[base + off[i]] == m;
-        if (take) gx[base + off[i]] = (bf16)((float)gx[base + off[i]] + (float)gy[k]);
-        hit |= take;
+        v[i] = load8(x + base + off[i]);
+        g[i] = load8(gx + base + off[i]);
     }
+    const bf16x8 m = load8(y + k * 8), t = load8(gy + k * 8);
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+        bool hit = false;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const bool take = !hit && (float)v[i][e] == (float)m[e];
+            if (take) g[i][e] = (bf16)((float)g[i][e] + (float)t[e]);
+            hit = hit || take;
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < 4; i++) store8(gx + base + off[i], g[i]);
 }
 
-// nearest 2x upsampling of x (nb, H/2, W/2, c) into channels [c0, c0 + c) of
-// y (nb, H, W, cy) -- the concatenation with the skip happens in place
-__global__ void k_upsample(const bf16* __restrict__ x, bf16* __restrict__ y, int nb, int H, int W,
-                           int c, int cy, int c0, const int* __restrict__ live)
+// The input of a decoder convolution: the nearest 2x upsampling of x (nb, H/2,
+// W/2, ca) in channels [0, ca) of y (nb, H, W, ca + cb), the skip s in the rest
+__global__ void __launch_bounds__(256)
+k_join(const bf16* __restrict__ x, int ca, const bf16* __restrict__ s, int cb,
+       bf16* __restrict__ y, int nb, int H, int W, const int* __restrict__ live)
 {
     const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int64_t n = (int64_t)(live ? min(nb, *live) : nb) * H * W * c;
+    const int nv = (ca + cb) / 8;
+    const int64_t n = (int64_t)(live ? min(nb, *live) : nb) * H * W * nv;
     if (k >= n) return;
-    const int ch = (int)(k % c);
-    const int64_t q = k / c;
+    const int ch = (int)(k % nv) * 8;
+    const int64_t q = k / nv;
     const int w = (int)(q % W), h = (int)((q / W) % H), b = (int)(q / ((int64_t)W * H));
-    y[q * cy + c0 + ch] = x[((int64_t)(b * (H / 2) + h / 2) * (W / 2) + w / 2) * c + ch];
+    const bf16* from = ch < ca ? x + ((int64_t)(b * (H / 2) + h / 2) * (W / 2) + w / 2) * ca + ch
+                               : s + q * cb + ch - ca;
+    store8(y + k * 8, load8(from));
 }
 
-__global__ void k_upsample_bwd(const bf16* __restrict__ gy, bf16* __restrict__ gx, int nb, int H,
-                               int W, int c, int cy, int c0)
+// Its backward: gx = the sums of gy's channels [0, ca) over each 2 x 2 block, gs
+// = its channels [ca, ca + cb).  A thread takes one block of eight channels.
+__global__ void __launch_bounds__(256)
+k_join_bwd(const bf16* __restrict__ gy, bf16* __restrict__ gx, int ca, bf16* __restrict__ gs,
+           int cb, int nb, int H, int W)
 {
     const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int Ho = H / 2, Wo = W / 2;
-    const int64_t n = (int64_t)nb * Ho * Wo * c;
-    if (k >= n) return;
-    const int ch = (int)(k % c);
-    const int64_t q = k / c;
+    const int Ho = H / 2, Wo = W / 2, cy = ca + cb, nv = cy / 8;
+    if (k >= (int64_t)nb * Ho * Wo * nv) return;
+    const int ch = (int)(k % nv) * 8;
+    const int64_t q = k / nv;
     const int wo = (int)(q % Wo), ho = (int)((q / Wo) % Ho), b = (int)(q / ((int64_t)Wo * Ho));
-    float s = 0.f;
-    for (int i = 0; i < 2; i++)
-        for (int j = 0; j < 2; j++)
-            s += (float)gy[((int64_t)(b * H + 2 * ho + i) * W + 2 * wo + j) * cy + c0 + ch];
-    gx[k] = (bf16)s;
-}
-
-// copy channels: y[:, c0:c0+c] = x (forward of the skip half of a concat) or
-// x = y[:, c0:c0+c] (its backward), add = accumulate into x
-__global__ void k_channel_copy(const bf16* __restrict__ src, int cs, int s0, bf16* __restrict__ dst,
-                               int cd, int d0, int c, int64_t npix, int add,
-                               const int* __restrict__ live, int64_t hw)
-{
-    const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= npix * c) return;
-    if (live && k / c >= (int64_t)*live * hw) return;
-    const int ch = (int)(k % c);
-    const int64_t p = k / c;
-    const bf16 v = src[p * cs + s0 + ch];
-    bf16& d = dst[p * cd + d0 + ch];
-    d = add ? (bf16)((float)d + (float)v) : v;
+    const int64_t p = (int64_t)(b * H + 2 * ho) * W + 2 * wo;
+    const int64_t at[4] = {p, p + 1, p + W, p + W + 1};
+    bf16x8 v[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) v[i] = load8(gy + at[i] * cy + ch);
+    if (ch < ca) {
+        bf16x8 r;
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+            float s = 0.f;
+#pragma unroll
+            for (int i = 0; i < 4; i++) s += (float)v[i][e];
+            r[e] = (bf16)s;
+        }
+        store8(gx + q * ca + ch, r);
+    } else {
+#pragma unroll
+        for (int i = 0; i < 4; i++) store8(gs + at[i] * cb + ch - ca, v[i]);
+    }
 }
 
 // 1x1 head: y[pix] = b + sum_c x[pix, c] * w[c]   (fp32 out)
@@ -740,29 +949,55 @@ __global__ void k_head(const bf16* __restrict__ x, int c, const float* __restric
     y[p] = s;
 }
 
-// head backward: gx[pix, c] = gy[pix] * w[c]; per block, part[block][0] = sum gy
-// and part[block][1 + c] = sum gy * x[c] over the block's pixels
-__global__ void k_head_bwd(const bf16* __restrict__ x, int c, const float* __restrict__ w,
-                           const float* __restrict__ gy, bf16* __restrict__ gx,
-                           float* __restrict__ part, int64_t npix)
+// head backward (32 channels): gx[pix, c] = gy[pix] * w[c]; per block,
+// part[block][0] = sum gy and part[block][1 + c] = sum gy * x[c] over the block's
+// pixels: per wave by shuffles, eight channels at a time, so that a shuffle's
+// latency is shared, then the four waves in LDS.  (33.6 us for 32 frames of 64 x
+// 64 with 2-byte accesses and the channels one after another, 9.5 now.)
+__global__ void __launch_bounds__(256)
+k_head_bwd(const bf16* __restrict__ x, const float* __restrict__ w,
+           const float* __restrict__ gy, bf16* __restrict__ gx,
+           float* __restrict__ part, int64_t npix)
 {
-    __shared__ float red[4][33];
+    constexpr int C = 32;
+    __shared__ float red[4][C + 1];
     const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const float g = p < npix ? gy[p] : 0.f;
-    if (p < npix)
-        for (int i = 0; i < c; i++) gx[p * c + i] = (bf16)(g * w[i]);
-    // per wave: shuffle sums of g and of g * x[i], then the 4 waves in LDS
-    for (int i = -1; i < c; i++) {
-        float v = i < 0 ? g : (p < npix ? g * (float)x[p * c + i] : 0.f);
-        for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
-        if (lane == 0) red[wave][i + 1] = v;
+    const bool in = p < npix;
+    const int64_t at = (in ? p : npix - 1) * C;
+    const float g = in ? gy[p] : 0.f;
+    bf16x8 v[C / 8];
+#pragma unroll
+    for (int k = 0; k < C / 8; k++) v[k] = load8(x + at + k * 8);
+    if (in)
+#pragma unroll
+        for (int k = 0; k < C / 8; k++) {
+            bf16x8 o;
+#pragma unroll
+            for (int e = 0; e < 8; e++) o[e] = (bf16)(g * w[k * 8 + e]);
+            store8(gx + at + k * 8, o);
+        }
+    float t = g;
+    for (int off = 32; off > 0; off >>= 1) t += __shfl_down(t, off, 64);
+    if (lane == 0) red[wave][0] = t;
+#pragma unroll
+    for (int k = 0; k < C / 8; k++) {
+        float s[8];
+#pragma unroll
+        for (int e = 0; e < 8; e++) s[e] = in ? g * (float)v[k][e] : 0.f;
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1)
+#pragma unroll
+            for (int e = 0; e < 8; e++) s[e] += __shfl_down(s[e], off, 64);
+        if (lane == 0)
+#pragma unroll
+            for (int e = 0; e < 8; e++) red[wave][1 + k * 8 + e] = s[e];
     }
     __syncthreads();
-    if (threadIdx.x <= c) {
-        const float t = (red[0][threadIdx.x] + red[1][threadIdx.x]) +
+    if (threadIdx.x <= C) {
+        const float r = (red[0][threadIdx.x] + red[1][threadIdx.x]) +
                         (red[2][threadIdx.x] + red[3][threadIdx.x]);
-        part[(int64_t)blockIdx.x * (c + 1) + threadIdx.x] = t;
+        part[(int64_t)blockIdx.x * (C + 1) + threadIdx.x] = r;
     }
 }
 
@@ -900,6 +1135,13 @@ void conv3x3(hipStream_t st, const bf16* in, int cin, const bf16* w, const float
         conv3x3_in(st, src, w, bias, out, out32, cout, nb, H, W, flags);
         return;
     }
+    if (H * W <= SMALL_PIXELS && small_patch_bytes(cin, H, W) <= SMALL_LDS) {
+        const int mt = H * W <= 16 ? 1 : H * W <= 32 ? 2 : 4;
+        dim3 grid(nb, (cout / 16 + 4 / mt - 1) / (4 / mt));
+        k_conv3x3_small<<<grid, 256, small_patch_bytes(cin, H, W), st>>>(
+            in, cin, w, bias, out, out32, cout, H, W, mt, flags, live);
+        return;
+    }
     if (npix >= 64 * 256) {
         dim3 grid(nblk(npix, 128), (cout + 63) / 64);
         k_conv3x3<128><<<grid, 256, 0, st>>>(in, cin, w, bias, out, out32, cout, nb, H, W, flags,
@@ -910,66 +1152,71 @@ void conv3x3(hipStream_t st, const bf16* in, int cin, const bf16* w, const float
                                             live);
     }
 }
-void weight_flip(hipStream_t st, const bf16* w, bf16* wt, int cin, int cout) {
-    const int64_t n = (int64_t)cin * 9 * cout;
-    k_weight_flip<<<nblk(n), 256, 0, st>>>(w, wt, cin, cout);
+void weight_flip(hipStream_t st, FlipList& l, const bf16* w, bf16* wt) {
+    unsigned n = 0;
+    for (int k = 0; k < l.n; k++) {
+        l.block[k] = n;
+        n += nblk((int64_t)l.cin[k] * 9 * l.cout[k]);
+    }
+    k_weight_flip<<<n, 256, 0, st>>>(l, w, wt);
 }
-void conv3x3_dw(hipStream_t st, const bf16* gz, int cout, const bf16* in, int cin, float* dw32,
-                int nb, int H, int W, float* part) {
+void conv_grads(hipStream_t st, const bf16* y, bf16* g, int cout, const bf16* in, int cin,
+                float* dw32, float* db, int nb, int H, int W, float* part, float* bpart) {
     const int64_t npix = (int64_t)nb * H * W;
-    const int ci_blocks = (cin + 63) / 64;
+    // the ReLU's backward and the bias: at most about one block per CU, so the
+    // sums of their partials stay short
+    const int bper = bias_pixels_per_block(npix);
+    const int bblocks = (int)bias_blocks(npix);   // partials: grad_partials (nn_sizes.h)
+    k_relu_bias_bwd<<<bblocks, 256, 0, st>>>(y, g, cout, (int)npix, bper, bpart);
     const int per = dw_pixels_per_chunk(npix);
     const int chunks = (int)dw_chunks(npix);   // partials: grad_partials (nn_sizes.h)
     const int64_t nw = (int64_t)cout * 9 * cin;
-    dim3 grid(ci_blocks, (cout + 63) / 64, 9 * chunks);
-    if (chunks == 1) {
-        k_conv3x3_dw<<<grid, 256, 0, st>>>(gz, cout, in, cin, dw32, 0, nb, H, W, per);
-        return;
+    float* dst = chunks == 1 ? dw32 : part;
+    const int64_t stride = chunks == 1 ? 0 : nw;
+    // the channels in tiles of 64, and of 32 what is left (three taps a block)
+    auto tiles = [&](auto kernel, int co, int ci, int first, int n) {
+        if (n > 0)
+            kernel<<<dim3(n / ci, cout / co, 3 * chunks), 256, 0, st>>>(
+                g, cout, in, cin, first, dst, stride, nb, H, W, per);
+    };
+    const int wide = cin / 64 * 64;
+    if (cout % 64 == 0) {
+        tiles(k_conv3x3_dw<64, 64>, 64, 64, 0, wide);
+        tiles(k_conv3x3_dw<64, 32>, 64, 32, wide, cin - wide);
+    } else {
+        tiles(k_conv3x3_dw<32, 64>, 32, 64, 0, wide);
+        tiles(k_conv3x3_dw<32, 32>, 32, 32, wide, cin - wide);
     }
-    k_conv3x3_dw<<<grid, 256, 0, st>>>(gz, cout, in, cin, part, nw, nb, H, W, per);
-    k_chunk_sum<<<nblk(nw), 256, 0, st>>>(part, chunks, nw, dw32);
-}
-void relu_bwd(hipStream_t st, int64_t n, const bf16* y, bf16* g) {
-    k_relu_bwd<<<nblk(n), 256, 0, st>>>(n, y, g);
-}
-void bias_grad(hipStream_t st, const bf16* g, int c, int64_t npix, float* db, float* part) {
-    // bias channels are 32, 64, 128 or 256; each block leaves c partial sums
-    // and at most about one block per CU runs, so the block sums stay short
-    const int per = bias_pixels_per_block(npix);
-    const int nblocks = (int)bias_blocks(npix);   // partials: grad_partials (nn_sizes.h)
-    k_bias_grad<<<nblocks, 256, 0, st>>>(g, c, (int)npix, per, part);
-    k_block_sum<<<c, 256, 0, st>>>(part, nblocks, c, 0, db, 1);
+    k_grad_finish<<<cout + (chunks > 1 ? nblk(nw) : 0), 256, 0, st>>>(part, chunks, nw, dw32, bpart,
+                                                                      bblocks, cout, db);
 }
 void maxpool(hipStream_t st, const bf16* x, bf16* y, int nb, int H, int W, int c, const int* live) {
-    k_maxpool<<<nblk((int64_t)nb * H * W * c / 4), 256, 0, st>>>(x, y, nb, H, W, c, live);
+    k_maxpool<<<nblk((int64_t)nb * H * W * c / 32), 256, 0, st>>>(x, y, nb, H, W, c, live);
 }
 void maxpool_bwd(hipStream_t st, const bf16* x, const bf16* y, const bf16* gy, bf16* gx, int nb,
                  int H, int W, int c) {
-    k_maxpool_bwd<<<nblk((int64_t)nb * H * W * c / 4), 256, 0, st>>>(x, y, gy, gx, nb, H, W, c);
+    k_maxpool_bwd<<<nblk((int64_t)nb * H * W * c / 32), 256, 0, st>>>(x, y, gy, gx, nb, H, W, c);
 }
-void upsample(hipStream_t st, const bf16* x, bf16* y, int nb, int H, int W, int c, int cy, int c0,
-              const int* live) {
-    k_upsample<<<nblk((int64_t)nb * H * W * c), 256, 0, st>>>(x, y, nb, H, W, c, cy, c0, live);
+void join(hipStream_t st, const bf16* x, int ca, const bf16* s, int cb, bf16* y, int nb, int H,
+          int W, const int* live) {
+    k_join<<<nblk((int64_t)nb * H * W * (ca + cb) / 8), 256, 0, st>>>(x, ca, s, cb, y, nb, H, W,
+                                                                      live);
 }
-void upsample_bwd(hipStream_t st, const bf16* gy, bf16* gx, int nb, int H, int W, int c, int cy,
-                  int c0) {
-    k_upsample_bwd<<<nblk((int64_t)nb * H * W * c / 4), 256, 0, st>>>(gy, gx, nb, H, W, c, cy, c0);
-}
-void channel_copy(hipStream_t st, const bf16* src, int cs, int s0, bf16* dst, int cd, int d0, int c,
-                  int64_t npix, int add, const int* live, int64_t hw) {
-    k_channel_copy<<<nblk(npix * c), 256, 0, st>>>(src, cs, s0, dst, cd, d0, c, npix, add, live,
-                                                   hw);
+void join_bwd(hipStream_t st, const bf16* gy, bf16* gx, int ca, bf16* gs, int cb, int nb, int H,
+              int W) {
+    k_join_bwd<<<nblk((int64_t)nb * H * W * (ca + cb) / 32), 256, 0, st>>>(gy, gx, ca, gs, cb, nb, H,
+                                                                           W);
 }
 void head(hipStream_t st, const bf16* x, int c, const float* w, const float* b, float* y,
           int64_t npix, const int* live, int64_t hw) {
     k_head<<<nblk(npix), 256, 0, st>>>(x, c, w, b, y, npix, live, hw);
 }
-void head_bwd(hipStream_t st, const bf16* x, int c, const float* w, const float* gy, bf16* gx,
+void head_bwd(hipStream_t st, const bf16* x, const float* w, const float* gy, bf16* gx,
               float* dw, float* db, int64_t npix, float* part) {
     const int nblocks = (int)nblk(npix);
-    k_head_bwd<<<nblocks, 256, 0, st>>>(x, c, w, gy, gx, part, npix);
-    k_block_sum<<<1, 256, 0, st>>>(part, nblocks, c + 1, 0, db, 1);
-    k_block_sum<<<c, 256, 0, st>>>(part, nblocks, c + 1, 1, dw, 1);
+    k_head_bwd<<<nblocks, 256, 0, st>>>(x, w, gy, gx, part, npix);
+    k_block_sum<<<1, 256, 0, st>>>(part, nblocks, 33, 0, db, 1);
+    k_block_sum<<<32, 256, 0, st>>>(part, nblocks, 33, 1, dw, 1);
 }
 void loss(hipStream_t st, const float* y, const float* t, const float* m, float* denom, float* gy,
           float* loss_out, int64_t npix_per, int nb, float* part) {

@@ -48,7 +48,8 @@ struct Net {
     int64_t nparam = 0, head_w = 0, head_b = 0;
     float *p32 = nullptr, *g32 = nullptr, *m32 = nullptr, *v32 = nullptr;
     nn::bf16* pb = nullptr;      // bf16 copy of the parameters
-    nn::bf16* wflip = nullptr;   // scratch for the backward-input weights
+    nn::bf16* wflip = nullptr;   // the backward-input weights of every layer, as pb
+    float* bpart = nullptr;      // partial sums of a layer's bias gradients
     // FP32 partial sums: one slice per split of a split-K convolution in the
     // forward pass, the per-block sums of the gradient and loss reductions in
     // training (scratch_floats in all, at least splitk_cap)

@@ -101,9 +101,12 @@ int Net::init(stm_ctx* c, int H_, int W_, int cap_, uint64_t seed) {
     NCHK(hipMemset(m32, 0, pbytes));
     NCHK(hipMemset(v32, 0, pbytes));
     NCHK(hipMemset(g32, 0, pbytes));
-    int64_t maxw = 0;
-    for (auto& cv : convs) maxw = std::max(maxw, (int64_t)cv.cout * 9 * cv.cin);
-    NCHK(hipMalloc(&wflip, sizeof(bf16) * maxw));
+    NCHK(hipMalloc(&wflip, sizeof(bf16) * nparam));
+    int64_t nbias = 0;
+    for (auto& cv : convs)
+        nbias = std::max(nbias,
+                         nn::bias_partials(cv.cout, (int64_t)cap * h(cv.level) * w(cv.level)));
+    NCHK(hipMalloc(&bpart, sizeof(float) * (size_t)nbias));
     // the largest conv output is level 0's: cap x H x W x 32 (levels below have
     // a quarter of the pixels and twice the channels)
     scratch_floats = std::max(splitk_cap(), nn::loss_partials((int64_t)H * W, cap, 32));
@@ -149,7 +152,7 @@ int Net::init(stm_ctx* c, int H_, int W_, int cap_, uint64_t seed) {
 }
 
 void Net::release() {
-    void* bufs[] = {p32, g32, m32, v32, pb, wflip, splitk, y, gy, target, mask, denom, loss,
+    void* bufs[] = {p32, g32, m32, v32, pb, wflip, bpart, splitk, y, gy, target, mask, denom, loss,
                     d_idx, dx, dt};
     for (void* b : bufs)
         if (b) hipFree(b);
@@ -178,16 +181,13 @@ void Net::forward(int nb) {
     nn::maxpool(stream, acts[8].v, acts[9].v, nb, h(2), w(2), 128);
     conv(6);
     conv(7);
-    nn::upsample(stream, acts[11].v, acts[12].v, nb, h(2), w(2), 256, 384, 0);
-    nn::channel_copy(stream, acts[8].v, 128, 0, acts[12].v, 384, 256, 128, npix(2), 0);
+    nn::join(stream, acts[11].v, 256, acts[8].v, 128, acts[12].v, nb, h(2), w(2));
     conv(8);
     conv(9);
-    nn::upsample(stream, acts[14].v, acts[15].v, nb, h(1), w(1), 128, 192, 0);
-    nn::channel_copy(stream, acts[5].v, 64, 0, acts[15].v, 192, 128, 64, npix(1), 0);
+    nn::join(stream, acts[14].v, 128, acts[5].v, 64, acts[15].v, nb, h(1), w(1));
     conv(10);
     conv(11);
-    nn::upsample(stream, acts[17].v, acts[18].v, nb, h(0), w(0), 64, 96, 0);
-    nn::channel_copy(stream, acts[2].v, 32, 0, acts[18].v, 96, 64, 32, npix(0), 0);
+    nn::join(stream, acts[17].v, 64, acts[2].v, 32, acts[18].v, nb, h(0), w(0));
     conv(12);
     conv(13);
     nn::head(stream, acts[20].v, 32, p32 + head_w, p32 + head_b, y, npix(0));
@@ -235,10 +235,8 @@ void Net::forward_infer(int nb, const int* live) {
         if (conv_tiles_fit(h(c.level), w(c.level))) {
             run(k, ConvIn{acts[low].v, cl, nn::IN_UP, acts[skip].v, cs});
         } else {
-            nn::upsample(stream, acts[low].v, acts[cat].v, nb, h(c.level), w(c.level), cl, cl + cs,
-                         0, live);
-            nn::channel_copy(stream, acts[skip].v, cs, 0, acts[cat].v, cl + cs, cl, cs,
-                             npix(c.level), 0, live, (int64_t)h(c.level) * w(c.level));
+            nn::join(stream, acts[low].v, cl, acts[skip].v, cs, acts[cat].v, nb, h(c.level),
+                     w(c.level), live);
             plain(k);
         }
     };
@@ -274,31 +272,30 @@ void Net::backward(int nb) {
     auto conv_bwd = [&](int k, bool need_gx) {
         const Conv& c = convs[k];
         const int hh = h(c.level), ww = w(c.level);
-        const int64_t np = npix(c.level);
-        nn::relu_bwd(stream, np * c.cout, acts[c.y].v, acts[c.y].g);
-        nn::conv3x3_dw(stream, acts[c.y].g, c.cout, acts[c.x].v, c.cin, g32 + c.woff, nb, hh, ww,
-                       splitk);
-        nn::bias_grad(stream, acts[c.y].g, c.cout, np, g32 + c.boff, splitk);
-        if (need_gx) {
-            nn::weight_flip(stream, pb + c.woff, wflip, c.cin, c.cout);
-            nn::conv3x3(stream, acts[c.y].g, c.cout, wflip, nullptr, acts[c.x].g, nullptr, c.cin,
-                        nb, hh, ww, 0);
-        }
+        nn::conv_grads(stream, acts[c.y].v, acts[c.y].g, c.cout, acts[c.x].v, c.cin, g32 + c.woff,
+                       g32 + c.boff, nb, hh, ww, splitk, bpart);
+        if (need_gx)
+            nn::conv3x3(stream, acts[c.y].g, c.cout, wflip + c.woff, nullptr, acts[c.x].g, nullptr,
+                        c.cin, nb, hh, ww, 0);
     };
-    nn::head_bwd(stream, acts[20].v, 32, p32 + head_w, gy, acts[20].g, g32 + head_w,
+    nn::FlipList flips;
+    for (size_t k = 1; k < convs.size(); k++) {   // (the first layer passes nothing on)
+        flips.cin[flips.n] = convs[k].cin;
+        flips.cout[flips.n] = convs[k].cout;
+        flips.off[flips.n++] = convs[k].woff;
+    }
+    nn::weight_flip(stream, flips, pb, wflip);
+    nn::head_bwd(stream, acts[20].v, p32 + head_w, gy, acts[20].g, g32 + head_w,
                  g32 + head_b, npix(0), splitk);
     conv_bwd(13, true);
     conv_bwd(12, true);
-    nn::upsample_bwd(stream, acts[18].g, acts[17].g, nb, h(0), w(0), 64, 96, 0);
-    nn::channel_copy(stream, acts[18].g, 96, 64, acts[2].g, 32, 0, 32, npix(0), 0);
+    nn::join_bwd(stream, acts[18].g, acts[17].g, 64, acts[2].g, 32, nb, h(0), w(0));
     conv_bwd(11, true);
     conv_bwd(10, true);
-    nn::upsample_bwd(stream, acts[15].g, acts[14].g, nb, h(1), w(1), 128, 192, 0);
-    nn::channel_copy(stream, acts[15].g, 192, 128, acts[5].g, 64, 0, 64, npix(1), 0);
+    nn::join_bwd(stream, acts[15].g, acts[14].g, 128, acts[5].g, 64, nb, h(1), w(1));
     conv_bwd(9, true);
     conv_bwd(8, true);
-    nn::upsample_bwd(stream, acts[12].g, acts[11].g, nb, h(2), w(2), 256, 384, 0);
-    nn::channel_copy(stream, acts[12].g, 384, 256, acts[8].g, 128, 0, 128, npix(2), 0);
+    nn::join_bwd(stream, acts[12].g, acts[11].g, 256, acts[8].g, 128, nb, h(2), w(2));
     conv_bwd(7, true);
     conv_bwd(6, true);
     nn::maxpool_bwd(stream, acts[8].v, acts[9].v, acts[9].g, acts[8].g, nb, h(2), w(2), 128);

@@ -38,15 +38,19 @@ inline int64_t bias_blocks(int64_t npix) {
     return (npix + per - 1) / per;
 }
 
-// Partials (floats) of conv3x3_dw and bias_grad for any pixel count up to
+// Partials (floats) of the bias gradients of a layer with cout channels.
+inline int64_t bias_partials(int cout, int64_t npix) {
+    return std::min<int64_t>((npix + 127) / 128, 257) * cout;
+}
+
+// Partials (floats) of the weight and bias gradients for any pixel count up to
 // npix.  The chunk counts are not monotone in the pixel count: at most 257
 // chunks until the chunk size stops growing, at most 257 bias blocks.
 inline int64_t grad_partials(int cin, int cout, int64_t npix) {
     const int64_t chunks =
         std::min((npix + 1023) / 1024, std::max<int64_t>(257, (npix + (1 << 20) - 1) >> 20));
     const int64_t dw = chunks > 1 ? chunks * cout * 9 * cin : 0;
-    const int64_t db = std::min<int64_t>((npix + 127) / 128, 257) * cout;
-    return std::max(dw, db);
+    return std::max(dw, bias_partials(cout, npix));
 }
 
 // Partials of loss (per-sample sums over 64 blocks, then one per 256-pixel
