@@ -1207,6 +1207,198 @@ int check_params(stm_ctx* ctx, const stm_params* q) {
     return STM_OK;
 }
 
+// ------------------------------------------------------------- transfers
+
+// Transfers between a channel's fields and the caller's dense arrays: kernels
+// pack and unpack the rows, since a pitched copy to or from pageable memory is
+// done row by row (7 to 9 us each: 0.70 ms for three fields of 102 x 22 cells,
+// 8.8 ms for one of 1026 x 1026).
+
+// Pinned staging, one per context, allocated at the first transfer.
+constexpr size_t STAGE_MOST = (size_t)8 << 20;
+// A download of this much or more is copied out of the staging buffer by
+// COPY_THREADS threads: writing fresh pages goes at 5 GB/s with one and at
+// 17 GB/s with eight; starting them takes some 60 us, so that 1 MB gains nothing.
+constexpr size_t COPY_SPLIT = (size_t)2 << 20;
+constexpr int COPY_THREADS = 8;
+// Below this the arrays of an upload go through the staging buffer and one
+// kernel (8 us and a copy at 10 GB/s); from there on a contiguous copy from
+// the caller's memory (35 GB/s, but 14 us for each array) is the faster one.
+constexpr size_t UPLOAD_STAGED = (size_t)256 << 10;
+
+// The staging buffer with at least min(bytes, STAGE_MOST) bytes; false if
+// there is no pinned memory for it.
+bool stage_buffer(stm_ctx* ctx, size_t bytes) {
+    if (std::min(bytes, STAGE_MOST) <= ctx->stage_bytes) return true;
+    size_t cap = (size_t)64 << 10;
+    while (cap < bytes && cap < STAGE_MOST) cap *= 2;
+    if (ctx->h_stage) hipHostFree(ctx->h_stage);
+    ctx->h_stage = nullptr;
+    ctx->stage_bytes = 0;
+    void* m = nullptr;
+    if (hipHostMalloc(&m, cap, hipHostMallocDefault) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    ctx->h_stage = (char*)m;
+    ctx->stage_bytes = cap;
+    return true;
+}
+
+// The general way, for rows longer than half the staging buffer and when there
+// is none.
+int copy_pitched(stm_ctx* ctx, const HostChan& c, double* dev, double* host, bool up) {
+    const size_t row = sizeof(double) * c.ny, pitch = sizeof(double) * c.pitch;
+    if (up)
+        HIPCHK(ctx, hipMemcpy2DAsync(dev + c.off, pitch, host, row, row, c.nx,
+                                     hipMemcpyHostToDevice, ctx->stream));
+    else
+        HIPCHK(ctx, hipMemcpy2DAsync(host, row, dev + c.off, pitch, row, c.nx,
+                                     hipMemcpyDeviceToHost, ctx->stream));
+    HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
+    return STM_OK;
+}
+
+FieldRows field_rows(const HostChan& c, uint32_t x0, uint32_t rows) {
+    FieldRows r{};
+    r.off = c.off;
+    r.pitch = c.pitch;
+    r.x0 = (int32_t)x0;
+    r.rows = (int32_t)rows;
+    r.ny = (int32_t)c.ny;
+    return r;
+}
+
+// Copies pieces of the chunks a download is cut into: piece i belongs to chunk
+// i / COPY_THREADS and may be taken once `ready` has passed that chunk.
+struct CopyOut {
+    std::atomic<int64_t> next{0}, done{0}, ready{0};
+    std::atomic<bool> stop{false};
+    int64_t pieces = 0;
+    std::function<void(int64_t chunk, int part)> copy;
+
+    void run() {
+        for (;;) {
+            const int64_t i = next.fetch_add(1);
+            if (i >= pieces) return;
+            while (ready.load(std::memory_order_acquire) <= i / COPY_THREADS) {
+                if (stop.load()) return;
+                std::this_thread::yield();
+            }
+            copy(i / COPY_THREADS, (int)(i % COPY_THREADS));
+            done.fetch_add(1, std::memory_order_release);
+        }
+    }
+};
+
+// `chunks` pieces of a download through the two halves of the staging buffer:
+// fill(k) queues what brings chunk k into half k & 1, and copy(k, part, parts)
+// copies a part of it out, while chunk k + 1 is on its way.
+template <class Fill, class Copy>
+int copy_chunks(stm_ctx* ctx, int64_t chunks, Fill fill, Copy copy) {
+    int rc = fill(0);
+    if (rc) return rc;
+    CopyOut out;
+    out.pieces = chunks * COPY_THREADS;
+    out.copy = [&](int64_t k, int part) { copy(k, part, COPY_THREADS); };
+    std::vector<std::thread> team;
+    for (int t = 0; t < COPY_THREADS; t++) {
+        try {
+            team.emplace_back([&out] { out.run(); });
+        } catch (const std::exception&) {   // no more threads to be had
+            break;
+        }
+    }
+    hipError_t e = hipSuccess;
+    for (int64_t k = 0; k < chunks; k++) {
+        // chunk k is in its half of the buffer; k + 1 goes into the other one,
+        // which chunk k - 1 has left (waited for below)
+        if ((e = hipStreamSynchronize(ctx->stream)) != hipSuccess) break;
+        if (k + 1 < chunks && (rc = fill(k + 1))) break;
+        if (team.empty())
+            copy(k, 0, 1);
+        else {
+            out.ready.store(k + 1, std::memory_order_release);
+            while (out.done.load(std::memory_order_acquire) < (k + 1) * COPY_THREADS)
+                std::this_thread::yield();
+        }
+    }
+    out.stop = true;
+    for (std::thread& t : team) t.join();
+    HIPCHK(ctx, e);
+    return rc;
+}
+
+// Part `part` of `parts` of n bytes: its start and end (multiples of 4 KB but the last).
+std::pair<size_t, size_t> part_of(size_t n, int part, int parts) {
+    const size_t step = (n / parts + 4096) / 4096 * 4096, a = std::min(n, part * step);
+    return {a, std::min(n, a + step)};
+}
+
+// Fields `dev` (n of them) of channel c into the arrays `host`.  What does not
+// fit goes in chunks of rows through the staging buffer.
+int pack_to_host(stm_ctx* ctx, const HostChan& c, int n, double* const* dev,
+                        double* const* host) {
+    const size_t row = sizeof(double) * c.ny, all = row * c.nx * n;
+    if (!stage_buffer(ctx, all) || row * n > ctx->stage_bytes / 2) {
+        int rc = STM_OK;
+        for (int f = 0; f < n && !rc; f++) rc = copy_pitched(ctx, c, dev[f], host[f], false);
+        return rc;
+    }
+    const bool whole = all <= ctx->stage_bytes && all < COPY_SPLIT;
+    const size_t half = whole ? ctx->stage_bytes : ctx->stage_bytes / 2;
+    const uint32_t most = whole ? c.nx : (uint32_t)(half / (row * n));
+    auto rows_of = [&](int64_t k) { return std::min<uint32_t>(most, c.nx - (uint32_t)k * most); };
+    auto fill = [&](int64_t k) {
+        FieldRows r = field_rows(c, (uint32_t)k * most, rows_of(k));
+        for (int f = 0; f < n; f++) {
+            r.dev[f] = dev[f];
+            r.dense[f] = (double*)(ctx->h_stage + (k & 1) * half + f * row * r.rows);
+        }
+        launch_rows(ctx->stream, r, n, true);
+        return check_launch(ctx);
+    };
+    auto copy = [&](int64_t k, int part, int parts) {
+        const size_t m = row * rows_of(k);
+        const auto [a, b] = part_of(m, part, parts);
+        for (int f = 0; f < n && a < b; f++)
+            memcpy((char*)host[f] + row * most * k + a,
+                   ctx->h_stage + (k & 1) * half + f * m + a, b - a);
+    };
+    if (!whole) return copy_chunks(ctx, (c.nx + most - 1) / most, fill, copy);
+    int rc = fill(0);
+    if (rc) return rc;
+    HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
+    copy(0, 0, 1);
+    return STM_OK;
+}
+
+// The caller's arrays into the fields.  A large one is copied as it is into
+// `scratch`, whose content no call leaves to the next.
+int unpack_from_host(stm_ctx* ctx, const HostChan& c, int n, double* const* dev,
+                            const double* const* host) {
+    const size_t bytes = sizeof(double) * c.nx * c.ny;
+    FieldRows r = field_rows(c, 0, c.nx);
+    if (bytes * n <= UPLOAD_STAGED && stage_buffer(ctx, bytes * n)) {
+        for (int f = 0; f < n; f++) {
+            memcpy(ctx->h_stage + f * bytes, host[f], bytes);
+            r.dev[f] = dev[f];
+            r.dense[f] = (double*)(ctx->h_stage + f * bytes);
+        }
+        launch_rows(ctx->stream, r, n, false);
+    } else {
+        for (int f = 0; f < n; f++) {
+            r.dev[0] = dev[f];
+            r.dense[0] = ctx->scratch + c.off;
+            HIPCHK(ctx, hipMemcpyAsync(r.dense[0], host[f], bytes, hipMemcpyHostToDevice,
+                                       ctx->stream));
+            launch_rows(ctx->stream, r, 1, false);
+        }
+    }
+    HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
+    return check_launch(ctx);
+}
+
 }  // namespace
 
 // =================================================================== C ABI
@@ -1399,185 +1591,6 @@ int stm_set_params(stm_ctx* ctx, uint32_t ch, const stm_params* params) {
     HIPCHK(ctx, hipMemcpyAsync(ctx->d_cs + ch, &s, sizeof s, hipMemcpyHostToDevice, ctx->stream));
     HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
     return STM_OK;
-}
-
-// Transfers between a channel's fields and the caller's dense arrays: kernels
-// pack and unpack the rows, since a pitched copy to or from pageable memory is
-// done row by row (7 to 9 us each: 0.70 ms for three fields of 102 x 22 cells,
-// 8.8 ms for one of 1026 x 1026).
-
-// Pinned staging, one per context, allocated at the first transfer.
-constexpr size_t STAGE_MOST = (size_t)8 << 20;
-// A download of this much or more is copied out of the staging buffer by
-// COPY_THREADS threads: writing fresh pages goes at 5 GB/s with one and at
-// 17 GB/s with eight; starting them takes some 60 us, so that 1 MB gains nothing.
-constexpr size_t COPY_SPLIT = (size_t)2 << 20;
-constexpr int COPY_THREADS = 8;
-// Below this the arrays of an upload go through the staging buffer and one
-// kernel (8 us and a copy at 10 GB/s); from there on a contiguous copy from
-// the caller's memory (35 GB/s, but 14 us for each array) is the faster one.
-constexpr size_t UPLOAD_STAGED = (size_t)256 << 10;
-
-// The staging buffer with at least min(bytes, STAGE_MOST) bytes; false if
-// there is no pinned memory for it.
-static bool stage_buffer(stm_ctx* ctx, size_t bytes) {
-    if (std::min(bytes, STAGE_MOST) <= ctx->stage_bytes) return true;
-    size_t cap = (size_t)64 << 10;
-    while (cap < bytes && cap < STAGE_MOST) cap *= 2;
-    if (ctx->h_stage) hipHostFree(ctx->h_stage);
-    ctx->h_stage = nullptr;
-    ctx->stage_bytes = 0;
-    void* m = nullptr;
-    if (hipHostMalloc(&m, cap, hipHostMallocDefault) != hipSuccess) {
-        (void)hipGetLastError();
-        return false;
-    }
-    ctx->h_stage = (char*)m;
-    ctx->stage_bytes = cap;
-    return true;
-}
-
-// The general way, for rows longer than half the staging buffer and when there
-// is none.
-static int copy_pitched(stm_ctx* ctx, const HostChan& c, double* dev, double* host, bool up) {
-    const size_t row = sizeof(double) * c.ny, pitch = sizeof(double) * c.pitch;
-    if (up)
-        HIPCHK(ctx, hipMemcpy2DAsync(dev + c.off, pitch, host, row, row, c.nx,
-                                     hipMemcpyHostToDevice, ctx->stream));
-    else
-        HIPCHK(ctx, hipMemcpy2DAsync(host, row, dev + c.off, pitch, row, c.nx,
-                                     hipMemcpyDeviceToHost, ctx->stream));
-    HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
-    return STM_OK;
-}
-
-static FieldRows field_rows(const HostChan& c, uint32_t x0, uint32_t rows) {
-    FieldRows r{};
-    r.off = c.off;
-    r.pitch = c.pitch;
-    r.x0 = (int32_t)x0;
-    r.rows = (int32_t)rows;
-    r.ny = (int32_t)c.ny;
-    return r;
-}
-
-// Copies pieces of the chunks a download is cut into: piece i belongs to chunk
-// i / COPY_THREADS and may be taken once `ready` has passed that chunk.
-struct CopyOut {
-    std::atomic<int64_t> next{0}, done{0}, ready{0};
-    std::atomic<bool> stop{false};
-    int64_t pieces = 0;
-    std::function<void(int64_t chunk, int part)> copy;
-
-    void run() {
-        for (;;) {
-            const int64_t i = next.fetch_add(1);
-            if (i >= pieces) return;
-            while (ready.load(std::memory_order_acquire) <= i / COPY_THREADS) {
-                if (stop.load()) return;
-                std::this_thread::yield();
-            }
-            copy(i / COPY_THREADS, (int)(i % COPY_THREADS));
-            done.fetch_add(1, std::memory_order_release);
-        }
-    }
-};
-
-// Fields `dev` (n of them) of channel c into the arrays `host`.  What does not
-// fit goes in chunks of rows through the two halves of the staging buffer, the
-// kernel filling one while the other is copied out.
-static int pack_to_host(stm_ctx* ctx, const HostChan& c, int n, double* const* dev,
-                        double* const* host) {
-    const size_t row = sizeof(double) * c.ny, all = row * c.nx * n;
-    if (!stage_buffer(ctx, all) || row * n > ctx->stage_bytes / 2) {
-        int rc = STM_OK;
-        for (int f = 0; f < n && !rc; f++) rc = copy_pitched(ctx, c, dev[f], host[f], false);
-        return rc;
-    }
-    const bool whole = all <= ctx->stage_bytes && all < COPY_SPLIT;
-    const size_t half = whole ? ctx->stage_bytes : ctx->stage_bytes / 2;
-    const uint32_t most = whole ? c.nx : (uint32_t)(half / (row * n));
-    const int64_t chunks = (c.nx + most - 1) / most;
-    auto rows_of = [&](int64_t k) { return std::min<uint32_t>(most, c.nx - (uint32_t)k * most); };
-    auto fill = [&](int64_t k) {
-        FieldRows r = field_rows(c, (uint32_t)k * most, rows_of(k));
-        for (int f = 0; f < n; f++) {
-            r.dev[f] = dev[f];
-            r.dense[f] = (double*)(ctx->h_stage + (k & 1) * half + f * row * r.rows);
-        }
-        launch_rows(ctx->stream, r, n, true);
-        return check_launch(ctx);
-    };
-    auto copy_part = [&](int64_t k, int part, int parts) {
-        const size_t m = row * rows_of(k);
-        const size_t step = (m / parts + 4096) / 4096 * 4096;
-        const size_t a = std::min(m, part * step), b = std::min(m, a + step);
-        for (int f = 0; f < n && a < b; f++)
-            memcpy((char*)host[f] + row * most * k + a,
-                   ctx->h_stage + (k & 1) * half + f * m + a, b - a);
-    };
-    int rc = fill(0);
-    if (rc) return rc;
-    if (whole) {
-        HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
-        copy_part(0, 0, 1);
-        return STM_OK;
-    }
-    CopyOut out;
-    out.pieces = chunks * COPY_THREADS;
-    out.copy = [&](int64_t k, int part) { copy_part(k, part, COPY_THREADS); };
-    std::vector<std::thread> team;
-    for (int t = 0; t < COPY_THREADS; t++) {
-        try {
-            team.emplace_back([&out] { out.run(); });
-        } catch (const std::exception&) {   // no more threads to be had
-            break;
-        }
-    }
-    hipError_t e = hipSuccess;
-    for (int64_t k = 0; k < chunks; k++) {
-        // chunk k is in its half of the buffer; k + 1 goes into the other one,
-        // which chunk k - 1 has left (waited for below)
-        if ((e = hipStreamSynchronize(ctx->stream)) != hipSuccess) break;
-        if (k + 1 < chunks && (rc = fill(k + 1))) break;
-        if (team.empty())
-            copy_part(k, 0, 1);
-        else {
-            out.ready.store(k + 1, std::memory_order_release);
-            while (out.done.load(std::memory_order_acquire) < (k + 1) * COPY_THREADS)
-                std::this_thread::yield();
-        }
-    }
-    out.stop = true;
-    for (std::thread& t : team) t.join();
-    HIPCHK(ctx, e);
-    return rc;
-}
-
-// The caller's arrays into the fields.  A large one is copied as it is into
-// `scratch`, whose content no call leaves to the next.
-static int unpack_from_host(stm_ctx* ctx, const HostChan& c, int n, double* const* dev,
-                            const double* const* host) {
-    const size_t bytes = sizeof(double) * c.nx * c.ny;
-    FieldRows r = field_rows(c, 0, c.nx);
-    if (bytes * n <= UPLOAD_STAGED && stage_buffer(ctx, bytes * n)) {
-        for (int f = 0; f < n; f++) {
-            memcpy(ctx->h_stage + f * bytes, host[f], bytes);
-            r.dev[f] = dev[f];
-            r.dense[f] = (double*)(ctx->h_stage + f * bytes);
-        }
-        launch_rows(ctx->stream, r, n, false);
-    } else {
-        for (int f = 0; f < n; f++) {
-            r.dev[0] = dev[f];
-            r.dense[0] = ctx->scratch + c.off;
-            HIPCHK(ctx, hipMemcpyAsync(r.dense[0], host[f], bytes, hipMemcpyHostToDevice,
-                                       ctx->stream));
-            launch_rows(ctx->stream, r, 1, false);
-        }
-    }
-    HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
-    return check_launch(ctx);
 }
 
 int stm_upload(stm_ctx* ctx, uint32_t ch, const double* u, const double* v, const double* p,
@@ -2201,6 +2214,30 @@ int stm_reset_stats(stm_ctx* ctx) {
 namespace stm {
 hipStream_t ctx_stream(stm_ctx* ctx) { return ctx->stream; }
 int ctx_device(stm_ctx* ctx) { return ctx->device; }
+// The staging buffer a download of n bytes uses, allocated ahead of it.
+void ctx_stage(stm_ctx* ctx, size_t n) {
+    if (n >= COPY_SPLIT) (void)stage_buffer(ctx, 2 * n);
+}
+// src (device) to dst (the caller's memory) in stream order, and waits for it.
+int ctx_download(stm_ctx* ctx, void* dst, const void* src, size_t n) {
+    if (n < COPY_SPLIT || !stage_buffer(ctx, 2 * n)) {
+        HIPCHK(ctx, hipMemcpyAsync(dst, src, n, hipMemcpyDeviceToHost, ctx->stream));
+        HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
+        return STM_OK;
+    }
+    const size_t half = ctx->stage_bytes / 2;
+    auto size = [&](int64_t k) { return std::min(half, n - k * half); };
+    auto fill = [&](int64_t k) -> int {
+        HIPCHK(ctx, hipMemcpyAsync(ctx->h_stage + (k & 1) * half, (const char*)src + k * half,
+                                   size(k), hipMemcpyDeviceToHost, ctx->stream));
+        return STM_OK;
+    };
+    auto copy = [&](int64_t k, int part, int parts) {
+        const auto [a, b] = part_of(size(k), part, parts);
+        if (a < b) memcpy((char*)dst + k * half + a, ctx->h_stage + (k & 1) * half + a, b - a);
+    };
+    return copy_chunks(ctx, (int64_t)((n + half - 1) / half), fill, copy);
+}
 
 void ctx_attach_net(stm_ctx* ctx, stm_net* net) { ctx->nets.push_back(net); }
 

@@ -24,6 +24,8 @@ namespace stm {
 
 hipStream_t ctx_stream(stm_ctx* ctx);
 int ctx_device(stm_ctx* ctx);
+void ctx_stage(stm_ctx* ctx, size_t n);
+int ctx_download(stm_ctx* ctx, void* dst, const void* src, size_t n);
 
 struct Conv {
     int cin, cout;
@@ -70,6 +72,7 @@ struct Net {
     float* dt = nullptr;         // n x H x W
     int dcap = 0, dsize = 0, dwrite = 0;   // capacity, samples held, next slot (ring)
     int32_t* d_idx = nullptr;
+    float* host_in = nullptr;    // a host batch on its way in: cap x H x W x (2 input + 1 target)
     // timing
     double fwd_ms = 0, train_ms = 0;
     uint64_t fwd_calls = 0, train_steps = 0, fwd_samples = 0, train_samples = 0;

@@ -93,6 +93,7 @@ int Net::init(stm_ctx* c, int H_, int W_, int cap_, uint64_t seed) {
 
     NCHK(hipSetDevice(ctx_device(c)));
     const size_t pbytes = sizeof(float) * nparam;
+    ctx_stage(c, pbytes);   // the gradients' way out
     NCHK(hipMalloc(&p32, pbytes));
     NCHK(hipMalloc(&g32, pbytes));
     NCHK(hipMalloc(&m32, pbytes));
@@ -130,6 +131,7 @@ int Net::init(stm_ctx* c, int H_, int W_, int cap_, uint64_t seed) {
     NCHK(hipMalloc(&denom, sizeof(float) * cap));
     NCHK(hipMalloc(&loss, sizeof(float)));
     NCHK(hipMalloc(&d_idx, sizeof(int32_t) * cap));
+    NCHK(hipMalloc(&host_in, sizeof(float) * npx * 3));
 
     // He initialisation from a SplitMix64 stream; the first layer sees two
     // real input channels.
@@ -153,7 +155,7 @@ int Net::init(stm_ctx* c, int H_, int W_, int cap_, uint64_t seed) {
 
 void Net::release() {
     void* bufs[] = {p32, g32, m32, v32, pb, wflip, bpart, splitk, y, gy, target, mask, denom, loss,
-                    d_idx, dx, dt};
+                    d_idx, dx, dt, host_in};
     for (void* b : bufs)
         if (b) hipFree(b);
     for (auto& a : acts) {
@@ -431,16 +433,14 @@ int stm_net_forward(stm_net* n, uint32_t nb, const float* x, float* y) {
     std::string& err = net.err;
     if ((int)nb > net.cap) return fail_net(n, STM_ERR_INVALID_ARG, "batch larger than capacity");
     const int64_t npix = (int64_t)nb * net.H * net.W;
-    float* dxh = nullptr;
-    NCHK(hipMalloc(&dxh, sizeof(float) * npix * 2));
+    float* dxh = net.host_in;
     hipMemcpyAsync(dxh, x, sizeof(float) * npix * 2, hipMemcpyHostToDevice, net.stream);
     k_pack_host<<<(unsigned)((npix + 255) / 256), 256, 0, net.stream>>>(dxh, nullptr, npix,
                                                                        net.input(), nullptr,
                                                                        nullptr);
     net.forward_infer((int)nb);
     hipMemcpyAsync(y, net.y, sizeof(float) * npix, hipMemcpyDeviceToHost, net.stream);
-    hipError_t e = hipStreamSynchronize(net.stream);
-    hipFree(dxh);
+    const hipError_t e = hipStreamSynchronize(net.stream);
     if (e != hipSuccess) return fail_net(n, STM_ERR_HIP, hipGetErrorString(e));
     return STM_OK;
 }
@@ -453,9 +453,7 @@ int stm_net_gradients(stm_net* n, uint32_t nb, const float* x, const float* t, f
     std::string& err = net.err;
     if ((int)nb > net.cap) return fail_net(n, STM_ERR_INVALID_ARG, "batch larger than capacity");
     const int64_t npix = (int64_t)nb * net.H * net.W;
-    float *dxh = nullptr, *dth = nullptr;
-    NCHK(hipMalloc(&dxh, sizeof(float) * npix * 2));
-    NCHK(hipMalloc(&dth, sizeof(float) * npix));
+    float *dxh = net.host_in, *dth = dxh + npix * 2;
     hipMemcpyAsync(dxh, x, sizeof(float) * npix * 2, hipMemcpyHostToDevice, net.stream);
     hipMemcpyAsync(dth, t, sizeof(float) * npix, hipMemcpyHostToDevice, net.stream);
     k_pack_host<<<(unsigned)((npix + 255) / 256), 256, 0, net.stream>>>(dxh, dth, npix,
@@ -468,12 +466,8 @@ int stm_net_gradients(stm_net* n, uint32_t nb, const float* x, const float* t, f
              (int64_t)net.H * net.W, (int)nb, net.splitk);
     net.backward((int)nb);
     hipMemcpyAsync(loss, net.loss, sizeof(float), hipMemcpyDeviceToHost, net.stream);
-    hipMemcpyAsync(grads, net.g32, sizeof(float) * net.nparam, hipMemcpyDeviceToHost, net.stream);
-    hipError_t e = hipStreamSynchronize(net.stream);
-    hipFree(dxh);
-    hipFree(dth);
-    if (e != hipSuccess) return fail_net(n, STM_ERR_HIP, hipGetErrorString(e));
-    return STM_OK;
+    return ctx_download(net.ctx, grads, net.g32, sizeof(float) * net.nparam)
+               ? fail_net(n, STM_ERR_HIP, stm_last_error(net.ctx)) : STM_OK;
 }
 
 int stm_net_dataset_reserve(stm_net* n, uint32_t capacity) {
