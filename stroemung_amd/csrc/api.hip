@@ -1216,11 +1216,13 @@ int check_params(stm_ctx* ctx, const stm_params* q) {
 
 // Pinned staging, one per context, allocated at the first transfer.
 constexpr size_t STAGE_MOST = (size_t)8 << 20;
-// A download of this much or more is copied out of the staging buffer by
-// COPY_THREADS threads: writing fresh pages goes at 5 GB/s with one and at
-// 17 GB/s with eight; starting them takes some 60 us, so that 1 MB gains nothing.
-constexpr size_t COPY_SPLIT = (size_t)2 << 20;
-constexpr int COPY_THREADS = 8;
+// A download of this much or more is copied out of the staging buffer by several
+// threads: writing fresh pages goes at 5 GB/s with one, 9 with four and 17 with
+// eight, starting a thread takes some 15 us (three fields of 258 x 258 cells, 1.5
+// MB: 292 us with one, 193 with four, 316 with eight, 221 with eight kept waiting
+// between downloads; 0.9 MB: 183, 189; 11.8 MB: 1077 with four, 989 with eight).
+constexpr size_t COPY_SPLIT = (size_t)1 << 20;
+constexpr int copy_threads(size_t bytes) { return bytes < ((size_t)8 << 20) ? 4 : 8; }
 // Below this the arrays of an upload go through the staging buffer and one
 // kernel (8 us and a copy at 10 GB/s); from there on a contiguous copy from
 // the caller's memory (35 GB/s, but 14 us for each array) is the faster one.
@@ -1270,8 +1272,9 @@ FieldRows field_rows(const HostChan& c, uint32_t x0, uint32_t rows) {
 }
 
 // Copies pieces of the chunks a download is cut into: piece i belongs to chunk
-// i / COPY_THREADS and may be taken once `ready` has passed that chunk.
+// i / parts and may be taken once `ready` has passed that chunk.
 struct CopyOut {
+    int parts = 1;
     std::atomic<int64_t> next{0}, done{0}, ready{0};
     std::atomic<bool> stop{false};
     int64_t pieces = 0;
@@ -1281,11 +1284,11 @@ struct CopyOut {
         for (;;) {
             const int64_t i = next.fetch_add(1);
             if (i >= pieces) return;
-            while (ready.load(std::memory_order_acquire) <= i / COPY_THREADS) {
+            while (ready.load(std::memory_order_acquire) <= i / parts) {
                 if (stop.load()) return;
                 std::this_thread::yield();
             }
-            copy(i / COPY_THREADS, (int)(i % COPY_THREADS));
+            copy(i / parts, (int)(i % parts));
             done.fetch_add(1, std::memory_order_release);
         }
     }
@@ -1295,14 +1298,15 @@ struct CopyOut {
 // fill(k) queues what brings chunk k into half k & 1, and copy(k, part, parts)
 // copies a part of it out, while chunk k + 1 is on its way.
 template <class Fill, class Copy>
-int copy_chunks(stm_ctx* ctx, int64_t chunks, Fill fill, Copy copy) {
+int copy_chunks(stm_ctx* ctx, size_t bytes, int64_t chunks, Fill fill, Copy copy) {
     int rc = fill(0);
     if (rc) return rc;
     CopyOut out;
-    out.pieces = chunks * COPY_THREADS;
-    out.copy = [&](int64_t k, int part) { copy(k, part, COPY_THREADS); };
+    const int parts = out.parts = copy_threads(bytes);
+    out.pieces = chunks * parts;
+    out.copy = [&](int64_t k, int part) { copy(k, part, parts); };
     std::vector<std::thread> team;
-    for (int t = 0; t < COPY_THREADS; t++) {
+    for (int t = 0; t < parts; t++) {
         try {
             team.emplace_back([&out] { out.run(); });
         } catch (const std::exception&) {   // no more threads to be had
@@ -1319,7 +1323,7 @@ int copy_chunks(stm_ctx* ctx, int64_t chunks, Fill fill, Copy copy) {
             copy(k, 0, 1);
         else {
             out.ready.store(k + 1, std::memory_order_release);
-            while (out.done.load(std::memory_order_acquire) < (k + 1) * COPY_THREADS)
+            while (out.done.load(std::memory_order_acquire) < (k + 1) * parts)
                 std::this_thread::yield();
         }
     }
@@ -1365,7 +1369,7 @@ int pack_to_host(stm_ctx* ctx, const HostChan& c, int n, double* const* dev,
             memcpy((char*)host[f] + row * most * k + a,
                    ctx->h_stage + (k & 1) * half + f * m + a, b - a);
     };
-    if (!whole) return copy_chunks(ctx, (c.nx + most - 1) / most, fill, copy);
+    if (!whole) return copy_chunks(ctx, all, (c.nx + most - 1) / most, fill, copy);
     int rc = fill(0);
     if (rc) return rc;
     HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
@@ -2236,7 +2240,7 @@ int ctx_download(stm_ctx* ctx, void* dst, const void* src, size_t n) {
         const auto [a, b] = part_of(size(k), part, parts);
         if (a < b) memcpy((char*)dst + k * half + a, ctx->h_stage + (k & 1) * half + a, b - a);
     };
-    return copy_chunks(ctx, (int64_t)((n + half - 1) / half), fill, copy);
+    return copy_chunks(ctx, n, (int64_t)((n + half - 1) / half), fill, copy);
 }
 
 void ctx_attach_net(stm_ctx* ctx, stm_net* net) { ctx->nets.push_back(net); }

@@ -43,6 +43,7 @@ def _round_trip(nx, ny, names):
 @pytest.mark.parametrize("nx,ny,names", [
     (3, 3, ALL), (3, 7, ("p",)), (9, 3, ("u", "rhs")), (33, 31, ("v", "p", "g")),
     (104, 105, ("u", "v", "p")), (105, 105, ("u", "v", "p")),        # 256 KB in three fields
+    (511, 256, ("p",)), (513, 256, ("p",)), (149, 147, ALL),         # 1 MB
     (511, 512, ("p",)), (513, 512, ("p",)), (211, 207, ALL),         # 2 MB
     (1031, 1027, ("p",)), (701, 1499, ("u", "v", "p")), (13, 60001, ALL),
     (3, 87000, ALL), (3, 88000, ALL), (3, 530000, ("f",)),           # rows of over 4 MB
