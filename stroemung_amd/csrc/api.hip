@@ -7,6 +7,8 @@
 // per-channel "still running" flags.
 #include <hip/hip_runtime.h>
 
+#include <sys/mman.h>
+
 #include <algorithm>
 #include <atomic>
 #include <chrono>
@@ -1216,13 +1218,12 @@ int check_params(stm_ctx* ctx, const stm_params* q) {
 
 // Pinned staging, one per context, allocated at the first transfer.
 constexpr size_t STAGE_MOST = (size_t)8 << 20;
-// A download of this much or more is copied out of the staging buffer by several
-// threads: writing fresh pages goes at 5 GB/s with one, 9 with four and 17 with
-// eight, starting a thread takes some 15 us (three fields of 258 x 258 cells, 1.5
-// MB: 292 us with one, 193 with four, 316 with eight, 221 with eight kept waiting
-// between downloads; 0.9 MB: 183, 189; 11.8 MB: 1077 with four, 989 with eight).
-constexpr size_t COPY_SPLIT = (size_t)1 << 20;
-constexpr int copy_threads(size_t bytes) { return bytes < ((size_t)8 << 20) ? 4 : 8; }
+// A download of this much or more is copied out of the staging buffer by
+// COPY_THREADS threads: writing fresh pages goes at 5 GB/s with one and at 17
+// GB/s with eight, which take 100 us to start.  A smaller one asks for its pages
+// while the kernel packs (see prefault).
+constexpr size_t COPY_SPLIT = (size_t)4 << 20;
+constexpr int COPY_THREADS = 8;
 // Below this the arrays of an upload go through the staging buffer and one
 // kernel (8 us and a copy at 10 GB/s); from there on a contiguous copy from
 // the caller's memory (35 GB/s, but 14 us for each array) is the faster one.
@@ -1272,9 +1273,8 @@ FieldRows field_rows(const HostChan& c, uint32_t x0, uint32_t rows) {
 }
 
 // Copies pieces of the chunks a download is cut into: piece i belongs to chunk
-// i / parts and may be taken once `ready` has passed that chunk.
+// i / COPY_THREADS and may be taken once `ready` has passed that chunk.
 struct CopyOut {
-    int parts = 1;
     std::atomic<int64_t> next{0}, done{0}, ready{0};
     std::atomic<bool> stop{false};
     int64_t pieces = 0;
@@ -1284,11 +1284,11 @@ struct CopyOut {
         for (;;) {
             const int64_t i = next.fetch_add(1);
             if (i >= pieces) return;
-            while (ready.load(std::memory_order_acquire) <= i / parts) {
+            while (ready.load(std::memory_order_acquire) <= i / COPY_THREADS) {
                 if (stop.load()) return;
                 std::this_thread::yield();
             }
-            copy(i / parts, (int)(i % parts));
+            copy(i / COPY_THREADS, (int)(i % COPY_THREADS));
             done.fetch_add(1, std::memory_order_release);
         }
     }
@@ -1298,15 +1298,14 @@ struct CopyOut {
 // fill(k) queues what brings chunk k into half k & 1, and copy(k, part, parts)
 // copies a part of it out, while chunk k + 1 is on its way.
 template <class Fill, class Copy>
-int copy_chunks(stm_ctx* ctx, size_t bytes, int64_t chunks, Fill fill, Copy copy) {
+int copy_chunks(stm_ctx* ctx, int64_t chunks, Fill fill, Copy copy) {
     int rc = fill(0);
     if (rc) return rc;
     CopyOut out;
-    const int parts = out.parts = copy_threads(bytes);
-    out.pieces = chunks * parts;
-    out.copy = [&](int64_t k, int part) { copy(k, part, parts); };
+    out.pieces = chunks * COPY_THREADS;
+    out.copy = [&](int64_t k, int part) { copy(k, part, COPY_THREADS); };
     std::vector<std::thread> team;
-    for (int t = 0; t < parts; t++) {
+    for (int t = 0; t < COPY_THREADS; t++) {
         try {
             team.emplace_back([&out] { out.run(); });
         } catch (const std::exception&) {   // no more threads to be had
@@ -1323,7 +1322,7 @@ int copy_chunks(stm_ctx* ctx, size_t bytes, int64_t chunks, Fill fill, Copy copy
             copy(k, 0, 1);
         else {
             out.ready.store(k + 1, std::memory_order_release);
-            while (out.done.load(std::memory_order_acquire) < (k + 1) * parts)
+            while (out.done.load(std::memory_order_acquire) < (k + 1) * COPY_THREADS)
                 std::this_thread::yield();
         }
     }
@@ -1331,6 +1330,17 @@ int copy_chunks(stm_ctx* ctx, size_t bytes, int64_t chunks, Fill fill, Copy copy
     for (std::thread& t : team) t.join();
     HIPCHK(ctx, e);
     return rc;
+}
+
+// Asks for the pages of memory that is about to be written, in one call instead
+// of a fault for each (0.9 MB in three fresh arrays, with their copy: 184 -> 109
+// us).  Nothing is written, and what it refuses the copy faults in.
+void prefault(void* p, size_t n) {
+#ifdef MADV_POPULATE_WRITE
+    const uintptr_t page = 4096, a = ((uintptr_t)p + page - 1) / page * page,
+                    b = ((uintptr_t)p + n) / page * page;
+    if (b >= a + 8 * page) (void)madvise((void*)a, b - a, MADV_POPULATE_WRITE);
+#endif
 }
 
 // Part `part` of `parts` of n bytes: its start and end (multiples of 4 KB but the last).
@@ -1369,9 +1379,10 @@ int pack_to_host(stm_ctx* ctx, const HostChan& c, int n, double* const* dev,
             memcpy((char*)host[f] + row * most * k + a,
                    ctx->h_stage + (k & 1) * half + f * m + a, b - a);
     };
-    if (!whole) return copy_chunks(ctx, all, (c.nx + most - 1) / most, fill, copy);
+    if (!whole) return copy_chunks(ctx, (c.nx + most - 1) / most, fill, copy);
     int rc = fill(0);
     if (rc) return rc;
+    for (int f = 0; f < n; f++) prefault(host[f], row * c.nx);
     HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
     copy(0, 0, 1);
     return STM_OK;
@@ -2225,6 +2236,7 @@ void ctx_stage(stm_ctx* ctx, size_t n) {
 // src (device) to dst (the caller's memory) in stream order, and waits for it.
 int ctx_download(stm_ctx* ctx, void* dst, const void* src, size_t n) {
     if (n < COPY_SPLIT || !stage_buffer(ctx, 2 * n)) {
+        prefault(dst, n);   // (the runtime's copy to pageable memory faults page by page too)
         HIPCHK(ctx, hipMemcpyAsync(dst, src, n, hipMemcpyDeviceToHost, ctx->stream));
         HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
         return STM_OK;
@@ -2240,7 +2252,7 @@ int ctx_download(stm_ctx* ctx, void* dst, const void* src, size_t n) {
         const auto [a, b] = part_of(size(k), part, parts);
         if (a < b) memcpy((char*)dst + k * half + a, ctx->h_stage + (k & 1) * half + a, b - a);
     };
-    return copy_chunks(ctx, n, (int64_t)((n + half - 1) / half), fill, copy);
+    return copy_chunks(ctx, (int64_t)((n + half - 1) / half), fill, copy);
 }
 
 void ctx_attach_net(stm_ctx* ctx, stm_net* net) { ctx->nets.push_back(net); }
