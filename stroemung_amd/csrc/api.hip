@@ -789,7 +789,7 @@ int blocked_solve(stm_ctx* ctx, int check, int fixed = 0) {
     }
     ctx->tb_cur = ctx->d_tb;
     ctx->ntb_cur = ctx->ntb;
-    LAUNCH("pbuf_fix", launch_pbuf_fix(ctx->stream, ctx->ntiles, nch(ctx), ctx->d_cd, ctx->d_cs,
+    LAUNCH("pbuf_fix", launch_pbuf_fix(ctx->stream, ctx->ntiles, ctx->d_cd, ctx->d_cs,
                                        ctx->d_tiles, ctx->p2, ctx->p));
     return STM_OK;
 }
@@ -845,7 +845,7 @@ int learn_phase(stm_ctx* ctx, int budget, int final_phase) {
                                                          ctx->d_lc, nl));
         // the channels whose latest p is in the second buffer copy it back
         // (after an odd number of launches, or a clamped budget's stop)
-        LAUNCH("pbuf_fix", launch_pbuf_fix(ctx->stream, ctx->ntiles, nch(ctx), ctx->d_cd,
+        LAUNCH("pbuf_fix", launch_pbuf_fix(ctx->stream, ctx->ntiles, ctx->d_cd,
                                            ctx->d_cs, ctx->d_tiles, ctx->p2, ctx->p));
         if (!final_phase) return STM_OK;   // the sweeps are counted by learn_phase_end
     } else {

@@ -103,7 +103,7 @@ void launch_rb_tb(hipStream_t, int variant, int ntb, const ChanDesc*, ChanState*
                   const TbWave* waves, const uint32_t* words, const double* rhs, double* pa,
                   double* pb, const double* part_prev, double* part_cur, int32_t* active, int L,
                   int mode);
-void launch_pbuf_fix(hipStream_t, int ntiles, int nchan, const ChanDesc*, ChanState*,
+void launch_pbuf_fix(hipStream_t, int ntiles, const ChanDesc*, const ChanState*,
                      const Tile*, const double* pb, double* pa);
 
 // kernels_view.hip: the GUI image of one channel (npix = nx * ny pixels)

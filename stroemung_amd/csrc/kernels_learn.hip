@@ -36,6 +36,7 @@
 
 #include "kernels.h"
 #include "stm_internal.h"
+#include "wave.h"
 
 namespace stm {
 
@@ -45,42 +46,21 @@ __device__ __forceinline__ bool interior(const ChanDesc& d, int x, int y) {
     return x >= 1 && x <= d.nx - 2 && y >= 1 && y <= d.ny - 2;
 }
 
-__device__ __forceinline__ double lap(const double* __restrict__ a, int64_t i, int64_t P,
-                                      double rdx2, double rdy2) {
-    const double c = a[i];
-    return fma((a[i + P] - c) - (c - a[i - P]), rdx2, ((a[i + 1] - c) - (c - a[i - 1])) * rdy2);
-}
-
-// Lap(a - b) at i, differences taken cell by cell.
-__device__ __forceinline__ double lap_diff(const double* __restrict__ a,
-                                           const double* __restrict__ b, int64_t i, int64_t P,
-                                           double rdx2, double rdy2) {
-    const double c = a[i] - b[i];
-    const double e = a[i + P] - b[i + P], w = a[i - P] - b[i - P];
-    const double n = a[i - 1] - b[i - 1], so = a[i + 1] - b[i + 1];
-    return fma((e - c) - (c - w), rdx2, ((so - c) - (c - n)) * rdy2);
-}
-
 // Sums of N values over one tile block into part[blockIdx.x * NPART +
-// slot[j]]: a fixed-order shuffle reduction inside each wave, then the
-// TILE_THREADS / 64 wave sums added in wave order.  sh holds N * that many
-// doubles; a call ends with a barrier, so sh can be reused at once.
+// slot[j]]: over the wave in a fixed order, then the TILE_THREADS / 64 wave sums
+// added in wave order.  sh holds N * that many doubles; a call ends with a
+// barrier, so sh can be reused at once.
 template <int N>
 __device__ void tile_sums(const double (&v)[N], double* sh, double* __restrict__ part,
                           const int (&slot)[N]) {
     constexpr int NW = TILE_THREADS / 64;
     const int tid = threadIdx.y * blockDim.x + threadIdx.x;
     const int lane = tid & 63, wave = tid >> 6;
-    double r[N];
 #pragma unroll
-    for (int j = 0; j < N; j++) r[j] = v[j];
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1)
-#pragma unroll
-        for (int j = 0; j < N; j++) r[j] = r[j] + __shfl_down(r[j], off, 64);
-    if (lane == 0)
-#pragma unroll
-        for (int j = 0; j < N; j++) sh[j * NW + wave] = r[j];
+    for (int j = 0; j < N; j++) {
+        const double r = wave_sum(v[j]);
+        if (lane == 0) sh[j * NW + wave] = r;
+    }
     __syncthreads();
     if (tid < N) {
         double acc = 0.0;
@@ -97,6 +77,42 @@ __device__ void tile_sum(double v, double* sh, double* __restrict__ part, int sl
     tile_sums<1>(vv, sh, part, ss);
 }
 
+// A wave per tile, its lanes the tile's columns: cell r of a lane is
+// (t.x0 + r, t.y0 + lane).  False beyond the list.
+__device__ __forceinline__ bool wave_tile(const Tile* __restrict__ tiles, int ntiles, int& k,
+                                          Tile& t) {
+    k = __builtin_amdgcn_readfirstlane(blockIdx.x * (TILE_THREADS / 64) + threadIdx.x / 64);
+    if (k >= ntiles) return false;
+    t = tiles[k];
+    return true;
+}
+
+// A lane's column of a tile: a, or a - b, at rows -1 .. TILE_X and the N and S
+// neighbours of rows 0 .. TILE_X - 1 (addresses clamped into the channel, so
+// the loads carry no branches; only interior cells use what they hold).
+struct Column {
+    double c[TILE_X + 2], n[TILE_X], s[TILE_X];
+    __device__ __forceinline__ void load(const ChanDesc& d, const Tile& t, int y,
+                                         const double* __restrict__ a,
+                                         const double* __restrict__ b) {
+        const int yc = min(y, d.ny - 1), yn = max(yc - 1, 0), ys = min(yc + 1, d.ny - 1);
+#pragma unroll
+        for (int r = 0; r < TILE_X + 2; r++) {
+            const int64_t row = d.off + min(max(t.x0 + r - 1, 0), d.nx - 1) * (int64_t)d.pitch;
+            c[r] = b ? a[row + yc] - b[row + yc] : a[row + yc];
+            if (r >= 1 && r <= TILE_X) {
+                n[r - 1] = b ? a[row + yn] - b[row + yn] : a[row + yn];
+                s[r - 1] = b ? a[row + ys] - b[row + ys] : a[row + ys];
+            }
+        }
+    }
+    __device__ __forceinline__ double at(int r) const { return c[r + 1]; }
+    __device__ __forceinline__ double lap(int r, double rdx2, double rdy2) const {
+        const double m = c[r + 1];
+        return fma((c[r + 2] - m) - (m - c[r]), rdx2, ((s[r] - m) - (m - n[r])) * rdy2);
+    }
+};
+
 // Block sum (256 threads, 1-D) returned to every thread.
 __device__ double block_total(double v, double* sh) {
     const int tid = threadIdx.x;
@@ -111,13 +127,33 @@ __device__ double block_total(double v, double* sh) {
     return r;
 }
 
-// One channel's partials of `slot` summed in a fixed order (256 threads).
+// One channel's partials of N slots, each summed in a fixed order (256
+// threads), returned to every thread; sh holds 4 * N doubles.  A tile's slots
+// share a 128-byte line, so they are read together.
+template <int N>
+__device__ void chan_totals(const ChanDesc& d, const double* __restrict__ part,
+                            const int (&slot)[N], double (&out)[N], double* sh) {
+    double acc[N] = {};
+    for (int k = d.tile0 + threadIdx.x; k < d.tile0 + d.ntiles; k += 256)
+#pragma unroll
+        for (int j = 0; j < N; j++) acc[j] = acc[j] + part[(int64_t)k * NPART + slot[j]];
+#pragma unroll
+    for (int j = 0; j < N; j++) {
+        const double w = wave_sum(acc[j]);
+        if ((threadIdx.x & 63) == 0) sh[j * 4 + threadIdx.x / 64] = w;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < N; j++)
+        out[j] = (sh[j * 4] + sh[j * 4 + 1]) + (sh[j * 4 + 2] + sh[j * 4 + 3]);
+    __syncthreads();
+}
 __device__ double chan_total(const ChanDesc& d, const double* __restrict__ part, int slot,
                              double* sh) {
-    double acc = 0.0;
-    for (int k = d.tile0 + threadIdx.x; k < d.tile0 + d.ntiles; k += blockDim.x)
-        acc = acc + part[(int64_t)k * NPART + slot];
-    return block_total(acc, sh);
+    const int slots[1] = {slot};
+    double out[1];
+    chan_totals<1>(d, part, slots, out, sh);
+    return out[0];
 }
 
 constexpr int S_RES2 = 2, S_RZ = 3, S_ZQ = 4, S_DSUM = 5;
@@ -156,30 +192,38 @@ __device__ __forceinline__ double block_fine_sum(const ChanDesc& d, const uint8_
 // r = Lap(p) - (rhs - mean) at interior fluid cells, 0 elsewhere; slot 2 = sum r^2.
 // p's ghosts must be current.  After the first phase of a solve, tiles of
 // channels that are no longer running are skipped (their r and slot 2 are
-// read only while a channel runs).
+// read only while a channel runs).  A wave per tile, four cells a lane (a
+// thread per cell spent as long on the sum as on memory: 16.5 us for 32
+// channels of 258 x 258, 12.8 now).
 __global__ void __launch_bounds__(TILE_THREADS)
 k_learn_residual(const ChanDesc* __restrict__ cd, const ChanState* __restrict__ cs,
                  const LearnChan* __restrict__ lc, int first,
-                 const Tile* __restrict__ tiles, const uint8_t* __restrict__ flags,
+                 const Tile* __restrict__ tiles, int ntiles, const uint8_t* __restrict__ flags,
                  const double* __restrict__ rhs, const double* __restrict__ p,
                  double* __restrict__ res, double* __restrict__ part)
 {
-    __shared__ double sh[TILE_THREADS];
-    const Tile t = tiles[blockIdx.x];
-    if (!first && !lc[t.chan].run) return;       // uniform over the block, before any barrier
+    int k;
+    Tile t;
+    if (!wave_tile(tiles, ntiles, k, t)) return;
+    if (!first && !lc[t.chan].run) return;
     const ChanDesc& d = cd[t.chan];
-    const int x = t.x0 + threadIdx.y, y = t.y0 + threadIdx.x;
+    const int lane = threadIdx.x & 63, y = t.y0 + lane;
+    const double mean = cs[t.chan].rhs_mean;
+    Column pc;
+    pc.load(d, t, y, p, nullptr);
     double r2 = 0.0;
-    if (x < d.nx && y < d.ny) {
+#pragma unroll
+    for (int q = 0; q < TILE_X; q++) {
+        const int x = t.x0 + q;
+        if (x >= d.nx || y >= d.ny) continue;
         const int64_t i = d.off + x * (int64_t)d.pitch + y;
-        double r = 0.0;
-        if (interior(d, x, y) && flag_fluid(flags[i])) {
-            r = lap(p, i, d.pitch, d.rdx2, d.rdy2) - (rhs[i] - cs[t.chan].rhs_mean);
-            r2 = r * r;
-        }
+        const double v = pc.lap(q, d.rdx2, d.rdy2) - (rhs[i] - mean);
+        const double r = interior(d, x, y) && flag_fluid(flags[i]) ? v : 0.0;
+        r2 = r2 + r * r;
         res[i] = r;
     }
-    tile_sum(r2, sh, part, S_RES2);
+    r2 = wave_sum(r2);
+    if (lane == 0) part[(int64_t)k * NPART + S_RES2] = r2;
 }
 
 // Per channel: has the solve converged?  first = 1 at the start of a solve.
@@ -334,39 +378,59 @@ k_learn_pack(const LearnChan* __restrict__ lc, const float* __restrict__ rc,
 // other cells (boundary ghosts are set afterwards).  Fine interior index u
 // lies at coarse coordinate (u + 1/2) / f - 1/2 (pixel centres at integers);
 // the four surrounding pixels are weighted bilinearly and by fluid fraction.
+// A wave per tile, four cells a lane: what a cell waits for (its tile, channel,
+// flag, pixels) is waited for once for four (17.7 us for 32 channels of 258 x 258
+// with a cell a thread, 12.5 now).
 __global__ void __launch_bounds__(TILE_THREADS)
-k_learn_prolong(const ChanDesc* __restrict__ cd, const Tile* __restrict__ tiles,
+k_learn_prolong(const ChanDesc* __restrict__ cd, const Tile* __restrict__ tiles, int ntiles,
                 const LearnChan* __restrict__ lc, const uint8_t* __restrict__ flags,
                 const float* __restrict__ y, const float* __restrict__ mc, int H, int W, int f,
                 const int32_t* __restrict__ inv, double* __restrict__ cf)
 {
-    const Tile t = tiles[blockIdx.x];
+    int k;
+    Tile t;
+    if (!wave_tile(tiles, ntiles, k, t)) return;
+    const int entry = inv ? inv[t.chan] : t.chan;     // its batch entry
     if (!lc[t.chan].run) return;                 // z of a stopped channel is never used
     const ChanDesc& d = cd[t.chan];
-    const int x = t.x0 + threadIdx.y, yy = t.y0 + threadIdx.x;
-    if (x >= d.nx || yy >= d.ny) return;
-    const int64_t i = d.off + x * (int64_t)d.pitch + yy;
-    double v = 0.0;
-    if (interior(d, x, yy) && flag_fluid(flags[i])) {
-        const int hc_n = (d.nx - 2 + f - 1) / f, wc_n = (d.ny - 2 + f - 1) / f;
-        const double xi = fmin(fmax(((x - 1) + 0.5) / f - 0.5, 0.0), (double)(hc_n - 1));
-        const double eta = fmin(fmax(((yy - 1) + 0.5) / f - 0.5, 0.0), (double)(wc_n - 1));
-        const int i0 = (int)xi, j0 = (int)eta;
-        const int i1 = i0 + 1 < hc_n ? i0 + 1 : i0, j1 = j0 + 1 < wc_n ? j0 + 1 : j0;
-        const double tx = xi - i0, ty = eta - j0;
-        const int64_t base = (int64_t)t.chan * H * W;     // channel's frame in mc
-        const int64_t ybase = (int64_t)(inv ? inv[t.chan] : t.chan) * H * W;  // its batch entry
-        const int64_t k00 = (int64_t)i0 * W + j0, k01 = (int64_t)i0 * W + j1;
-        const int64_t k10 = (int64_t)i1 * W + j0, k11 = (int64_t)i1 * W + j1;
-        const double w00 = (1.0 - tx) * (1.0 - ty) * mc[base + k00];
-        const double w01 = (1.0 - tx) * ty * mc[base + k01];
-        const double w10 = tx * (1.0 - ty) * mc[base + k10], w11 = tx * ty * mc[base + k11];
-        const double ws = (w00 + w01) + (w10 + w11);
-        if (ws > 0.0)
-            v = ((w00 * y[ybase + k00] + w01 * y[ybase + k01]) +
-                 (w10 * y[ybase + k10] + w11 * y[ybase + k11])) / ws;
+    const int yy = t.y0 + (threadIdx.x & 63);
+    if (yy >= d.ny) return;
+    const int hc_n = (d.nx - 2 + f - 1) / f, wc_n = (d.ny - 2 + f - 1) / f;
+    const double rf = 1.0 / f;   // f is a power of two: exact, and so are the products
+    const double eta = fmin(fmax(((yy - 1) + 0.5) * rf - 0.5, 0.0), (double)(wc_n - 1));
+    const int j0 = (int)eta, j1 = j0 + 1 < wc_n ? j0 + 1 : j0;
+    const double ty = eta - j0;
+    const float* mb = mc + (int64_t)t.chan * H * W;     // channel's frame in mc
+    const float* yb = y + (int64_t)entry * H * W;
+    uint8_t fl[TILE_X];
+    float m[TILE_X][4], v[TILE_X][4];
+    double tx[TILE_X];
+#pragma unroll
+    for (int q = 0; q < TILE_X; q++) {
+        const int x = min(t.x0 + q, d.nx - 1);
+        fl[q] = flags[d.off + x * (int64_t)d.pitch + yy];
+        const double xi = fmin(fmax(((x - 1) + 0.5) * rf - 0.5, 0.0), (double)(hc_n - 1));
+        const int i0 = (int)xi, i1 = i0 + 1 < hc_n ? i0 + 1 : i0;
+        tx[q] = xi - i0;
+        const int at[4] = {i0 * W + j0, i0 * W + j1, i1 * W + j0, i1 * W + j1};
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            m[q][j] = mb[at[j]];
+            v[q][j] = yb[at[j]];
+        }
     }
-    cf[i] = v;
+#pragma unroll
+    for (int q = 0; q < TILE_X; q++) {
+        const int x = t.x0 + q;
+        if (x >= d.nx) continue;
+        const double w00 = (1.0 - tx[q]) * (1.0 - ty) * m[q][0];
+        const double w01 = (1.0 - tx[q]) * ty * m[q][1];
+        const double w10 = tx[q] * (1.0 - ty) * m[q][2], w11 = tx[q] * ty * m[q][3];
+        const double ws = (w00 + w01) + (w10 + w11);
+        const double z = ((w00 * v[q][0] + w01 * v[q][1]) + (w10 * v[q][2] + w11 * v[q][3])) / ws;
+        cf[d.off + x * (int64_t)d.pitch + yy] =
+            interior(d, x, yy) && flag_fluid(fl[q]) && ws > 0.0 ? z : 0.0;
+    }
 }
 
 // q = Lap(z) at interior fluid cells: slot 3 = sum r z, slot 4 = sum z q
@@ -374,55 +438,68 @@ k_learn_prolong(const ChanDesc* __restrict__ cd, const Tile* __restrict__ tiles,
 // prev != nullptr also s = p - prev, the change of p over the previous cycle
 // (p and prev both hold ghosts consistent with their interiors, so s does):
 // slot 0 = sum r s, slot 1 = sum s Lap(s), slot 6 = sum z Lap(s).
+// A wave per tile, four cells a lane, summed by DPP (a thread per cell, its nine
+// sums shuffled
+// through LDS, took 32.6 us for 32 channels of 258 x 258, 29.4 now).
 __global__ void __launch_bounds__(TILE_THREADS)
-k_learn_dots(const ChanDesc* __restrict__ cd, const Tile* __restrict__ tiles,
+k_learn_dots(const ChanDesc* __restrict__ cd, const Tile* __restrict__ tiles, int ntiles,
              const LearnChan* __restrict__ lc, const uint8_t* __restrict__ flags,
              const double* __restrict__ res, const double* __restrict__ cf,
              const double* __restrict__ p, const double* __restrict__ prev,
              const double* __restrict__ prev2, double* __restrict__ part)
 {
-    __shared__ double sh[TILE_THREADS];
-    const Tile t = tiles[blockIdx.x];
-    if (!lc[t.chan].run) return;                 // uniform over the block, before any barrier
+    int k;
+    Tile t;
+    if (!wave_tile(tiles, ntiles, k, t) || !lc[t.chan].run) return;
     const ChanDesc& d = cd[t.chan];
-    const int x = t.x0 + threadIdx.y, y = t.y0 + threadIdx.x;
-    double rz = 0.0, zq = 0.0, rs = 0.0, sq = 0.0, zs = 0.0;
-    double rs2 = 0.0, s2q = 0.0, zs2 = 0.0, s1s2 = 0.0;
-    if (x < d.nx && y < d.ny && interior(d, x, y)) {
-        const int64_t i = d.off + x * (int64_t)d.pitch + y;
-        if (flag_fluid(flags[i])) {
-            const double q = lap(cf, i, d.pitch, d.rdx2, d.rdy2);
-            rz = res[i] * cf[i];
-            zq = cf[i] * q;
-            if (prev) {
-                const double sv = p[i] - prev[i];
-                const double ls = lap_diff(p, prev, i, d.pitch, d.rdx2, d.rdy2);
-                rs = res[i] * sv;
-                sq = sv * ls;
-                zs = cf[i] * ls;
-                if (prev2) {
-                    const double s2 = prev[i] - prev2[i];
-                    const double l2 = lap_diff(prev, prev2, i, d.pitch, d.rdx2, d.rdy2);
-                    rs2 = res[i] * s2;
-                    s2q = s2 * l2;
-                    zs2 = cf[i] * l2;
-                    s1s2 = sv * l2;
-                }
+    const int lane = threadIdx.x & 63, y = t.y0 + lane;
+    double v[9] = {};   // rz, zq; rs, sq, zs; rs2, s2q, zs2, s1s2
+    bool use[TILE_X];
+    double r[TILE_X];
+#pragma unroll
+    for (int q = 0; q < TILE_X; q++) {
+        const int x = t.x0 + q;
+        const int64_t i = d.off + min(x, d.nx - 1) * (int64_t)d.pitch + min(y, d.ny - 1);
+        use[q] = interior(d, x, y) && flag_fluid(flags[i]);
+        r[q] = res[i];
+    }
+    auto add = [&](int j, int q, double term) { v[j] = v[j] + (use[q] ? term : 0.0); };
+    Column z;
+    z.load(d, t, y, cf, nullptr);
+#pragma unroll
+    for (int q = 0; q < TILE_X; q++) {
+        add(0, q, r[q] * z.at(q));
+        add(1, q, z.at(q) * z.lap(q, d.rdx2, d.rdy2));
+    }
+    if (prev) {
+        Column s;
+        s.load(d, t, y, p, prev);
+#pragma unroll
+        for (int q = 0; q < TILE_X; q++) {
+            const double ls = s.lap(q, d.rdx2, d.rdy2);
+            add(2, q, r[q] * s.at(q));
+            add(3, q, s.at(q) * ls);
+            add(4, q, z.at(q) * ls);
+        }
+        if (prev2) {
+            Column s2;
+            s2.load(d, t, y, prev, prev2);
+#pragma unroll
+            for (int q = 0; q < TILE_X; q++) {
+                const double l2 = s2.lap(q, d.rdx2, d.rdy2);
+                add(5, q, r[q] * s2.at(q));
+                add(6, q, s2.at(q) * l2);
+                add(7, q, z.at(q) * l2);
+                add(8, q, s.at(q) * l2);
             }
         }
     }
-    if (prev2) {
-        const double v[9] = {rz, zq, rs, sq, zs, rs2, s2q, zs2, s1s2};
-        const int slots[9] = {S_RZ, S_ZQ, S_RS, S_SQ, S_ZS, S_RS2, S_S2Q, S_ZS2, S_S1S2};
-        tile_sums<9>(v, sh, part, slots);
-    } else if (prev) {
-        const double v[5] = {rz, zq, rs, sq, zs};
-        const int slots[5] = {S_RZ, S_ZQ, S_RS, S_SQ, S_ZS};
-        tile_sums<5>(v, sh, part, slots);
-    } else {
-        const double v[2] = {rz, zq};
-        const int slots[2] = {S_RZ, S_ZQ};
-        tile_sums<2>(v, sh, part, slots);
+    constexpr int slots[9] = {S_RZ, S_ZQ, S_RS, S_SQ, S_ZS, S_RS2, S_S2Q, S_ZS2, S_S1S2};
+    const int n = prev2 ? 9 : prev ? 5 : 2;
+#pragma unroll
+    for (int j = 0; j < 9; j++) {
+        const double w = j < n ? wave_sum(v[j]) : 0.0;
+        if (j < n && lane == 0) part[(int64_t)k * NPART + slots[j]] = w;
     }
 }
 
@@ -441,23 +518,15 @@ k_learn_alpha(const ChanDesc* __restrict__ cd, LearnChan* __restrict__ lc,
     __shared__ double sh[256];
     const int c = blockIdx.x;
     const ChanDesc& d = cd[c];
-    const double rz = chan_total(d, part, S_RZ, sh);
-    const double zq = chan_total(d, part, S_ZQ, sh);
     // kept previous p's: step 2 has one after the first cycle, step 3 counts
-    // them per channel (the graph-replayed cycles cannot be told apart)
+    // them per channel (the graph-replayed cycles cannot be told apart); the
+    // sums of those there are not are read but not used
     const int hist = step == 3 ? lc[c].hist : ((step == 2 && !first) ? 1 : 0);
-    double rs = 0.0, sq = 0.0, zs = 0.0, rs2 = 0.0, s2q = 0.0, zs2 = 0.0, s1s2 = 0.0;
-    if (hist >= 1) {
-        rs = chan_total(d, part, S_RS, sh);
-        sq = chan_total(d, part, S_SQ, sh);
-        zs = chan_total(d, part, S_ZS, sh);
-    }
-    if (hist >= 2) {
-        rs2 = chan_total(d, part, S_RS2, sh);
-        s2q = chan_total(d, part, S_S2Q, sh);
-        zs2 = chan_total(d, part, S_ZS2, sh);
-        s1s2 = chan_total(d, part, S_S1S2, sh);
-    }
+    constexpr int slots[9] = {S_RZ, S_ZQ, S_RS, S_SQ, S_ZS, S_RS2, S_S2Q, S_ZS2, S_S1S2};
+    double v[9];
+    chan_totals<9>(d, part, slots, v, sh);
+    const double rz = v[0], zq = v[1], rs = v[2], sq = v[3], zs = v[4];
+    const double rs2 = v[5], s2q = v[6], zs2 = v[7], s1s2 = v[8];
     if (threadIdx.x) return;
     LearnChan& l = lc[c];
     double a = 0.0, b = 0.0, g = 0.0;
@@ -505,36 +574,52 @@ k_learn_alpha(const ChanDesc* __restrict__ cd, LearnChan* __restrict__ lc,
 // p += alpha * z at interior fluid cells; with prev != nullptr (the
 // two-direction step) p += alpha * z + beta * (p - prev), and prev takes the
 // old p.
+// (A wave per tile, as k_learn_prolong.)
 __global__ void __launch_bounds__(TILE_THREADS)
-k_learn_apply(const ChanDesc* __restrict__ cd, const Tile* __restrict__ tiles,
+k_learn_apply(const ChanDesc* __restrict__ cd, const Tile* __restrict__ tiles, int ntiles,
               const LearnChan* __restrict__ lc, const uint8_t* __restrict__ flags,
               const double* __restrict__ cf, double* __restrict__ p, double* __restrict__ prev,
               double* __restrict__ prev2)
 {
-    const Tile t = tiles[blockIdx.x];
+    int k;
+    Tile t;
+    if (!wave_tile(tiles, ntiles, k, t)) return;
     const ChanDesc& d = cd[t.chan];
-    const double a = lc[t.chan].alpha;
-    const int x = t.x0 + threadIdx.y, y = t.y0 + threadIdx.x;
-    if (prev) {
-        // two-direction step: every cell of a running channel also keeps
-        // the p it had (ghosts included) for the next cycle's s
-        if (!lc[t.chan].run || x >= d.nx || y >= d.ny) return;
-        const double b = lc[t.chan].beta;
+    const LearnChan& l = lc[t.chan];
+    const double a = l.alpha, b = l.beta, g = l.gamma;
+    const int y = t.y0 + (threadIdx.x & 63);
+    if (y >= d.ny) return;
+    // two-direction step: every cell of a running channel also keeps
+    // the p it had (ghosts included) for the next cycle's s
+    if (prev ? !l.run : a == 0.0) return;
+    double po[TILE_X], pp[TILE_X], p2[TILE_X], z[TILE_X];
+    bool in[TILE_X];
+#pragma unroll
+    for (int q = 0; q < TILE_X; q++) {
+        const int x = min(t.x0 + q, d.nx - 1);
         const int64_t i = d.off + x * (int64_t)d.pitch + y;
-        const double po = p[i], pp = prev[i];
-        if (interior(d, x, y) && flag_fluid(flags[i])) {
-            double v = fma(b, po - pp, fma(a, cf[i], po));
-            if (prev2) v = fma(lc[t.chan].gamma, pp - prev2[i], v);
-            p[i] = v;
-        }
-        if (prev2) prev2[i] = pp;
-        prev[i] = po;
-        return;
+        in[q] = interior(d, x, y) && flag_fluid(flags[i]);
+        po[q] = p[i];
+        z[q] = cf[i];
+        pp[q] = prev ? prev[i] : 0.0;
+        p2[q] = prev2 ? prev2[i] : 0.0;
     }
-    if (a == 0.0) return;
-    if (x >= d.nx || y >= d.ny || !interior(d, x, y)) return;
-    const int64_t i = d.off + x * (int64_t)d.pitch + y;
-    if (flag_fluid(flags[i])) p[i] = fma(a, cf[i], p[i]);
+#pragma unroll
+    for (int q = 0; q < TILE_X; q++) {
+        const int x = t.x0 + q;
+        if (x >= d.nx) continue;
+        const int64_t i = d.off + x * (int64_t)d.pitch + y;
+        double v = fma(a, z[q], po[q]);
+        if (prev) {
+            v = fma(b, po[q] - pp[q], v);
+            if (prev2) {
+                v = fma(g, pp[q] - p2[q], v);
+                prev2[i] = pp[q];
+            }
+            prev[i] = po[q];
+        }
+        if (in[q]) p[i] = v;
+    }
 }
 
 // Start of a blocked phase: running channels get `budget` sweeps (0 = the
@@ -666,11 +751,15 @@ static const dim3 TB(TILE_Y, TILE_X);
 
 int learn_coarse_blocks(int H, int W) { return (int)nb256((int64_t)H * W); }
 
+static unsigned wave_tiles(int ntiles) {   // workgroups of a wave per tile
+    return (unsigned)((ntiles + TILE_THREADS / 64 - 1) / (TILE_THREADS / 64));
+}
 void launch_learn_residual(hipStream_t st, int ntiles, const ChanDesc* cd, const ChanState* cs,
                            const LearnChan* lc, int first, const Tile* tiles,
                            const uint8_t* flags, const double* rhs, const double* p, double* res,
                            double* part) {
-    k_learn_residual<<<ntiles, TB, 0, st>>>(cd, cs, lc, first, tiles, flags, rhs, p, res, part);
+    k_learn_residual<<<wave_tiles(ntiles), TILE_THREADS, 0, st>>>(cd, cs, lc, first, tiles, ntiles, flags,
+                                                              rhs, p, res, part);
 }
 void launch_learn_check(hipStream_t st, int nch, const ChanDesc* cd, ChanState* cs, LearnChan* lc,
                         const double* part, int first) {
@@ -696,13 +785,14 @@ void launch_learn_pack(hipStream_t st, int nch, const LearnChan* lc, const float
 void launch_learn_prolong(hipStream_t st, int ntiles, const ChanDesc* cd, const Tile* tiles,
                           const LearnChan* lc, const uint8_t* flags, const float* y,
                           const float* mc, int H, int W, int f, const int32_t* inv, double* cf) {
-    k_learn_prolong<<<ntiles, TB, 0, st>>>(cd, tiles, lc, flags, y, mc, H, W, f, inv, cf);
+    k_learn_prolong<<<wave_tiles(ntiles), TILE_THREADS, 0, st>>>(cd, tiles, ntiles, lc, flags, y, mc, H, W, f, inv, cf);
 }
 void launch_learn_dots(hipStream_t st, int ntiles, const ChanDesc* cd, const Tile* tiles,
                        const LearnChan* lc, const uint8_t* flags, const double* res,
                        const double* cf, const double* p, const double* prev,
                        const double* prev2, double* part) {
-    k_learn_dots<<<ntiles, TB, 0, st>>>(cd, tiles, lc, flags, res, cf, p, prev, prev2, part);
+    k_learn_dots<<<wave_tiles(ntiles), TILE_THREADS, 0, st>>>(cd, tiles, ntiles, lc, flags, res, cf, p, prev,
+                                                          prev2, part);
 }
 void launch_learn_alpha(hipStream_t st, int nch, const ChanDesc* cd, LearnChan* lc,
                         const double* part, int step, int f, int first) {
@@ -711,7 +801,7 @@ void launch_learn_alpha(hipStream_t st, int nch, const ChanDesc* cd, LearnChan* 
 void launch_learn_apply(hipStream_t st, int ntiles, const ChanDesc* cd, const Tile* tiles,
                         const LearnChan* lc, const uint8_t* flags, const double* cf, double* p,
                         double* prev, double* prev2) {
-    k_learn_apply<<<ntiles, TB, 0, st>>>(cd, tiles, lc, flags, cf, p, prev, prev2);
+    k_learn_apply<<<wave_tiles(ntiles), TILE_THREADS, 0, st>>>(cd, tiles, ntiles, lc, flags, cf, p, prev, prev2);
 }
 void launch_learn_arm(hipStream_t st, int nch, const ChanDesc* cd, ChanState* cs,
                       const LearnChan* lc, int32_t* active, int budget) {

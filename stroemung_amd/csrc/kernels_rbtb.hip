@@ -64,6 +64,7 @@
 
 #include "kernels.h"
 #include "stm_internal.h"
+#include "wave.h"
 
 namespace stm {
 
@@ -94,33 +95,6 @@ enum : uint32_t { K_UPD = 1, K_OUT = 2, K_REST = 4, K_GHOST = 8 };
 // cell of slot 0 (0) or 1 (1) is a straight ghost of its N or S neighbour, or
 // feeds nothing (walls along x).  0S and 1N are ghosts of the pair's other cell.
 enum : uint32_t { G_0S = 1, G_1N = 2, G_0N = 4, G_1S = 8 };
-
-// One DPP move of a double (both halves); lanes of rows outside ROWS keep
-// `old`'s value.
-template <int CTRL, int ROWS = 0xf>
-__device__ __forceinline__ double dpp_move(double v, double old) {
-    const int lo = __builtin_amdgcn_update_dpp(__double2loint(old), __double2loint(v), CTRL,
-                                               ROWS, 0xf, false);
-    const int hi = __builtin_amdgcn_update_dpp(__double2hiint(old), __double2hiint(v), CTRL,
-                                               ROWS, 0xf, false);
-    return __hiloint2double(hi, lo);
-}
-
-// The sum of v over the wave, in VALU (DPP) steps rather than LDS round
-// trips, in a fixed order: pairs, quads, the quads of a row, then rows
-// (r0 + r1) and (r2 + r3), then (r2 + r3) + (r0 + r1).  Uniform result.
-__device__ __forceinline__ double wave_sum(double v) {
-    v = v + dpp_move<0xb1>(v, 0.0);          // quad_perm [1, 0, 3, 2]
-    v = v + dpp_move<0x4e>(v, 0.0);          // quad_perm [2, 3, 0, 1]
-    v = v + dpp_move<0x124>(v, 0.0);         // row_ror 4
-    v = v + dpp_move<0x128>(v, 0.0);         // row_ror 8
-    v = v + dpp_move<0x142, 0xa>(v, 0.0);    // row_bcast 15 into rows 1, 3
-    v = v + dpp_move<0x143, 0xc>(v, 0.0);    // row_bcast 31 into rows 2, 3
-    const int lo = __builtin_amdgcn_readlane(__double2loint(v), 63);
-    const int hi = __builtin_amdgcn_readlane(__double2hiint(v), 63);
-    return __hiloint2double(hi, lo);
-}
-
 
 // The workgroup's sum of v, in wave order, for thread 0 (the last use of
 // wsum in the kernel: no barrier after it).
@@ -614,7 +588,7 @@ k_rb_codes(const TbTile* __restrict__ tiles, const uint8_t* __restrict__ flags, 
 }
 
 // After a blocked solve: channels whose latest p is in the second buffer
-// copy it back.
+// copy it back (what arms the next one sets pbuf to 0).
 __global__ void __launch_bounds__(TILE_THREADS)
 k_pbuf_fix(const ChanDesc* __restrict__ cd, const ChanState* __restrict__ cs,
            const stm::Tile* __restrict__ tiles, const double* __restrict__ pb,
@@ -627,11 +601,6 @@ k_pbuf_fix(const ChanDesc* __restrict__ cd, const ChanState* __restrict__ cs,
     if (x >= d.nx || y >= d.ny) return;
     const int64_t i = d.off + x * (int64_t)d.pitch + y;
     pa[i] = pb[i];
-}
-
-__global__ void k_pbuf_reset(int nchan, ChanState* __restrict__ cs) {
-    const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c < nchan) cs[c].pbuf = 0;
 }
 
 // ---------------------------------------------------------------- variants
@@ -692,10 +661,9 @@ void launch_rb_codes(hipStream_t st, int variant, int ntb, const TbTile* tiles,
                                      waves, words);
 }
 
-void launch_pbuf_fix(hipStream_t st, int ntiles, int nchan, const ChanDesc* cd, ChanState* cs,
+void launch_pbuf_fix(hipStream_t st, int ntiles, const ChanDesc* cd, const ChanState* cs,
                      const stm::Tile* tiles, const double* pb, double* pa) {
     k_pbuf_fix<<<ntiles, dim3(TILE_Y, TILE_X), 0, st>>>(cd, cs, tiles, pb, pa);
-    k_pbuf_reset<<<(nchan + 63) / 64, 64, 0, st>>>(nchan, cs);
 }
 
 }  // namespace stm
