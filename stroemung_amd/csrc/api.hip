@@ -74,6 +74,7 @@ struct stm_ctx {
     bool any_rb = false, any_lex = false;
     double *u = nullptr, *v = nullptr, *p = nullptr, *f = nullptr, *g = nullptr, *rhs = nullptr;
     double* scratch = nullptr;
+    bool lex_few = false;          // see stage_lex
     double* lexwork = nullptr;     // pipelined lexicographic solve: its channels' scratch
     int64_t* d_lexoff = nullptr;   // ... and each channel's offset in it
     double* p2 = nullptr;          // second pressure buffer of the blocked solver
@@ -638,9 +639,11 @@ int nch(stm_ctx* ctx) { return (int)ctx->chans.size(); }
 
 // ------------------------------------------------------------- stages
 
-int stage_bc(stm_ctx* ctx) {
+// SETBCOND; at the start of a tick also the time steps
+int stage_bc(stm_ctx* ctx, bool tick = false) {
     LAUNCH("bc_velocity", launch_bc_velocity(ctx->stream, ctx->nbtot, ctx->d_be, ctx->d_restore,
-                                             ctx->u, ctx->v));
+                                             ctx->u, ctx->v, tick ? nch(ctx) : 0, ctx->d_cd,
+                                             ctx->d_cs));
     return STM_OK;
 }
 
@@ -1112,35 +1115,49 @@ int lex_buffers(stm_ctx* ctx) {
                                hipMemcpyHostToDevice, ctx->stream));
     HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
     HIPCHK(ctx, hipMalloc(&ctx->lexwork, sizeof(double) * (size_t)n));
-    return STM_OK;
+    launch_fill(ctx->stream, n, ctx->lexwork, 0.0);
+    for (int k = 0; k < N_LEX_CLASSES; k++)
+        launch_lex_init(ctx->stream, k, nch(ctx), ctx->d_cd, ctx->d_lexoff, ctx->lexwork);
+    return check_launch(ctx);
 }
 
-// The lexicographic channels: a launch per class in use.
+// The lexicographic channels: a launch per class in use.  The kernel in front of
+// them is launched if it has channels of its own or if, when the states were last
+// read, some channel's solve was one that it begins (it decides on the present
+// state; without it the pipelined solve takes them all).
 int stage_lex(stm_ctx* ctx) {
     int rc = lex_buffers(ctx);
     if (rc) return rc;
     std::vector<bool> used(N_LEX_CLASSES + 1, false);
     for (const HostChan& c : ctx->chans)
         if (c.prm.solver == STM_SOLVER_LEX) used[1 + lex_class((int)c.nx, (int)c.ny)] = true;
+    if (used[0] || ctx->lex_few)
+        LAUNCH("lex_solve", launch_lex_solve(ctx->stream, nch(ctx), ctx->d_cd, ctx->d_cs,
+                                             ctx->d_be, ctx->flags, ctx->rhs, ctx->p,
+                                             ctx->scratch));
     for (int k = 0; k < N_LEX_CLASSES; k++)
         if (used[1 + k])
             LAUNCH("lex_solve", launch_lex_pipe(ctx->stream, k, nch(ctx), ctx->d_cd, ctx->d_cs,
                                                 ctx->d_lexoff, ctx->flags, ctx->rhs, ctx->p,
                                                 ctx->lexwork));
-    if (used[0])
-        LAUNCH("lex_solve", launch_lex_solve(ctx->stream, nch(ctx), ctx->d_cd, ctx->d_cs,
-                                             ctx->d_be, ctx->flags, ctx->rhs, ctx->p,
-                                             ctx->scratch));
     return STM_OK;
 }
 
 // POISSON: the rhs statistics, tol2 and the per-channel flags, then each
 // channel's solver.
 int stage_solve(stm_ctx* ctx) {
-    int rc = stage_rhs_stats(ctx);
-    if (rc) return rc;
-    LAUNCH("solve_begin", launch_solve_begin(ctx->stream, nch(ctx), ctx->d_cd, ctx->d_cs,
-                                             ctx->d_part, ctx->d_active));
+    int rc;
+    bool small = true;   // every channel's statistics in one workgroup
+    for (const HostChan& c : ctx->chans) small = small && c.ntiles <= STATS_TILES;
+    if (small) {
+        LAUNCH("rhs_stats", launch_solve_stats(ctx->stream, nch(ctx), ctx->d_cd, ctx->d_cs,
+                                               ctx->d_tiles, ctx->flags, ctx->rhs,
+                                               ctx->d_active));
+    } else {
+        if ((rc = stage_rhs_stats(ctx))) return rc;
+        LAUNCH("solve_begin", launch_solve_begin(ctx->stream, nch(ctx), ctx->d_cd, ctx->d_cs,
+                                                 ctx->d_part, ctx->d_active));
+    }
     if (ctx->any_lex && (rc = stage_lex(ctx))) return rc;
     if (!ctx->any_rb) return STM_OK;
     if (ctx->cnet || (ctx->lnet && ctx->lcycles > 0)) return phased_solve(ctx);
@@ -1150,13 +1167,13 @@ int stage_solve(stm_ctx* ctx) {
 // ADAP_UV with the restore list (src/simulation.rs:287-322) and the ranges
 // that follow it: the restore list first (it sets every boundary cell), then
 // ADAP_UV of the fluid cells fused with the range reductions.
-int stage_adap(stm_ctx* ctx, int want_pressure) {
+int stage_adap(stm_ctx* ctx, int want_pressure, bool tick = false) {
     LAUNCH("restore", launch_restore(ctx->stream, ctx->nbtot, ctx->d_be, ctx->d_restore,
                                      ctx->u, ctx->v));
     LAUNCH("adap_ranges", launch_adap_ranges(ctx->stream, ctx->ntiles, nch(ctx), ctx->d_cd,
                                              ctx->d_cs, ctx->d_tiles, ctx->flags, ctx->f, ctx->g,
                                              ctx->p, ctx->u, ctx->v, ctx->d_part,
-                                             want_pressure));
+                                             want_pressure, tick ? 1 : 0));
     return STM_OK;
 }
 
@@ -1169,12 +1186,10 @@ int stage_ranges(stm_ctx* ctx, int want_pressure) {
 
 int tick(stm_ctx* ctx) {
     int rc;
-    LAUNCH("delt", launch_delt(ctx->stream, nch(ctx), ctx->d_cd, ctx->d_cs));
-    if ((rc = stage_bc(ctx))) return rc;
+    if ((rc = stage_bc(ctx, true))) return rc;
     if ((rc = stage_fg_rhs(ctx))) return rc;
     if ((rc = stage_solve(ctx))) return rc;
-    if ((rc = stage_adap(ctx, 2))) return rc;
-    LAUNCH("advance_time", launch_advance_time(ctx->stream, nch(ctx), ctx->d_cs));
+    if ((rc = stage_adap(ctx, 2, true))) return rc;
     return check_launch(ctx);
 }
 
@@ -1182,6 +1197,13 @@ int read_states(stm_ctx* ctx) {
     HIPCHK(ctx, hipMemcpyAsync(ctx->h_cs, ctx->d_cs, sizeof(ChanState) * nch(ctx),
                                hipMemcpyDeviceToHost, ctx->stream));
     HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
+    ctx->lex_few = false;
+    for (int k = 0; k < nch(ctx); k++) {
+        const HostChan& c = ctx->chans[k];
+        ctx->lex_few = ctx->lex_few || (c.prm.solver == STM_SOLVER_LEX &&
+                                        lex_few((int)(c.nx * c.ny), ctx->h_cs[k].sor_iters,
+                                                ctx->h_cs[k].exhausted));
+    }
     return check_launch(ctx);
 }
 

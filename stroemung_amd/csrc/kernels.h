@@ -8,7 +8,7 @@ namespace stm {
 
 // kernels_step.hip
 void launch_bc_velocity(hipStream_t, int nbtot, const BEntry*, double2* restore, double* u,
-                        double* v);
+                        double* v, int nchan, const ChanDesc*, ChanState*);
 void launch_fg(hipStream_t, int ntiles, const ChanDesc*, const ChanState*, const Tile*,
                const uint8_t* flags, const double* u, const double* v, double* f, double* g);
 void launch_rhs(hipStream_t, int ntiles, const ChanDesc*, const ChanState*, const Tile*,
@@ -26,9 +26,7 @@ void launch_ranges(hipStream_t, int ntiles, int nchan, const ChanDesc*, ChanStat
 void launch_adap_ranges(hipStream_t, int ntiles, int nchan, const ChanDesc*, ChanState*,
                         const Tile*, const uint8_t* flags, const double* f, const double* g,
                         const double* p, double* u, double* v, double* part,
-                        int want_pressure);
-void launch_delt(hipStream_t, int nchan, const ChanDesc*, ChanState*);
-void launch_advance_time(hipStream_t, int nchan, ChanState*);
+                        int want_pressure, int end_tick);
 void launch_fill(hipStream_t, int64_t n, double* a, double val);
 void launch_zero_cells(hipStream_t, int n, const int64_t* idx, double* u, double* v,
                        double* p);
@@ -49,10 +47,21 @@ void launch_ghost(hipStream_t, int nbtot, const BEntry*, const ChanState*, doubl
 // rhs_mean and the sum of (rhs - mean)^2 per channel (partials in slots 0, 1)
 void launch_rhs_stats(hipStream_t, int ntiles, int nchan, const ChanDesc*, ChanState*,
                       const Tile*, const uint8_t* flags, const double* rhs, double* part);
+// The same and launch_solve_begin in one launch, for channels of at most
+// STATS_TILES tiles each.
+constexpr int STATS_TILES = 256;
+void launch_solve_stats(hipStream_t, int nchan, const ChanDesc*, ChanState*, const Tile*,
+                        const uint8_t* flags, const double* rhs, int32_t* active);
 void launch_solve_begin(hipStream_t, int nchan, const ChanDesc*, ChanState*, const double* part,
                         int32_t* active);
 void launch_initial_norm(hipStream_t, int nchan, const ChanDesc*, ChanState*, const double* rhs,
                          const double* p, double* scratch);
+// Does launch_lex_solve begin the solve of a channel that the pipelined solve
+// takes too?  (cells, ring included; how its last solve ended)
+constexpr int LEX_LDS_CELLS = 4608;
+__host__ __device__ inline bool lex_few(int cells, uint32_t last_sweeps, int32_t exhausted) {
+    return cells <= LEX_LDS_CELLS && last_sweeps == 1 && !exhausted;
+}
 void launch_lex_solve(hipStream_t, int nchan, const ChanDesc*, ChanState*, const BEntry*,
                       const uint8_t* flags, const double* rhs, double* p, double* scratch);
 
@@ -66,6 +75,9 @@ extern const LexClass LEX_CLASSES[];
 extern const int N_LEX_CLASSES;
 int lex_class(int nx, int ny);
 int64_t lex_work_doubles(int cls, int nx, int ny);   // scratch of one channel
+// What the scratch of class `cls` holds where there is no cell (the rest zeroed before).
+void launch_lex_init(hipStream_t, int cls, int nchan, const ChanDesc*, const int64_t* work_off,
+                     double* work);
 // The channels of class `cls`; work_off: each channel's element offset in work.
 void launch_lex_pipe(hipStream_t, int cls, int nchan, const ChanDesc*, ChanState*,
                      const int64_t* work_off, const uint8_t* flags, const double* rhs, double* p,

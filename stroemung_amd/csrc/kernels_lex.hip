@@ -232,6 +232,13 @@ struct Pipe {
         return c | ((uint32_t)(dd * (int)ROWP + (y % RPL + dy) * 8) & (RINGB - 8));
     }
 
+    // Where the code of row y of a diagonal (a row of the codes) is.  (A lane of
+    // three rows leaves its fourth code unread.)
+    __device__ static __forceinline__ uint16_t* code_place(char* codes, uint32_t row, uint32_t y) {
+        return reinterpret_cast<uint16_t*>(codes) + row * (ROWC / 2) +
+               y / RPL * 2 * code_words(RPL) + y % RPL;
+    }
+
     // Groups of a sweep, and of a round: a slot starts its next sweep a round
     // after this one.  Slot 0's ring takes row q of C in step q of its round,
     // loaded a group earlier; the last slot stores row q in step 3 NSLOT + q of
@@ -546,6 +553,23 @@ int64_t lex_work_doubles(int cls, int nx, int ny) {
 
 constexpr int LIGHT_MOST = 256;   // sweeps of a LIGHT batch
 
+// Entries of the scratch that are no cell: code of a cell that is its own input
+// (the fields hold 0 from the allocation on).  Once, with the allocation.
+template <int CLASS, int LW, int RPL, int NSLOT, int TS>
+__global__ void __launch_bounds__(256)
+k_lex_init(const ChanDesc* __restrict__ cd, const int64_t* __restrict__ work_off,
+           double* __restrict__ work)
+{
+    using P = Pipe<LW, RPL, NSLOT, TS>;
+    const ChanDesc& d = cd[blockIdx.y];
+    if (d.lex_class != CLASS) return;
+    const uint32_t cells = (uint32_t)(d.nx + d.ny - 1 + 2 * LEX_PAD) * P::ROW;
+    char* codes = reinterpret_cast<char*>(work + work_off[blockIdx.y]) + (4 + TS) * (uint64_t)cells * 8;
+    for (uint32_t k = blockIdx.x * 256 + threadIdx.x; k < cells; k += gridDim.x * 256)
+        *P::code_place(codes, k / P::ROW, k % P::ROW) =
+            (uint16_t)P::code(make_flag(T_NOSLIP, E_NONE), (int)(k % P::ROW), false);
+}
+
 template <int CLASS, int LW, int RPL, int NSLOT, int TS>
 __global__ void __launch_bounds__(LW * NSLOT)
 k_lex_pipe(const ChanDesc* __restrict__ cd, ChanState* __restrict__ cs,
@@ -559,6 +583,8 @@ k_lex_pipe(const ChanDesc* __restrict__ cd, ChanState* __restrict__ cs,
     const ChanDesc d = cd[blockIdx.x];
     if (d.solver != SOLVER_LEX || d.lex_class != CLASS) return;
     ChanState& s = cs[blockIdx.x];
+    const int begun = s.budget;    // sweeps that k_lex_solve has done
+    if (begun < 0) return;         // it has ended the solve
     const int tid = threadIdx.x;
     const int nxi = d.nx - 2, nyi = d.ny - 2;
     LexWork w;
@@ -578,28 +604,26 @@ k_lex_pipe(const ChanDesc* __restrict__ cd, ChanState* __restrict__ cs,
     w.t = 4 * w.bytes;
     w.codes = (4 + TS) * w.bytes;
 
-    // the fields, diagonal-major; entries that are no cell hold 0 and code 0
+    // the fields, diagonal-major, cell by cell (entries that are no cell keep what
+    // k_lex_init gave them: 0, and the code of a cell that is its own input; a
+    // sweep stores there what it read).  All entries, a parallelogram of which a
+    // 152 x 152 channel fills a quarter, took 92 us to set of 403 for a solve of
+    // one sweep; its cells take 49 of 360.
     bool odd = !divisible(d.delx2) || !divisible(d.dely2) ||
                !(d.omega >= 0x1p-10 && d.omega <= 0x1p10);
-    // (every load from a clamped place: a batch of them is in flight at once)
+    const uint32_t ny = (uint32_t)d.ny, ncell = (uint32_t)d.nx * ny;
 #pragma unroll 8
-    for (uint32_t k = tid; k < cells; k += NT) {
-        const int row = (int)(k / ROW), y = (int)(k % ROW), x = row - LEX_PAD - y;
-        const bool in = x >= 0 && x < d.nx && y < d.ny;
-        const int64_t g = d.off + min(max(x, 0), d.nx - 1) * (int64_t)d.pitch + min(y, d.ny - 1);
-        const double pg = p[g], rg = rhs[g];
-        const uint8_t fg = flags[g];
-        const double pv = in ? pg : 0.0, rv = in ? rg : 0.0;
-        const uint8_t f = in ? fg : make_flag(T_NOSLIP, E_NONE);
+    for (uint32_t k0 = tid; k0 < ncell; k0 += NT) {
+        const uint32_t x = k0 / ny, y = k0 - x * ny, row = x + y + LEX_PAD;
+        const int64_t g = d.off + x * (int64_t)d.pitch + y;
+        const double pv = p[g], rv = rhs[g];
+        const uint8_t f = flags[g];
+        const uint32_t k = row * ROW + y;
         double* e = reinterpret_cast<double*>(w.base) + k;
         e[0] = pv;
-        e[cells] = 0.0;
-        e[2 * (int64_t)cells] = 0.0;
         e[3 * (int64_t)cells] = rv;
-        // (a lane of three rows leaves its fourth code unread)
-        reinterpret_cast<uint16_t*>(w.base + w.codes)[row * (P::ROWC / 2) + y / RPL * 2 * code_words(RPL) +
-                                                      y % RPL] =
-            (uint16_t)P::code(f, y, x >= 1 && x <= nxi && y >= 1 && y <= nyi);
+        *P::code_place(w.base + w.codes, row, y) =
+            (uint16_t)P::code(f, (int)y, x >= 1 && (int)x <= nxi && y >= 1 && (int)y <= nyi);
         odd |= tiny(pv) | !finite(pv) | tiny(rv);
     }
     __syncthreads();
@@ -610,8 +634,8 @@ k_lex_pipe(const ChanDesc* __restrict__ cd, ChanState* __restrict__ cs,
     // (the factor covers the roundings of this product and of the norm's division)
     const double bound = (init > d.eps2 ? init : d.eps2) * fluid * (1.0 + 0x1p-48);
     double norm2 = 0.0;
-    int iters = d.itermax, exhausted = 1, done = 0;
-    const int before = (int)min(s.sor_iters, (uint32_t)LIGHT_MOST);
+    int iters = d.itermax, exhausted = 1, done = begun;
+    const int before = begun > 0 ? 0 : (int)min(s.sor_iters, (uint32_t)LIGHT_MOST);
     bool light = before == 0 || s.exhausted;
     int len = before > 0 ? before : NSLOT;
     int replay = 0;   // sweeps of the batch to be repeated, ending with the one that met the rule
@@ -699,6 +723,16 @@ const LexClass LEX_CLASSES[] = {STM_LEX_CLASSES(L_ENTRY)};
 #undef L_ENTRY
 const int N_LEX_CLASSES = sizeof(LEX_CLASSES) / sizeof(LEX_CLASSES[0]);
 
+void launch_lex_init(hipStream_t st, int cls, int nchan, const ChanDesc* cd,
+                     const int64_t* work_off, double* work) {
+#define L_CASE(c, LW, RPL, NSLOT, TS)                                                          \
+    case c: k_lex_init<c, LW, RPL, NSLOT, TS><<<dim3(16, nchan), 256, 0, st>>>(cd, work_off, work); break;
+    switch (cls) {
+        STM_LEX_CLASSES(L_CASE)
+    default: break;
+    }
+#undef L_CASE
+}
 void launch_lex_pipe(hipStream_t st, int cls, int nchan, const ChanDesc* cd, ChanState* cs,
                      const int64_t* work_off, const uint8_t* flags, const double* rhs, double* p,
                      double* work) {

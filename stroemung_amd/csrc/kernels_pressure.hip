@@ -105,8 +105,24 @@ k_rhs_mean(const ChanDesc* __restrict__ cd, ChanState* __restrict__ cs,
     if (threadIdx.x == 0) cs[blockIdx.x].rhs_mean = d.n_inner > 0.0 ? sum / d.n_inner : 0.0;
 }
 
-// Start of a red-black solve: tol2 = eps^2 * sum((rhs - mean)^2) over
-// interior fluid cells.
+// Start of a solve: tol2 = eps^2 * sum((rhs - mean)^2) over interior fluid
+// cells, and what runs.
+__device__ __forceinline__ void begin_solve(const ChanDesc& d, ChanState& s, double rsum2,
+                                            int32_t* active_out) {
+    const bool rb = d.solver == SOLVER_RB;
+    s.rhs2 = rsum2;
+    s.tol2 = d.eps2 * rsum2;
+    if (rb) {   // (a lexicographic solve looks at how its last one ended)
+        s.sor_iters = 0;
+        s.exhausted = 0;
+    }
+    s.active = (rb && d.itermax > 0) ? 1 : 0;
+    s.stop_launch = s.active ? -1 : 0;
+    s.pbuf = 0;
+    s.budget = 0;
+    *active_out = s.active;
+}
+
 __global__ void __launch_bounds__(256)
 k_solve_begin(const ChanDesc* __restrict__ cd, ChanState* __restrict__ cs,
               const double* __restrict__ part, int32_t* __restrict__ active_out)
@@ -114,20 +130,57 @@ k_solve_begin(const ChanDesc* __restrict__ cd, ChanState* __restrict__ cs,
     __shared__ double sh[256];
     const ChanDesc& d = cd[blockIdx.x];
     const double rsum2 = chan_sum(d, part, 1, sh);
-    if (threadIdx.x == 0) {
-        ChanState& s = cs[blockIdx.x];
-        const bool rb = d.solver == SOLVER_RB;
-        s.rhs2 = rsum2;
-        s.tol2 = d.eps2 * rsum2;
-        if (rb) {   // (a lexicographic solve looks at how its last one ended)
-            s.sor_iters = 0;
-            s.exhausted = 0;
+    if (threadIdx.x == 0) begin_solve(d, cs[blockIdx.x], rsum2, active_out + blockIdx.x);
+}
+
+// The sum of v over a wave as the tree of offsets 32, 16, .. 1 gives it (lane 0).
+__device__ __forceinline__ double wave_tree(double v) {
+    for (int off = 32; off > 0; off >>= 1) v = v + __shfl_down(v, off, 64);
+    return v;
+}
+
+// k_rhs_sums, k_rhs_mean, k_rhs_sums and k_solve_begin of one channel in one
+// workgroup, in the same order: a wave sums a tile, a lane taking its column's
+// four cells as the first two steps of the tile's tree pair them, and the first
+// wave folds the tiles likewise.  For small channels, whose four launches took
+// 12 us of kernels and the gaps between them (a one-sweep solve of 102 x 22 cells:
+// 102 us with them, 92 so).
+__global__ void __launch_bounds__(1024)
+k_solve_stats(const ChanDesc* __restrict__ cd, ChanState* __restrict__ cs,
+              const Tile* __restrict__ tiles, const uint8_t* __restrict__ flags,
+              const double* __restrict__ rhs, int32_t* __restrict__ active_out)
+{
+    static_assert(TILE_X == 4 && TILE_Y == 64, "a lane's four cells");
+    __shared__ double part[STATS_TILES], total;
+    const ChanDesc& d = cd[blockIdx.x];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    double mean = 0.0;
+    for (int pass = 0; pass < 2; pass++) {
+        for (int k = wave; k < d.ntiles; k += 16) {
+            const Tile t = tiles[d.tile0 + k];
+            const int y = t.y0 + lane;
+            double v[TILE_X];
+#pragma unroll
+            for (int r = 0; r < TILE_X; r++) {
+                const int x = t.x0 + r;
+                const bool in = x >= 1 && x <= d.nx - 2 && y >= 1 && y <= d.ny - 2;
+                const int64_t i = d.off + (in ? x * (int64_t)d.pitch + y : 0);
+                const double a = rhs[i] - mean;   // (pass 0: the value itself)
+                v[r] = in && flag_fluid(flags[i]) ? (pass ? a * a : rhs[i]) : 0.0;
+            }
+            const double s = wave_tree((v[0] + v[2]) + (v[1] + v[3]));
+            if (lane == 0) part[k] = s;
         }
-        s.active = (rb && d.itermax > 0) ? 1 : 0;
-        s.stop_launch = s.active ? -1 : 0;
-        s.pbuf = 0;
-        s.budget = 0;
-        active_out[blockIdx.x] = s.active;
+        __syncthreads();
+        if (wave == 0) {
+            auto at = [&](int k) { return k < d.ntiles ? 0.0 + part[k] : 0.0; };
+            const double s = wave_tree((at(lane) + at(lane + 128)) + (at(lane + 64) + at(lane + 192)));
+            if (lane == 0) total = s;
+        }
+        __syncthreads();
+        if (pass == 0) mean = d.n_inner > 0.0 ? total / d.n_inner : 0.0;
+        else if (threadIdx.x == 0) begin_solve(d, cs[blockIdx.x], total, active_out + blockIdx.x);
+        if (pass == 0 && threadIdx.x == 0) cs[blockIdx.x].rhs_mean = mean;
     }
 }
 
@@ -327,12 +380,16 @@ __device__ __forceinline__ double lex_update(const ChanDesc& d, double pc, doubl
     return (d.omw * pc) + (d.mid * ((((pxp + pxm) / d.delx2) + ((pyp + pym) / d.dely2)) - r));
 }
 
-// Channels of at most this many cells (ring included) solve with p, rhs, the
+// Channels of at most LEX_LDS_CELLS cells (ring included) solve with p, rhs, the
 // flags and the norm's terms in LDS (115 KB).
-constexpr int LEX_LDS_CELLS = 4608;
+constexpr int LEX_FEW = 2;
 
 // src/simulation.rs:239-285 for the channels with solver == SOLVER_LEX that no
-// instance of the pipelined solve takes (kernels_lex.hip: more than 512 rows).
+// instance of the pipelined solve takes (kernels_lex.hip: more than 512 rows), and
+// the first LEX_FEW sweeps of channels in LDS whose last solve took one: the
+// pipeline's set-up (its diagonal-major copies) and its longer step pay from the
+// second or third sweep on.  A solve (statistics included) of 102 x 22 cells in
+// one sweep: 73 us here, 87 there; in two 113 and 88, in four 196 and 90.
 // Lexicographic Gauss-Seidel order (x outer, y inner, in place) makes cell
 // (x, y) read the new W and N values and the old E and S values; sweeping the
 // anti-diagonals x + y = const in increasing order, with a barrier between
@@ -353,8 +410,11 @@ k_lex_solve(const ChanDesc* __restrict__ cd, ChanState* __restrict__ cs,
     __shared__ double sp[LEX_LDS_CELLS], srhs[LEX_LDS_CELLS], ssq[LEX_LDS_CELLS];
     __shared__ uint8_t sfl[LEX_LDS_CELLS];
     const ChanDesc d = cd[blockIdx.x];
-    if (d.solver != SOLVER_LEX || d.lex_class >= 0) return;
+    if (d.solver != SOLVER_LEX) return;
     ChanState& s = cs[blockIdx.x];
+    const bool few = d.lex_class >= 0;
+    if (few && !lex_few(d.nx * d.ny, s.sor_iters, s.exhausted)) return;
+    const int limit = few ? min(d.itermax, LEX_FEW) : d.itermax;
     const int nxi = d.nx - 2, nyi = d.ny - 2;
     const int64_t P = d.pitch;
     const double init = s.init_norm2;
@@ -371,7 +431,7 @@ k_lex_solve(const ChanDesc* __restrict__ cd, ChanState* __restrict__ cs,
             sfl[l] = flags[g];
         }
         __syncthreads();
-        for (int it = 0; it < d.itermax; it++) {
+        for (int it = 0; it < limit; it++) {
             // copy_pressure_to_boundaries, src/grid/mod.rs:343-412
             for (int k = tid; k < d.nb; k += blockDim.x) {
                 const BEntry e = be[d.boff + k];
@@ -425,7 +485,12 @@ k_lex_solve(const ChanDesc* __restrict__ cd, ChanState* __restrict__ cs,
             const int x = l / ny, y = l - (l / ny) * ny;
             p[d.off + x * P + y] = sp[l];
         }
+        if (few && exhausted && limit < d.itermax) {   // the pipeline goes on from here
+            if (tid == 0) s.budget = limit;
+            return;
+        }
         if (tid == 0) {
+            s.budget = -1;
             s.sor_iters = (uint32_t)iters;
             s.norm2 = norm2;
             s.exhausted = exhausted;
@@ -484,6 +549,11 @@ void launch_rhs_stats(hipStream_t st, int ntiles, int nchan, const ChanDesc* cd,
     k_rhs_sums<<<ntiles, dim3(TILE_Y, TILE_X), 0, st>>>(cd, cs, tiles, flags, rhs, part, 0);
     k_rhs_mean<<<nchan, 256, 0, st>>>(cd, cs, part);
     k_rhs_sums<<<ntiles, dim3(TILE_Y, TILE_X), 0, st>>>(cd, cs, tiles, flags, rhs, part, 1);
+}
+void launch_solve_stats(hipStream_t st, int nchan, const ChanDesc* cd, ChanState* cs,
+                        const Tile* tiles, const uint8_t* flags, const double* rhs,
+                        int32_t* active) {
+    k_solve_stats<<<nchan, 1024, 0, st>>>(cd, cs, tiles, flags, rhs, active);
 }
 void launch_solve_begin(hipStream_t st, int nchan, const ChanDesc* cd, ChanState* cs,
                         const double* part, int32_t* active) {

@@ -24,6 +24,16 @@ __device__ __forceinline__ double reflect(bool moving, double b, double fluid) {
     return moving ? (2.0 * b) - fluid : -fluid;
 }
 
+// Adaptive time step (Griebel, Dornseifer, Neunhoeffer: NaSt2D COMP_DELT):
+// delt = tau * min(Re/2 / (1/dx^2 + 1/dy^2), dx/|u|max, dy/|v|max).
+__device__ __forceinline__ void set_delt(const ChanDesc& d, ChanState& s) {
+    if (!(d.tau > 0.0)) return;
+    double dt = (d.reynolds / 2.0) / ((1.0 / sq(d.delx)) + (1.0 / sq(d.dely)));
+    if (s.umax > 0.0) { const double t = d.delx / s.umax; if (t < dt) dt = t; }
+    if (s.vmax > 0.0) { const double t = d.dely / s.vmax; if (t < dt) dt = t; }
+    s.delt = d.tau * dt;
+}
+
 // ---------------------------------------------------------------- SETBCOND
 //
 // src/grid/mod.rs:414-651.  The reference walks the (x, y)-sorted boundary
@@ -36,11 +46,15 @@ __device__ __forceinline__ double reflect(bool moving, double b, double fluid) {
 // constant for v[W]); phase 2, after a barrier, stores the fluid-face
 // constants.  Each phase is a kernel over every boundary cell of every
 // channel (one thread per cell); the kernel boundary is the barrier.
+// At the start of a tick (nchan > 0) the first also sets the channels' time
+// steps, which it does not use: a launch of its own took 2.9 us of a tick.
 __global__ void __launch_bounds__(256)
 k_bc_cells(int nbtot, const BEntry* __restrict__ be, double2* __restrict__ restore,
-           double* __restrict__ u, double* __restrict__ v)
+           double* __restrict__ u, double* __restrict__ v, int nchan,
+           const ChanDesc* __restrict__ cd, ChanState* __restrict__ cs)
 {
     const int k = blockIdx.x * blockDim.x + threadIdx.x;
+    if (k < nchan) set_delt(cd[k], cs[k]);
     if (k < nbtot) {
         const BEntry e = be[k];
         const int64_t i = e.gidx, P = e.pitch;
@@ -439,10 +453,11 @@ k_adap_ranges(const ChanDesc* __restrict__ cd, const ChanState* __restrict__ cs,
 // One workgroup per channel: fold the range partials of its tiles (min and
 // max are order-free, so the result is exact).
 // want_pressure: 1 = always (construction), 2 = only if the solve hit
-// itermax (src/simulation.rs:283), 0 = never.
+// itermax (src/simulation.rs:283), 0 = never.  end_tick: the last stage of a
+// tick, which also advances the time (src/simulation.rs:330-331).
 __global__ void __launch_bounds__(256)
 k_ranges_reduce(const ChanDesc* __restrict__ cd, ChanState* __restrict__ cs,
-                const double* __restrict__ part, int want_pressure)
+                const double* __restrict__ part, int want_pressure, int end_tick)
 {
     __shared__ double sh[6][256];
     const int c = blockIdx.x, tid = threadIdx.x;
@@ -482,30 +497,10 @@ k_ranges_reduce(const ChanDesc* __restrict__ cd, ChanState* __restrict__ cs,
         s.pressure_range[0] = pmin;
         s.pressure_range[1] = pmax;
     }
-}
-
-// Adaptive time step (Griebel, Dornseifer, Neunhoeffer: NaSt2D COMP_DELT):
-// delt = tau * min(Re/2 / (1/dx^2 + 1/dy^2), dx/|u|max, dy/|v|max).
-__global__ void k_delt(int nchan, const ChanDesc* __restrict__ cd, ChanState* __restrict__ cs)
-{
-    const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= nchan) return;
-    const ChanDesc& d = cd[c];
-    if (!(d.tau > 0.0)) return;
-    ChanState& s = cs[c];
-    double dt = (d.reynolds / 2.0) / ((1.0 / sq(d.delx)) + (1.0 / sq(d.dely)));
-    if (s.umax > 0.0) { const double t = d.delx / s.umax; if (t < dt) dt = t; }
-    if (s.vmax > 0.0) { const double t = d.dely / s.vmax; if (t < dt) dt = t; }
-    s.delt = d.tau * dt;
-}
-
-// src/simulation.rs:330-331
-__global__ void k_advance_time(int nchan, ChanState* __restrict__ cs)
-{
-    const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= nchan) return;
-    cs[c].time = cs[c].time + cs[c].delt;
-    cs[c].iterations += 1;
+    if (end_tick) {
+        s.time = s.time + s.delt;
+        s.iterations += 1;
+    }
 }
 
 // Plain streaming copy (16 B per lane per step): the bandwidth probe and the
@@ -570,10 +565,10 @@ k_fill(int64_t n, double* __restrict__ a, double val)
 #define TB dim3(TILE_Y, TILE_X)
 
 void launch_bc_velocity(hipStream_t st, int nbtot, const BEntry* be, double2* restore, double* u,
-                        double* v) {
-    if (nbtot <= 0) return;
-    k_bc_cells<<<(nbtot + 255) / 256, 256, 0, st>>>(nbtot, be, restore, u, v);
-    k_bc_faces<<<(nbtot + 255) / 256, 256, 0, st>>>(nbtot, be, u, v);
+                        double* v, int nchan, const ChanDesc* cd, ChanState* cs) {
+    const int n = std::max(nbtot, nchan);
+    if (n > 0) k_bc_cells<<<(n + 255) / 256, 256, 0, st>>>(nbtot, be, restore, u, v, nchan, cd, cs);
+    if (nbtot > 0) k_bc_faces<<<(nbtot + 255) / 256, 256, 0, st>>>(nbtot, be, u, v);
 }
 void launch_fg(hipStream_t st, int ntiles, const ChanDesc* cd, const ChanState* cs,
                const Tile* tiles, const uint8_t* flags, const double* u, const double* v,
@@ -597,20 +592,14 @@ void launch_ranges(hipStream_t st, int ntiles, int nchan, const ChanDesc* cd, Ch
                    const Tile* tiles, const uint8_t* flags, const double* u, const double* v,
                    const double* p, double* part, int want_pressure) {
     k_ranges<<<ntiles, TB, 0, st>>>(cd, tiles, flags, u, v, p, part);
-    k_ranges_reduce<<<nchan, 256, 0, st>>>(cd, cs, part, want_pressure);
+    k_ranges_reduce<<<nchan, 256, 0, st>>>(cd, cs, part, want_pressure, 0);
 }
 void launch_adap_ranges(hipStream_t st, int ntiles, int nchan, const ChanDesc* cd, ChanState* cs,
                         const Tile* tiles, const uint8_t* flags, const double* f,
                         const double* g, const double* p, double* u, double* v, double* part,
-                        int want_pressure) {
+                        int want_pressure, int end_tick) {
     k_adap_ranges<<<ntiles, TB, 0, st>>>(cd, cs, tiles, flags, f, g, p, u, v, part);
-    k_ranges_reduce<<<nchan, 256, 0, st>>>(cd, cs, part, want_pressure);
-}
-void launch_delt(hipStream_t st, int nchan, const ChanDesc* cd, ChanState* cs) {
-    k_delt<<<(nchan + 63) / 64, 64, 0, st>>>(nchan, cd, cs);
-}
-void launch_advance_time(hipStream_t st, int nchan, ChanState* cs) {
-    k_advance_time<<<(nchan + 63) / 64, 64, 0, st>>>(nchan, cs);
+    k_ranges_reduce<<<nchan, 256, 0, st>>>(cd, cs, part, want_pressure, end_tick);
 }
 void launch_zero_cells(hipStream_t st, int n, const int64_t* idx, double* u, double* v,
                        double* p) {

@@ -216,3 +216,41 @@ def test_a_batch_of_every_instance():
         ct, vel = mixed_grid(70 + k, nx, ny)
         grids.append((ct, vel, random_fields(k, ct.shape), dict(KW, max_iterations=10 + 3 * k)))
     _solve_both(grids)
+
+
+@pytest.mark.parametrize("nx,ny", [(3, 3), (102, 22), (96, 48), (97, 48), (15, 300), (9, 512)])
+def test_a_solve_after_one_of_a_single_sweep(nx, ny):
+    """The kernel that begins the solve of a channel in LDS after a solve of one
+    sweep: the next one ends in it (one or two sweeps, or itermax), or goes on
+    elsewhere (three and more), at 4608 cells and just beyond, alone and beside a
+    channel whose last solve was long."""
+    ct, vel = mixed_grid(5, nx, ny) if min(nx, ny) > 8 else presets.lid_cavity(nx - 2, ny - 2)
+    f = random_fields(11, ct.shape)
+    fields = dict(zip(("u", "v", "p", "f", "g", "rhs"), f))
+    always = dict(KW, initial_norm_squared=1e300)
+    norms = [_sim(ct, vel, f, **dict(KW, max_iterations=j)).solve()[1] for j in range(1, 8)]
+    cases = [dict(KW, initial_norm_squared=float(np.nextafter(norms[j], np.inf)))
+             for j in (0, 1, 2, 6)]
+    cases += [dict(KW, max_iterations=m) for m in (1, 2, 3, 37)]
+    other = mixed_grid(6, 50, 40)
+    of = random_fields(12, other[0].shape)
+    for kw in cases:
+        ctx = Context(0)
+        ctx.add_grid(_params(always), ct, vel)
+        ctx.add_grid(_params(KW), *other)
+        for rep in range(2):
+            ctx.upload(0, **fields)
+            ctx.upload(1, **dict(zip(("u", "v", "p", "f", "g", "rhs"), of)))
+            ctx.stage("solve_pressure")
+            if rep == 0:
+                assert ctx.state(0)["sor_iterations"] == 1
+                ctx.set_params(0, _params(kw))
+        s = _sim(ct, vel, f, **kw)
+        it, n2 = s.solve()
+        st = ctx.state(0)
+        assert (st["sor_iterations"], st["norm_squared"]) == (it, n2), kw
+        assert_bits_equal(ctx.download(0)["p"], s.p, "p of %s" % (ct.shape,))
+        o = _sim(*other, of, **KW)
+        assert (ctx.state(1)["sor_iterations"], ctx.state(1)["norm_squared"]) == o.solve()
+        assert_bits_equal(ctx.download(1)["p"], o.p, "the other channel's p")
+        ctx.close()
