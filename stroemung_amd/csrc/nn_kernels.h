@@ -50,15 +50,41 @@ struct FlipList {
     unsigned block[16];   // first workgroup of each layer (filled by weight_flip)
 };
 void weight_flip(hipStream_t, FlipList& layers, const bf16* w, bf16* wt);
-// The gradient and loss reductions leave per-block partial sums in `part`
-// (device scratch, reused launch after launch on one stream) and add them in
-// a fixed order, so a gradient is the same from run to run.  Sizes in floats:
-// grad_partials and loss_partials (nn_sizes.h).
-// Through a ReLU and a convolution's parameters: g = g * (y > 0);
-// db[c] += sum_pix g[pix][c]; dw32[co][tap][ci] += sum_pix g[pix][co] * in[pix + off(tap)][ci]
-// (bpart: the bias' partials, bias_partials floats).
-void conv_grads(hipStream_t, const bf16* y, bf16* g, int cout, const bf16* in, int cin,
-                float* dw32, float* db, int nb, int H, int W, float* part, float* bpart);
+// The gradient and loss reductions leave per-block partial sums (device scratch)
+// that are added in a fixed order, so a gradient is the same from run to run.
+// Sizes in floats: dw_partials, bias_partials and loss_partials (nn_sizes.h).
+// Through a ReLU, g = g * (y > 0), and the partials of db[c] = sum_pix g[pix][c].
+void relu_bias_bwd(hipStream_t, const bf16* y, bf16* g, int c, int64_t npix, float* bpart);
+// The partials of dw32[co][tap][ci] = sum_pix gz[pix][co] * in[pix + off(tap)][ci] of
+// every layer, at part + poff (added to grads + woff at once if the pixels are
+// one chunk).  All layers together: the deep ones alone leave the chip idle.
+struct DwLayer {
+    const bf16 *gz, *in;
+    int cout, cin, nb, H, W;
+    int64_t woff, poff;
+    // filled by conv3x3_dw
+    float* out;
+    int64_t chunk_stride;
+    int per, ci_first, ntile_ci;
+};
+struct DwList {
+    int n = 0;
+    unsigned block[16];
+    DwLayer layer[16];
+};
+void conv3x3_dw(hipStream_t, const DwLayer* layers, int n, float* grads, float* part);
+// Then the partials of every layer into its gradients (added to grads), in one
+// launch: layer k's weights at woff[k], its bias at boff[k]; its partials at
+// part + poff[k] and bpart + bpoff[k], of npix[k] pixels.
+struct GradList {
+    int n = 0;
+    int cin[16], cout[16];
+    int64_t npix[16], woff[16], boff[16], poff[16], bpoff[16];
+    int chunks[16], bblocks[16];   // (filled by grad_finish)
+    unsigned block[16];
+};
+void grad_finish(hipStream_t, GradList& layers, const float* part, const float* bpart,
+                 float* grads);
 void maxpool(hipStream_t, const bf16* x, bf16* y, int nb, int H, int W, int c,
              const int* live = nullptr);
 // accumulates into gx

@@ -521,18 +521,28 @@ k_conv_finish(const float* __restrict__ acc32, int ks, const float* __restrict__
 
 // w'[ci][8 - tap][co] = w[co][tap][ci] for every layer of the list, each at the
 // offset of its own weights: one launch in front of the backward pass (3.7 us
-// for each layer by itself before, 12.6 for all now)
+// for each layer by itself before, 6.5 for all now)
 __global__ void __launch_bounds__(256)
 k_weight_flip(FlipList l, const bf16* __restrict__ w, bf16* __restrict__ wt)
 {
+    // a block turns 32 co x 32 ci of one tap in LDS, so that reads and stores both
+    // run along the channels
+    __shared__ bf16 tile[32][33];
     int k = 0;
     while (k + 1 < l.n && blockIdx.x >= l.block[k + 1]) k++;
     const int cin = l.cin[k], cout = l.cout[k];
-    // consecutive threads take consecutive co: the stores are contiguous
-    const int i = (blockIdx.x - l.block[k]) * 256 + threadIdx.x;
-    if (i >= cin * 9 * cout) return;
-    const int co = i % cout, t = i / cout, tap = t % 9, ci = t / 9;
-    wt[l.off[k] + i] = w[l.off[k] + ((int64_t)co * 9 + 8 - tap) * cin + ci];
+    const int b = blockIdx.x - l.block[k], tap = b % 9, ci0 = b / 9 % (cin / 32) * 32,
+              co0 = b / 9 / (cin / 32) * 32;
+    const int lane = threadIdx.x & 31, row = threadIdx.x >> 5;   // eight rows at a time
+    const bf16* from = w + l.off[k];
+    bf16* to = wt + l.off[k];
+#pragma unroll
+    for (int r = row; r < 32; r += 8)
+        tile[r][lane] = from[((int64_t)(co0 + r) * 9 + 8 - tap) * cin + ci0 + lane];
+    __syncthreads();
+#pragma unroll
+    for (int r = row; r < 32; r += 8)
+        to[((int64_t)(ci0 + r) * 9 + tap) * cout + co0 + lane] = tile[lane][r];
 }
 
 // dw[co][tap][ci] over a pixel chunk: sum of gz[pix][co] * in[pix+off][ci].
@@ -542,26 +552,41 @@ k_weight_flip(FlipList l, const bf16* __restrict__ w, bf16* __restrict__ wt)
 // 130 pixels that the three dx reach, whatever the width), and
 // ds_read_b64_tr_b16 hands lane c of 16 the channel c of four pixels; a lane
 // whose pixel has no neighbour there reads a row of zeros instead.  The next
-// 128 pixels are loaded while these are multiplied.  Transposing with 2-byte
-// LDS stores, for each tap by itself, was what bounded the pass before: 29.7 us
-// on average over the 14 layers of 32 frames of 64 x 64, 16.0
-// now.  What bounds a round is the transposed reads (16 for 12 MFMAs): eight
-// waves with 32 x 16 pieces, loads two and three rounds ahead and a pixel padded
-// to 160 bytes measured 15.7 to 16.6.
+// 128 pixels are loaded while these are multiplied.  Transposing with 2-byte LDS
+// stores, for each tap by itself, was what bounded the pass before.  What bounds
+// a round is the transposed reads (16 for 12 MFMAs): eight waves with 32 x 16
+// pieces, loads two and three rounds ahead and a pixel padded to 160 bytes
+// measured no faster (16.0 us for a layer on average, 15.7 to 16.6 those).  The
+// layers of a network run together, a launch for each kind of tile: by themselves
+// most are a few dozen workgroups.  All 14 layers of 32 frames of 64 x 64: 416 us
+// with the stores, 224 layer by layer, 135 in four launches.
 //
 // The four waves cover the tile in 32 x 32 pieces and split the four 32-pixel
 // k steps among themselves when the tile is narrower than 64 x 64, so no wave
 // multiplies padding; those waves then add their sums in LDS in wave order.
 // With one pixel chunk (chunk_stride 0) the block adds its sums into dw; with
 // several, chunk z writes its own slice out[z * chunk_stride + ...] and
-// k_chunk_sum adds the slices in chunk order, so the result does not depend
+// k_grad_finish adds the slices in chunk order, so the result does not depend
 // on the order in which blocks finish.
 template <int CO, int CI>   // the tile: 32 or 64 of each
 __global__ void __launch_bounds__(256)
-k_conv3x3_dw(const bf16* __restrict__ gz, int cout, const bf16* __restrict__ in, int cin,
-             int ci_first, float* __restrict__ out, int64_t chunk_stride, int nb, int H, int W,
-             int pix_per_block)
+k_conv3x3_dw(DwList l)
 {
+    int q = 0;
+    while (q + 1 < l.n && blockIdx.x >= l.block[q + 1]) q++;
+    const DwLayer& a = l.layer[q];
+    const bf16* __restrict__ gz = a.gz;
+    const bf16* __restrict__ in = a.in;
+    float* __restrict__ out = a.out;
+    const int cout = a.cout, cin = a.cin, H = a.H, W = a.W, npix = a.nb * a.H * a.W;
+    // workgroups of a layer: input tile, output tile, dy, chunk
+    int at_block = blockIdx.x - l.block[q];
+    const int ti = at_block % a.ntile_ci;
+    at_block /= a.ntile_ci;
+    const int to = at_block % (cout / CO);
+    at_block /= cout / CO;
+    const int dy = at_block % 3 - 1, chunk = at_block / 3;
+    const int64_t chunk_stride = a.chunk_stride;
     // KP pixels at once; a staged pixel takes LS channels (144 bytes: the 16
     // rows of a read then cover the banks evenly)
     constexpr int KP = 128, WP = KP + 2, LS = 72;
@@ -573,12 +598,10 @@ k_conv3x3_dw(const bf16* __restrict__ gz, int cout, const bf16* __restrict__ in,
     bf16* sg = smem;               // [pixel][co]
     bf16* si = smem + KP * LS;     // [pixel + dx + 1][ci], then a row of zeros
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int dy = (int)(blockIdx.z % 3) - 1;
-    const int co0 = blockIdx.y * CO;
-    const int ci0 = ci_first + blockIdx.x * CI;
-    const int npix = nb * H * W;
-    const int p_begin = (blockIdx.z / 3) * pix_per_block;
-    const int p_end = min(npix, p_begin + pix_per_block);
+    const int co0 = to * CO;
+    const int ci0 = a.ci_first + ti * CI;
+    const int p_begin = chunk * a.per;
+    const int p_end = min(npix, p_begin + a.per);
     const int mo = wave % WO, ni = wave / WO % WI, kg = wave / (WO * WI);
     f32x4 acc[3][2][2];
     for (int x = 0; x < 3; x++)
@@ -694,7 +717,7 @@ k_conv3x3_dw(const bf16* __restrict__ gz, int cout, const bf16* __restrict__ in,
     }
     // the wave's piece: lane l % 16 is a ci, so each store writes four runs of 64 bytes
     const int cr = co0 + mo * 32 + (lane >> 4) * 4, cc = ci0 + ni * 32 + row;
-    float* dst = out + (int64_t)(blockIdx.z / 3) * chunk_stride + ((int64_t)cr * 9 + (dy + 1) * 3) * cin + cc;
+    float* dst = out + (int64_t)chunk * chunk_stride + ((int64_t)cr * 9 + (dy + 1) * 3) * cin + cc;
     auto at = [&](int x, int t, int u, int i) -> float& {
         return dst[((t * 16 + i) * 9 + x) * cin + u * 16];
     };
@@ -724,30 +747,49 @@ __device__ __forceinline__ float tree256(float s, float* red) {
     return red[0];
 }
 
-// A layer's partial gradients into its gradients, in one launch.  Weights (the
-// blocks from `c` on, none if there was one chunk): dw[i] += part[i] + part[n +
-// i] + ... + part[(chunks - 1) n + i], in that order.  Bias channel j (block j):
-// db[j] += the sum over k of bpart[k * c + j], thread t adding k = t, t + 256,
-// ... in order, then a fixed LDS tree.
+// The layers' partial gradients into their gradients, in one launch (a launch of
+// 4.6 us for each of 14 layers before; 28 us for all of 64 x 64 frames' now, 13 of
+// 64 x 32 ones').  A layer's first `cout`
+// blocks take its bias: channel j's db += the sum over k of bpart[k * cout + j],
+// thread t adding k = t, t + 256, ... in order, then a fixed LDS tree.  The others
+// take its weights, if there were several chunks: dw[i] += part[i] + part[n + i]
+// + ... + part[(chunks - 1) n + i], in that order.
 __global__ void __launch_bounds__(256)
-k_grad_finish(const float* __restrict__ part, int chunks, int64_t n, float* __restrict__ dw,
-              const float* __restrict__ bpart, int nparts, int c, float* __restrict__ db)
+k_grad_finish(GradList l, const float* __restrict__ parts, const float* __restrict__ bparts,
+              float* __restrict__ grads)
 {
     __shared__ float red[256];
-    const int j = blockIdx.x;
+    int q = 0;
+    while (q + 1 < l.n && blockIdx.x >= l.block[q + 1]) q++;
+    const int j = blockIdx.x - l.block[q], c = l.cout[q];
     if (j < c) {
+        const float* bpart = bparts + l.bpoff[q];
         float s = 0.f;
-        for (int k = threadIdx.x; k < nparts; k += 256) s += bpart[(int64_t)k * c + j];
+        for (int k = threadIdx.x; k < l.bblocks[q]; k += 256) s += bpart[(int64_t)k * c + j];
         s = tree256(s, red);
+        float* db = grads + l.boff[q];
         if (threadIdx.x == 0) db[j] = db[j] + s;
         return;
     }
-    const int64_t i = (int64_t)(j - c) * 256 + threadIdx.x;
-    if (i >= n) return;
-    float s = part[i];
+    const float* part = parts + l.poff[q];
+    const int64_t n = (int64_t)c * 9 * l.cin[q], i = ((int64_t)(j - c) * 256 + threadIdx.x) * 4;
+    if (i >= n) return;   // (n is a multiple of 4)
+    float4 s = *reinterpret_cast<const float4*>(part + i);
 #pragma unroll 8
-    for (int k = 1; k < chunks; k++) s += part[(int64_t)k * n + i];
-    dw[i] += s;
+    for (int k = 1; k < l.chunks[q]; k++) {
+        const float4 v = *reinterpret_cast<const float4*>(part + (int64_t)k * n + i);
+        s.x += v.x;
+        s.y += v.y;
+        s.z += v.z;
+        s.w += v.w;
+    }
+    float4* dw = reinterpret_cast<float4*>(grads + l.woff[q] + i);
+    float4 o = *dw;
+    o.x += s.x;
+    o.y += s.y;
+    o.z += s.z;
+    o.w += s.w;
+    *dw = o;
 }
 
 // Block j: the sum over k of part[k * stride + col0 + j], k in [0, nparts):
@@ -1156,39 +1198,53 @@ void weight_flip(hipStream_t st, FlipList& l, const bf16* w, bf16* wt) {
     unsigned n = 0;
     for (int k = 0; k < l.n; k++) {
         l.block[k] = n;
-        n += nblk((int64_t)l.cin[k] * 9 * l.cout[k]);
+        n += (unsigned)(l.cin[k] / 32 * 9 * (l.cout[k] / 32));
     }
     k_weight_flip<<<n, 256, 0, st>>>(l, w, wt);
 }
-void conv_grads(hipStream_t st, const bf16* y, bf16* g, int cout, const bf16* in, int cin,
-                float* dw32, float* db, int nb, int H, int W, float* part, float* bpart) {
-    const int64_t npix = (int64_t)nb * H * W;
-    // the ReLU's backward and the bias: at most about one block per CU, so the
-    // sums of their partials stay short
-    const int bper = bias_pixels_per_block(npix);
-    const int bblocks = (int)bias_blocks(npix);   // partials: grad_partials (nn_sizes.h)
-    k_relu_bias_bwd<<<bblocks, 256, 0, st>>>(y, g, cout, (int)npix, bper, bpart);
-    const int per = dw_pixels_per_chunk(npix);
-    const int chunks = (int)dw_chunks(npix);   // partials: grad_partials (nn_sizes.h)
-    const int64_t nw = (int64_t)cout * 9 * cin;
-    float* dst = chunks == 1 ? dw32 : part;
-    const int64_t stride = chunks == 1 ? 0 : nw;
-    // the channels in tiles of 64, and of 32 what is left (three taps a block)
-    auto tiles = [&](auto kernel, int co, int ci, int first, int n) {
-        if (n > 0)
-            kernel<<<dim3(n / ci, cout / co, 3 * chunks), 256, 0, st>>>(
-                g, cout, in, cin, first, dst, stride, nb, H, W, per);
+void relu_bias_bwd(hipStream_t st, const bf16* y, bf16* g, int c, int64_t npix, float* bpart) {
+    // at most about one block per CU, so the sums of their partials stay short
+    k_relu_bias_bwd<<<(int)bias_blocks(npix), 256, 0, st>>>(y, g, c, (int)npix,
+                                                           bias_pixels_per_block(npix), bpart);
+}
+void conv3x3_dw(hipStream_t st, const DwLayer* layers, int n, float* grads, float* part) {
+    // the channels in tiles of 64, and of 32 what is left: a launch per kind of tile
+    auto launch = [&](auto kernel, int co, int ci) {
+        DwList l;
+        unsigned blocks = 0;
+        for (int k = 0; k < n; k++) {
+            const DwLayer& d = layers[k];
+            const int wide = d.cin / 64 * 64, left = d.cin - wide;
+            if ((d.cout % 64 == 0) != (co == 64) || (ci == 64 ? wide : left) == 0) continue;
+            DwLayer& o = l.layer[l.n];
+            o = d;
+            const int64_t npix = (int64_t)d.nb * d.H * d.W, nw = (int64_t)d.cout * 9 * d.cin;
+            const int chunks = (int)dw_chunks(npix);
+            o.per = dw_pixels_per_chunk(npix);
+            o.ci_first = ci == 64 ? 0 : wide;
+            o.ntile_ci = (ci == 64 ? wide : left) / ci;
+            o.out = chunks == 1 ? grads + d.woff : part + d.poff;
+            o.chunk_stride = chunks == 1 ? 0 : nw;
+            l.block[l.n++] = blocks;
+            blocks += (unsigned)(o.ntile_ci * (d.cout / co) * 3 * chunks);
+        }
+        if (blocks) kernel<<<blocks, 256, 0, st>>>(l);
     };
-    const int wide = cin / 64 * 64;
-    if (cout % 64 == 0) {
-        tiles(k_conv3x3_dw<64, 64>, 64, 64, 0, wide);
-        tiles(k_conv3x3_dw<64, 32>, 64, 32, wide, cin - wide);
-    } else {
-        tiles(k_conv3x3_dw<32, 64>, 32, 64, 0, wide);
-        tiles(k_conv3x3_dw<32, 32>, 32, 32, wide, cin - wide);
+    launch(k_conv3x3_dw<64, 64>, 64, 64);
+    launch(k_conv3x3_dw<64, 32>, 64, 32);
+    launch(k_conv3x3_dw<32, 64>, 32, 64);
+    launch(k_conv3x3_dw<32, 32>, 32, 32);
+}
+void grad_finish(hipStream_t st, GradList& l, const float* part, const float* bpart,
+                 float* grads) {
+    unsigned n = 0;
+    for (int k = 0; k < l.n; k++) {
+        l.block[k] = n;
+        l.chunks[k] = (int)dw_chunks(l.npix[k]);
+        l.bblocks[k] = (int)bias_blocks(l.npix[k]);
+        n += l.cout[k] + (l.chunks[k] > 1 ? nblk((int64_t)l.cout[k] * 9 * l.cin[k] / 4) : 0);
     }
-    k_grad_finish<<<cout + (chunks > 1 ? nblk(nw) : 0), 256, 0, st>>>(part, chunks, nw, dw32, bpart,
-                                                                      bblocks, cout, db);
+    k_grad_finish<<<n, 256, 0, st>>>(l, part, bpart, grads);
 }
 void maxpool(hipStream_t st, const bf16* x, bf16* y, int nb, int H, int W, int c, const int* live) {
     k_maxpool<<<nblk((int64_t)nb * H * W * c / 32), 256, 0, st>>>(x, y, nb, H, W, c, live);

@@ -30,6 +30,7 @@ int ctx_download(stm_ctx* ctx, void* dst, const void* src, size_t n);
 struct Conv {
     int cin, cout;
     int64_t woff, boff;          // offsets into the parameter buffers
+    int64_t poff = 0, bpoff = 0; // offsets of its partials (weights, bias)
     int level;                   // spatial level 0..3
     int x, y;                    // activation indices of input and output
 };
@@ -51,9 +52,10 @@ struct Net {
     float *p32 = nullptr, *g32 = nullptr, *m32 = nullptr, *v32 = nullptr;
     nn::bf16* pb = nullptr;      // bf16 copy of the parameters
     nn::bf16* wflip = nullptr;   // the backward-input weights of every layer, as pb
-    float* bpart = nullptr;      // partial sums of a layer's bias gradients
+    // partial sums of the layers' gradients (weights, bias), each at its layer's offset
+    float *gpart = nullptr, *bpart = nullptr;
     // FP32 partial sums: one slice per split of a split-K convolution in the
-    // forward pass, the per-block sums of the gradient and loss reductions in
+    // forward pass, the per-block sums of the head's and the loss' reductions in
     // training (scratch_floats in all, at least splitk_cap)
     float* splitk = nullptr;
     int64_t scratch_floats = 0;

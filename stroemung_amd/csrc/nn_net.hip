@@ -103,18 +103,19 @@ int Net::init(stm_ctx* c, int H_, int W_, int cap_, uint64_t seed) {
     NCHK(hipMemset(v32, 0, pbytes));
     NCHK(hipMemset(g32, 0, pbytes));
     NCHK(hipMalloc(&wflip, sizeof(bf16) * nparam));
-    int64_t nbias = 0;
-    for (auto& cv : convs)
-        nbias = std::max(nbias,
-                         nn::bias_partials(cv.cout, (int64_t)cap * h(cv.level) * w(cv.level)));
+    int64_t ngrad = 0, nbias = 0;
+    for (auto& cv : convs) {
+        const int64_t np = (int64_t)cap * h(cv.level) * w(cv.level);
+        cv.poff = ngrad;
+        cv.bpoff = nbias;
+        ngrad += nn::dw_partials(cv.cin, cv.cout, np);
+        nbias += nn::bias_partials(cv.cout, np);
+    }
+    NCHK(hipMalloc(&gpart, sizeof(float) * (size_t)std::max<int64_t>(ngrad, 1)));
     NCHK(hipMalloc(&bpart, sizeof(float) * (size_t)nbias));
     // the largest conv output is level 0's: cap x H x W x 32 (levels below have
     // a quarter of the pixels and twice the channels)
     scratch_floats = std::max(splitk_cap(), nn::loss_partials((int64_t)H * W, cap, 32));
-    for (auto& cv : convs)
-        scratch_floats = std::max(
-            scratch_floats,
-            nn::grad_partials(cv.cin, cv.cout, (int64_t)cap * h(cv.level) * w(cv.level)));
     NCHK(hipMalloc(&splitk, sizeof(float) * (size_t)scratch_floats));
     NCHK(hipMemset(splitk, 0, sizeof(float) * (size_t)scratch_floats));
     for (auto& a : acts) {
@@ -154,7 +155,7 @@ int Net::init(stm_ctx* c, int H_, int W_, int cap_, uint64_t seed) {
 }
 
 void Net::release() {
-    void* bufs[] = {p32, g32, m32, v32, pb, wflip, bpart, splitk, y, gy, target, mask, denom, loss,
+    void* bufs[] = {p32, g32, m32, v32, pb, wflip, gpart, bpart, splitk, y, gy, target, mask, denom, loss,
                     d_idx, dx, dt, host_in};
     for (void* b : bufs)
         if (b) hipFree(b);
@@ -270,12 +271,11 @@ void Net::forward_infer(int nb, const int* live) {
 
 void Net::backward(int nb) {
     auto npix = [&](int level) { return (int64_t)nb * h(level) * w(level); };
-    // gradient through conv k (ReLU included); the gradient of its output is in acts[y].g
+    // gradient through conv k (ReLU included) to its input; that of its output is in acts[y].g
     auto conv_bwd = [&](int k, bool need_gx) {
         const Conv& c = convs[k];
         const int hh = h(c.level), ww = w(c.level);
-        nn::conv_grads(stream, acts[c.y].v, acts[c.y].g, c.cout, acts[c.x].v, c.cin, g32 + c.woff,
-                       g32 + c.boff, nb, hh, ww, splitk, bpart);
+        nn::relu_bias_bwd(stream, acts[c.y].v, acts[c.y].g, c.cout, npix(c.level), bpart + c.bpoff);
         if (need_gx)
             nn::conv3x3(stream, acts[c.y].g, c.cout, wflip + c.woff, nullptr, acts[c.x].g, nullptr,
                         c.cin, nb, hh, ww, 0);
@@ -309,6 +309,23 @@ void Net::backward(int nb) {
     nn::maxpool_bwd(stream, acts[2].v, acts[3].v, acts[3].g, acts[2].g, nb, h(0), w(0), 32);
     conv_bwd(1, true);
     conv_bwd(0, false);
+    // the parameters' gradients: every layer's output gradient is still there
+    nn::DwLayer dw[16];
+    nn::GradList grads;
+    for (const Conv& c : convs) {
+        const int k = grads.n++;
+        dw[k] = nn::DwLayer{acts[c.y].g, acts[c.x].v, c.cout, c.cin, nb, h(c.level), w(c.level),
+                            c.woff, c.poff};
+        grads.cin[k] = c.cin;
+        grads.cout[k] = c.cout;
+        grads.npix[k] = npix(c.level);
+        grads.woff[k] = c.woff;
+        grads.boff[k] = c.boff;
+        grads.poff[k] = c.poff;
+        grads.bpoff[k] = c.bpoff;
+    }
+    nn::conv3x3_dw(stream, dw, grads.n, g32, gpart);
+    nn::grad_finish(stream, grads, gpart, bpart, g32);
 }
 
 // One Adam step on the batch already in acts[0].v / target / mask.

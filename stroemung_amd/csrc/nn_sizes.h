@@ -43,14 +43,17 @@ inline int64_t bias_partials(int cout, int64_t npix) {
     return std::min<int64_t>((npix + 127) / 128, 257) * cout;
 }
 
-// Partials (floats) of the weight and bias gradients for any pixel count up to
+// Partials (floats) of the weight gradient of a layer for any pixel count up to
 // npix.  The chunk counts are not monotone in the pixel count: at most 257
 // chunks until the chunk size stops growing, at most 257 bias blocks.
-inline int64_t grad_partials(int cin, int cout, int64_t npix) {
+inline int64_t dw_partials(int cin, int cout, int64_t npix) {
     const int64_t chunks =
         std::min((npix + 1023) / 1024, std::max<int64_t>(257, (npix + (1 << 20) - 1) >> 20));
-    const int64_t dw = chunks > 1 ? chunks * cout * 9 * cin : 0;
-    return std::max(dw, bias_partials(cout, npix));
+    return chunks > 1 ? chunks * cout * 9 * cin : 0;
+}
+// The larger of a layer's two kinds of partials.
+inline int64_t grad_partials(int cin, int cout, int64_t npix) {
+    return std::max(dw_partials(cin, cout, npix), bias_partials(cout, npix));
 }
 
 // Partials of loss (per-sample sums over 64 blocks, then one per 256-pixel
