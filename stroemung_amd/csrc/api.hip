@@ -48,6 +48,7 @@ struct HostChan {
     double n_inner = 0.0;          // interior fluid cells
     int32_t tile0 = 0, ntiles = 0, boff = 0;
     int32_t tb0 = 0, ntb = 0;      // blocked-solver tiles of the current variant
+    int32_t lex = -1;              // instance of the pipelined lexicographic solve, -1: none
 };
 
 struct KStat {
@@ -279,7 +280,7 @@ ChanDesc make_desc(const HostChan& c) {
     d.check_every = q.check_every > 0 ? q.check_every : 1;
     d.tb0 = c.tb0;
     d.ntb = c.ntb;
-    d.lex_class = lex_class(d.nx, d.ny);
+    d.lex_class = c.lex;
     d.delx = q.delx;
     d.dely = q.dely;
     d.gamma = q.gamma;
@@ -504,6 +505,7 @@ int finalize(stm_ctx* ctx) {
     for (size_t k = 0; k < ctx->chans.size(); k++) {
         HostChan& c = ctx->chans[k];
         c.pitch = (uint32_t)round_up(c.ny, 16);
+        c.lex = lex_class((int)c.nx, (int)c.ny);
         c.off = off;
         off += round_up((int64_t)c.nx * c.pitch, 64);
         c.tile0 = tiles;
@@ -1107,14 +1109,20 @@ int lex_buffers(stm_ctx* ctx) {
     int64_t n = 0;
     for (const HostChan& c : ctx->chans) {
         off.push_back(n);
-        n += round_up(lex_work_doubles(lex_class((int)c.nx, (int)c.ny), (int)c.nx, (int)c.ny), 16);
+        n += round_up(lex_work_doubles(c.lex, (int)c.nx, (int)c.ny), 16);
     }
     if (n == 0) return STM_OK;
     if (!ctx->d_lexoff) HIPCHK(ctx, hipMalloc(&ctx->d_lexoff, sizeof(int64_t) * off.size()));
     HIPCHK(ctx, hipMemcpyAsync(ctx->d_lexoff, off.data(), sizeof(int64_t) * off.size(),
                                hipMemcpyHostToDevice, ctx->stream));
     HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
-    HIPCHK(ctx, hipMalloc(&ctx->lexwork, sizeof(double) * (size_t)n));
+    if (hipMalloc(&ctx->lexwork, sizeof(double) * (size_t)n) != hipSuccess) {
+        // no memory for it: k_lex_solve takes every channel, in the fields alone
+        (void)hipGetLastError();
+        ctx->lexwork = nullptr;
+        for (HostChan& c : ctx->chans) c.lex = -1;
+        return upload_descs(ctx);
+    }
     launch_fill(ctx->stream, n, ctx->lexwork, 0.0);
     for (int k = 0; k < N_LEX_CLASSES; k++)
         launch_lex_init(ctx->stream, k, nch(ctx), ctx->d_cd, ctx->d_lexoff, ctx->lexwork);
@@ -1130,7 +1138,7 @@ int stage_lex(stm_ctx* ctx) {
     if (rc) return rc;
     std::vector<bool> used(N_LEX_CLASSES + 1, false);
     for (const HostChan& c : ctx->chans)
-        if (c.prm.solver == STM_SOLVER_LEX) used[1 + lex_class((int)c.nx, (int)c.ny)] = true;
+        if (c.prm.solver == STM_SOLVER_LEX) used[1 + c.lex] = true;
     if (used[0] || ctx->lex_few)
         LAUNCH("lex_solve", launch_lex_solve(ctx->stream, nch(ctx), ctx->d_cd, ctx->d_cs,
                                              ctx->d_be, ctx->flags, ctx->rhs, ctx->p,
