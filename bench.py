@@ -57,10 +57,10 @@ SWEEP_BYTES_PER_CELL = 33.0
 STAGE_BYTES_PER_CELL = {"fg": 33.0, "rhs": 24.0, "fg_rhs": 41.0, "adap_ranges": 41.0,
                         "ranges": 25.0}
 COPY_PROBE_BYTES = 256 << 20
-# template arguments (R, HY, NS) of each blocked-solver variant, after K
-VARIANT_SHAPES = {0: "4, 32, 16", 1: "4, 32, 16", 2: "4, 64, 16", 3: "4, 32, 16",
-                  4: "4, 64, 16", 5: "6, 64, 16", 6: "6, 64, 16", 7: "2, 64, 16",
-                  8: "12, 64, 8", 9: "6, 48, 16"}
+# template arguments (rows per strip, row pairs, strips) of each blocked-solver variant
+VARIANT_SHAPES = {0: "4, 64, 8", 1: "4, 64, 8", 2: "6, 64, 8", 3: "4, 64, 8",
+                  4: "10, 64, 8", 5: "10, 64, 8", 6: "10, 64, 8", 7: "6, 64, 12",
+                  8: "6, 64, 16", 9: "6, 48, 16"}
 
 
 def parse():
@@ -288,7 +288,7 @@ def sweeps_run(a):
                                "autotune_us_per_sweep": tuned[1]},
                    "wall_us_per_sweep": (t1 - t0) * 1e6 / (launches * k),
                    "timing": "wall time of the sweeps stage / working launches"},
-        "roofline": {"kernel": "k_rb_strip<%d, %s>" % (k, VARIANT_SHAPES.get(variant, "?")),
+        "roofline": {"kernel": "k_rb_strip<%s>, %d sweeps" % (VARIANT_SHAPES.get(variant, "?"), k),
                      "bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": achieved / HBM_PEAK_GBS, "traffic": None,
                      "bytes_per_launch": unique, "loaded_bytes_per_launch": loaded,
@@ -446,7 +446,7 @@ def channels_run(a):
     if not timed:
         ms, timed = sms, stimed
     avg_s = ms / 1e3 / max(timed, 1)
-    # every launch moves at most each cell of every channel once (25 B); launches
+    # every launch moves at most each cell of every channel once (24 B); launches
     # after compaction move only the running channels', so this is an upper bound
     unique, loaded = ctx.solver_bytes()
     achieved = unique / avg_s / 1e9 if timed else None
@@ -473,12 +473,12 @@ def channels_run(a):
             "cell_sweeps_per_s": swept / elapsed,
         },
         "roofline": {
-            "kernel": "k_rb_strip<%d, %s>" % (ksweeps, VARIANT_SHAPES.get(variant, "?")),
+            "kernel": "k_rb_strip<%s>, %d sweeps" % (VARIANT_SHAPES.get(variant, "?"), ksweeps),
             "bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": achieved / HBM_PEAK_GBS if achieved else None, "traffic": None,
             "bytes_per_launch": unique, "loaded_bytes_per_launch": loaded,
             "halo_factor": loaded / unique,
-            "model": "25 B per cell of every channel per launch (an upper bound: launches "
+            "model": "24 B per cell of every channel per launch (an upper bound: launches "
                      "after compaction cover only the running channels)",
             "effective_sweep_gbs": effective,
             "avg_launch_us": avg_s * 1e6, "launches": launches,
@@ -841,7 +841,7 @@ def main():
     value = cells * a.steps / elapsed
 
     kname = "rb_tb"
-    kernel_id = "k_rb_strip<%d, %s>" % (ksweeps, VARIANT_SHAPES.get(variant, "?"))
+    kernel_id = "k_rb_strip<%s>, %d sweeps" % (VARIANT_SHAPES.get(variant, "?"), ksweeps)
     traffic = None
     try:
         with open(os.path.join(ROOT, "profiles", "traffic.json")) as fh:
@@ -859,7 +859,7 @@ def main():
     _, _, launches = ctx.kernel_stats(kname)
     avg_s = ms / 1e3 / max(timed, 1)
     # one launch advances every cell by ksweeps red-black sweeps on chip: it
-    # must move each cell's p, rhs and flags in and p out once (25 B per cell);
+    # must move each cell's p and rhs in and p out once (24 B per cell);
     # its tiles' overlapping halos load more (loaded / unique = halo factor)
     unique, loaded = ctx.solver_bytes()
     achieved = unique / avg_s / 1e9 if timed else None
@@ -916,7 +916,7 @@ def main():
                                "scaled by a 256 MiB copy (profiles/traffic.json); not "
                                "measured in this run" if traffic else None),
             "bytes_per_launch": unique,
-            "model": "25 B per cell per launch: p read, rhs read, flags read, p written",
+            "model": "24 B per cell per launch: p read, rhs read, p written",
             "loaded_bytes_per_launch": loaded,
             "halo_factor": loaded / unique,
             "effective_sweep_gbs": effective,

@@ -28,9 +28,10 @@
 // per sweep.
 //
 // Registers and LDS: the region is EX x EY cells; a strip is R rows of it,
-// held by one wave in registers, p and rhs, lane m the y-pair (2m, 2m + 1) of every row -- one red and one black
-// cell each.  E / W neighbours are the lane's own registers, one of N / S is
-// the pair's other cell and the other comes from the next lane by DPP; only a
+// held by one wave in registers, p and rhs, lane m the y-pair (2m, 2m + 1) of
+// every row -- one red and one black cell each.  E / W neighbours are the
+// lane's own registers, one of N / S is the pair's other cell and the other
+// comes from the next lane by DPP; only a
 // strip's first and last row go through LDS, for the strips next to it.  A
 // cell then costs 7 FP64 operations and two 32-bit moves (43 cycles per wave
 // and row measured, 36 issued), and a half-sweep 150 cycles on top for the

@@ -158,7 +158,7 @@ class Context:
 
     def solver_bytes(self):
         """(unique, loaded) bytes of one blocked launch of the current
-        variant: every cell once (25 B) and what the overlapping tiles move."""
+        variant: every cell once (24 B) and what the overlapping tiles move."""
         u, l = C.c_double(), C.c_double()
         self._check(lib().stm_solver_bytes(self._ctx, C.byref(u), C.byref(l)))
         return u.value, l.value
