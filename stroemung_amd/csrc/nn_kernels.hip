@@ -223,6 +223,16 @@ k_conv3x3_small(const bf16* __restrict__ in, int cin, const bf16* __restrict__ w
 // slices of matrix work.  The other launches (few slices, or enough
 // workgroups that occupancy hides the latency) stage each slice and then
 // multiply, in half the LDS.
+//
+// LDS strides: a 16-byte read serves 16 lanes at once, lanes 0 to 3 and 12 to 15
+// of one 8-channel group (kq) with lanes 4 to 11 of the next, over 64 banks.  In
+// units of 16 bytes an operand's 16 rows then miss each other if their stride is 2
+// more than a multiple of 4: a pixel takes 6 units, a channel's nine weight rows
+// 38, and where a fragment is eight pixels of two image rows, those lie 4 units
+// further apart.  With 5 units a pixel and 45 a channel a read took 8 to 12 cycles
+// instead of 4 (4.8 cycles of conflicts per LDS instruction counted, 0.7 now, the
+// stores'): the 14 layers of 32 frames of 64 x 64 147 us, 138 now; of 64 frames of
+// 128 x 64 399 and 381.
 template <int TW, int TH, int WN, bool POOL, bool PIPE>
 __global__ void __launch_bounds__(256)
 k_conv3x3_tile(ConvIn src, const bf16* __restrict__ w, const float* __restrict__ bias,
@@ -230,8 +240,9 @@ k_conv3x3_tile(ConvIn src, const bf16* __restrict__ w, const float* __restrict__
                int flags)
 {
     constexpr int PH = TH + 2, PW = TW + 2;
-    constexpr int CS = 40;                       // padded channel stride of a staged pixel
-    constexpr int CSW = 40;                      // ... of a staged (channel, tap) weight row
+    constexpr int CS = 48;                       // padded channel stride of a staged pixel
+    constexpr int RS = PW * CS + (TW == 8 ? 32 : 0);   // stride of a patch row
+    constexpr int CHS = 9 * 32 + 16;             // stride of a channel's nine weight rows
     constexpr int NW = 32 * WN;                  // output channels of the workgroup
     constexpr int WM = 4 / WN;                   // waves along M
     constexpr int RM = 16 / TW;                  // image rows per M tile
@@ -244,8 +255,8 @@ k_conv3x3_tile(ConvIn src, const bf16* __restrict__ w, const float* __restrict__
     constexpr int NB = PIPE ? 2 : 1;
     static_assert(TW == 8 || TW == 16, "tile width");
     static_assert(MT >= 1 && TH * TW % (WM * 16) == 0, "tile shape");
-    __shared__ __attribute__((aligned(16))) bf16 patch[NB][PH * PW * CS];
-    __shared__ __attribute__((aligned(16))) bf16 wl[NB][NW * 9 * CSW];
+    __shared__ __attribute__((aligned(16))) bf16 patch[NB][PH * RS];
+    __shared__ __attribute__((aligned(16))) bf16 wl[NB][NW * CHS];
 
     const int cin = src.ca + src.cb;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -263,8 +274,8 @@ k_conv3x3_tile(ConvIn src, const bf16* __restrict__ w, const float* __restrict__
 
     // this lane's LDS offsets: its pixel of the wave's first M tile at tap
     // (0, 0), and its weight row (channel n_base + row) at tap 0
-    const int aoff = ((wm * MT * RM + row / TW) * PW + row % TW) * CS + kq;
-    const int boff = (wn * 32 + row) * 9 * CSW + kq;
+    const int aoff = (wm * MT * RM + row / TW) * RS + row % TW * CS + kq;
+    const int boff = (wn * 32 + row) * CHS + kq;
     f32x4 acc[MT][2];
 #pragma unroll
     for (int i = 0; i < MT; i++)
@@ -335,13 +346,14 @@ k_conv3x3_tile(ConvIn src, const bf16* __restrict__ w, const float* __restrict__
                                        fmaxf((float)g.raw[k][2][e], (float)g.raw[k][3][e]));
             }
             if (!((g.valid >> k) & 1u)) x = zero8();
-            *reinterpret_cast<bf16x8*>(&patch[buf][(v >> 2) * CS + (v & 3) * 8]) = x;
+            *reinterpret_cast<bf16x8*>(&patch[buf][(v >> 2) * CS + (v >> 2) / PW * (RS - PW * CS) +
+                                                    (v & 3) * 8]) = x;
         }
 #pragma unroll
         for (int k = 0; k < NWV; k++) {
             const int v = threadIdx.x + k * 256;
             if (v >= NWVEC) continue;
-            *reinterpret_cast<bf16x8*>(&wl[buf][(v >> 2) * CSW + (v & 3) * 8]) = g.w[k];
+            *reinterpret_cast<bf16x8*>(&wl[buf][v * 8 + v / 36 * (CHS - 288)]) = g.w[k];
         }
     };
     auto mfmas = [&](int buf) {
@@ -354,10 +366,10 @@ k_conv3x3_tile(ConvIn src, const bf16* __restrict__ w, const float* __restrict__
             for (int dy = 0; dy < 3; dy++)
 #pragma unroll
                 for (int u = 0; u < 2; u++)
-                    bq[dy][u] = *reinterpret_cast<const bf16x8*>(pb + (u * 16 * 9 + dy * 3 + dx) * CSW);
+                    bq[dy][u] = *reinterpret_cast<const bf16x8*>(pb + u * 16 * CHS + (dy * 3 + dx) * 32);
 #pragma unroll
             for (int s = 0; s < NS; s++) {
-                const bf16x8 a = *reinterpret_cast<const bf16x8*>(pa + (s * PW + dx) * CS);
+                const bf16x8 a = *reinterpret_cast<const bf16x8*>(pa + s * RS + dx * CS);
 #pragma unroll
                 for (int dy = 0; dy < 3; dy++) {
                     const int d = s - dy;
