@@ -31,7 +31,8 @@ struct ConvIn {
 };
 
 // 3x3 convolution, padding 1, NHWC bf16, fp32 accumulation on the matrix
-// cores.  w is [cout][9][cin] bf16; flags 1 = add bias (fp32), 2 = ReLU.
+// cores.  w is bf16 [cin / 32][9][cout][32], the last the channels of a slice;
+// flags 1 = add bias (fp32), 2 = ReLU.
 // Writes bf16 `out` and/or fp32 `out32` (either may be null).
 // live (device int, may be null): only images [0, *live) are computed
 void conv3x3(hipStream_t, const bf16* in, int cin, const bf16* w, const float* bias, bf16* out,
@@ -41,12 +42,14 @@ void conv3x3(hipStream_t, const bf16* in, int cin, const bf16* w, const float* b
 bool conv_tiles_fit(int H, int W);
 void conv3x3_in(hipStream_t, const ConvIn& src, const bf16* w, const float* bias, bf16* out,
                 float* out32, int cout, int nb, int H, int W, int flags);
-// w'[ci][8 - tap][co] = w[co][tap][ci]: the backward-input weights of each layer
-// of the list, at the offset of its weights
-struct FlipList {
+struct WeightList {       // the 3x3 layers' weights in the parameter buffers
     int n = 0;
     int cin[16], cout[16];
     int64_t off[16];
+};
+// w'[ci][8 - tap][co] = w[co][tap][ci]: the backward-input weights of each layer
+// of the list, at the offset of its weights (both in the form that conv3x3 reads)
+struct FlipList : WeightList {
     unsigned block[16];   // first workgroup of each layer (filled by weight_flip)
 };
 void weight_flip(hipStream_t, FlipList& layers, const bf16* w, bf16* wt);
@@ -103,9 +106,11 @@ void head_bwd(hipStream_t, const bf16* x, const float* w, const float* gy, bf16*
 // denom[s] = sum m t^2 of sample s; loss_out += the masked, normalised MSE; gy its gradient
 void loss(hipStream_t, const float* y, const float* t, const float* m, float* denom, float* gy,
           float* loss_out, int64_t npix_per, int nb, float* part);
-void adam(hipStream_t, int64_t n, float* p, const float* g, float* m, float* v, bf16* pb, float lr,
-          float b1, float b2, float eps, int step, float clip);
-void to_bf16(hipStream_t, int64_t n, const float* x, bf16* y);
+void adam(hipStream_t, const WeightList& layers, int64_t n, float* p, const float* g, float* m,
+          float* v, bf16* pb, float lr, float b1, float b2, float eps, int step, float clip);
+// The bf16 copy of the parameters, the layers' weights as [ci / 32][tap][co][ci % 32]: the
+// form that every kernel here reads (n a multiple of 4).
+void to_bf16(hipStream_t, const WeightList& layers, int64_t n, const float* x, bf16* y);
 
 }  // namespace nn
 }  // namespace stm

@@ -82,13 +82,13 @@ k_conv3x3(const bf16* __restrict__ in, int cin, const bf16* __restrict__ w,
         }
         const bf16* brow[2];
 #pragma unroll
-        for (int u = 0; u < 2; u++) brow[u] = w + ((int64_t)(n_base + u * 16 + row) * 9 + tap) * cin;
+        for (int u = 0; u < 2; u++) brow[u] = w + ((int64_t)tap * cout + n_base + u * 16 + row) * 32 + kq;
         for (int c0 = 0; c0 < cin; c0 += 32) {
             bf16x8 a[MT], b[2];
 #pragma unroll
             for (int t = 0; t < MT; t++) a[t] = aok[t] ? load8(arow[t] + c0 + kq) : zero8();
 #pragma unroll
-            for (int u = 0; u < 2; u++) b[u] = load8(brow[u] + c0 + kq);
+            for (int u = 0; u < 2; u++) b[u] = load8(brow[u] + (int64_t)c0 * 9 * cout);
 #pragma unroll
             for (int t = 0; t < MT; t++)
 #pragma unroll
@@ -119,10 +119,10 @@ k_conv3x3(const bf16* __restrict__ in, int cin, const bf16* __restrict__ w,
 // of at most 64 pixels whose sides the tiles below do not divide: the deep
 // levels of a small frame.  A workgroup holds one whole image with its border of
 // zeros in LDS (all its channels), and each of its four waves one 16-pixel by
-// 16-channel tile.  A channel's weights are contiguous in the order they are
-// used, so a lane streams its own from L2, nine steps ahead.  The kernel above
+// 16-channel tile.  A step's weights are a kilobyte in one piece (packed_at), and a
+// wave streams them from L2, nine steps ahead.  The kernel above
 // waits for two loads from memory at every step, with a workgroup on a few CUs:
-// 31 us for 32 images of 8 x 4 pixels and 256 to 256 channels, 13.8 here.
+// 31 us for 32 images of 8 x 4 pixels and 256 to 256 channels, 12.6 here.
 constexpr int SMALL_PIXELS = 64, SMALL_LDS = 64 * 1024;
 static inline int small_patch_bytes(int cin, int H, int W) {
     return (H + 2) * (W + 2) * (cin + 8) * (int)sizeof(bf16);
@@ -150,18 +150,26 @@ k_conv3x3_small(const bf16* __restrict__ in, int cin, const bf16* __restrict__ w
     if (n0 >= cout || tile * 16 >= HW) return;
     const int pix = min(tile * 16 + row, HW - 1), py = pix / W, px = pix - py * W;
     const bf16* pa = &patch[(py * PW + px) * cs + kq];   // tap 0: one row up, one left
-    const bf16* pw = w + (int64_t)(n0 + row) * 9 * cin + kq;
+    const bf16* pw = w + (n0 + row) * 32 + kq;
     // steps of 32 k's: tap-major, then the channels; nine at a time
     const int per = cin / 32, batches = per;             // 9 * per steps
     bf16x8 cur[9], nxt[9];
+    int tw = 0, cw = 0;                                  // step of the next load
+    auto weights = [&](bf16x8 (&q)[9]) {
 #pragma unroll
-    for (int j = 0; j < 9; j++) cur[j] = load8(pw + j * 32);
+        for (int j = 0; j < 9; j++) {
+            q[j] = load8(pw + (int64_t)(cw * 9 + tw) * cout * 32);
+            if (++cw == per) {
+                cw = 0;
+                tw = tw == 8 ? 0 : tw + 1;               // (past the end: loaded, not used)
+            }
+        }
+    };
+    weights(cur);
     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
     int tap = 0, c = 0;
     for (int b = 0; b < batches; b++) {
-        const bf16* ahead = pw + (int64_t)min(b + 1, batches - 1) * 9 * 32;
-#pragma unroll
-        for (int j = 0; j < 9; j++) nxt[j] = load8(ahead + j * 32);
+        weights(nxt);
         __builtin_amdgcn_sched_barrier(0);   // the loads issue before the MFMAs
 #pragma unroll
         for (int j = 0; j < 9; j++) {
@@ -323,14 +331,13 @@ k_conv3x3_tile(ConvIn src, const bf16* __restrict__ w, const float* __restrict__
                 g.raw[k][3] = load8(base + r0 + rs + cs);
             }
         }
-        // the weights w[nb0 + n][tap][c0 .. c0 + 31] of the slice: vector
-        // v = (n * 9 + tap) * 4 + part
+        // the slice's weights: vector v = (tap * NW + n) * 4 + part
+        const bf16* ws = w + ((int64_t)(c0 / 32) * 9 * cout + nb0) * 32;
 #pragma unroll
         for (int k = 0; k < NWV; k++) {
             const int v = threadIdx.x + k * 256;
             const int vv = v < NWVEC ? v : 0;
-            g.w[k] = load8(w + (int64_t)(nb0 + (vv >> 2) / 9) * 9 * cin +
-                           (int64_t)((vv >> 2) % 9) * cin + c0 + (vv & 3) * 8);
+            g.w[k] = load8(ws + (int64_t)(vv / (NW * 4)) * cout * 32 + vv % (NW * 4) * 8);
         }
     };
     auto put = [&](const Stage& g, int buf) {
@@ -353,7 +360,7 @@ k_conv3x3_tile(ConvIn src, const bf16* __restrict__ w, const float* __restrict__
         for (int k = 0; k < NWV; k++) {
             const int v = threadIdx.x + k * 256;
             if (v >= NWVEC) continue;
-            *reinterpret_cast<bf16x8*>(&wl[buf][v * 8 + v / 36 * (CHS - 288)]) = g.w[k];
+            *reinterpret_cast<bf16x8*>(&wl[buf][(v >> 2) % NW * CHS + v / (NW * 4) * 32 + (v & 3) * 8]) = g.w[k];
         }
     };
     auto mfmas = [&](int buf) {
@@ -550,11 +557,11 @@ k_weight_flip(FlipList l, const bf16* __restrict__ w, bf16* __restrict__ wt)
     bf16* to = wt + l.off[k];
 #pragma unroll
     for (int r = row; r < 32; r += 8)
-        tile[r][lane] = from[((int64_t)(co0 + r) * 9 + 8 - tap) * cin + ci0 + lane];
+        tile[r][lane] = from[((int64_t)(ci0 / 32 * 9 + 8 - tap) * cout + co0 + r) * 32 + lane];
     __syncthreads();
 #pragma unroll
     for (int r = row; r < 32; r += 8)
-        to[((int64_t)(ci0 + r) * 9 + tap) * cout + co0 + lane] = tile[lane][r];
+        to[((int64_t)(co0 / 32 * 9 + tap) * cin + ci0 + r) * 32 + lane] = tile[lane][r];
 }
 
 // dw[co][tap][ci] over a pixel chunk: sum of gz[pix][co] * in[pix+off][ci].
@@ -1104,27 +1111,67 @@ __global__ void k_target_norm(const float* __restrict__ t, const float* __restri
         part[(int64_t)blockIdx.x * gridDim.y + s] = red[0] + (blockIdx.x == 0 ? 1e-30f : 0.f);
 }
 
-// Adam on fp32 master weights; refreshes the bf16 copy used by the kernels
-__global__ void k_adam(int64_t n, float* __restrict__ p, const float* __restrict__ g,
-                       float* __restrict__ m, float* __restrict__ v, bf16* __restrict__ pb,
-                       float lr, float b1, float b2, float eps, float c1, float c2, float clip)
-{
-    const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= n) return;
-    float gk = g[k] * clip;
-    const float mk = b1 * m[k] + (1.f - b1) * gk;
-    const float vk = b2 * v[k] + (1.f - b2) * gk * gk;
-    m[k] = mk;
-    v[k] = vk;
-    const float upd = lr * (mk / c1) / (sqrtf(vk / c2) + eps);
-    p[k] -= upd;
-    if (pb) pb[k] = (bf16)p[k];
+// Where the bf16 copy keeps parameter k: a layer's weights w[co][tap][ci] lie there
+// as [ci / 32][tap][co][ci % 32], so that what a workgroup reads for 32 input
+// channels is whole lines.  (In the masters' order they were 64-byte pieces cin * 2
+// bytes apart, in as few as four of an L2's 16 channels at once: the forward pass of
+// 64 frames of 128 x 64 379 us, 358 so, of 32 of 64 x 64 139 and 137, a training
+// step of 32 of 64 x 32 481 and 472.)
+// Four parameters from a multiple of 4 on stay together (all counts and offsets
+// are multiples of 4); what is no 3x3 weight keeps its place.
+typedef __bf16 bf16x4p __attribute__((ext_vector_type(4)));
+static __device__ __forceinline__ int64_t packed_at(const WeightList& l, int64_t k) {
+    int q = 0;
+    while (q + 1 < l.n && k >= l.off[q + 1]) q++;
+    const int r = (int)(k - l.off[q]), cin = l.cin[q];
+    if (r < 0 || r >= 9 * cin * l.cout[q]) return k;
+    const int t = r / cin, ci = r - t * cin, co = t / 9, tap = t - co * 9;
+    return l.off[q] + ((int64_t)(ci / 32 * 9 + tap) * l.cout[q] + co) * 32 + ci % 32;
+}
+static __device__ __forceinline__ void put_packed(const WeightList& l, int64_t k, float4 p,
+                                                  bf16* __restrict__ pb) {
+    *reinterpret_cast<bf16x4p*>(pb + packed_at(l, k)) =
+        bf16x4p{(bf16)p.x, (bf16)p.y, (bf16)p.z, (bf16)p.w};
 }
 
-__global__ void k_to_bf16(int64_t n, const float* __restrict__ x, bf16* __restrict__ y)
+// Adam on fp32 master weights; refreshes the bf16 copy used by the kernels.  Four
+// parameters a thread (n a multiple of 4), so that finding their place in the copy,
+// two divisions, is a small part: 12 us for the 1 955 240 of a network with one a
+// thread and no place to find, 21 with it, 12 now.
+__global__ void __launch_bounds__(256)
+k_adam(WeightList l, int64_t n, float* __restrict__ p, const float* __restrict__ g,
+       float* __restrict__ m, float* __restrict__ v, bf16* __restrict__ pb, float lr, float b1,
+       float b2, float eps, float c1, float c2, float clip)
 {
-    const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (k < n) y[k] = (bf16)x[k];
+    const int64_t k = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
+    if (k >= n) return;
+    const float4 g4 = *reinterpret_cast<const float4*>(g + k);
+    float4 m4 = *reinterpret_cast<const float4*>(m + k), v4 = *reinterpret_cast<const float4*>(v + k);
+    float4 p4 = *reinterpret_cast<const float4*>(p + k);
+    auto step = [&](float gk, float& mq, float& vq, float& pq) {
+        gk = gk * clip;
+        const float mk = b1 * mq + (1.f - b1) * gk;
+        const float vk = b2 * vq + (1.f - b2) * gk * gk;
+        mq = mk;
+        vq = vk;
+        const float upd = lr * (mk / c1) / (sqrtf(vk / c2) + eps);
+        pq -= upd;
+    };
+    step(g4.x, m4.x, v4.x, p4.x);
+    step(g4.y, m4.y, v4.y, p4.y);
+    step(g4.z, m4.z, v4.z, p4.z);
+    step(g4.w, m4.w, v4.w, p4.w);
+    *reinterpret_cast<float4*>(m + k) = m4;
+    *reinterpret_cast<float4*>(v + k) = v4;
+    *reinterpret_cast<float4*>(p + k) = p4;
+    put_packed(l, k, p4, pb);
+}
+
+__global__ void __launch_bounds__(256)
+k_to_bf16(WeightList l, int64_t n, const float* __restrict__ x, bf16* __restrict__ y)
+{
+    const int64_t k = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
+    if (k < n) put_packed(l, k, *reinterpret_cast<const float4*>(x + k), y);
 }
 
 // ------------------------------------------------------------ launchers
@@ -1294,13 +1341,13 @@ void loss(hipStream_t st, const float* y, const float* t, const float* m, float*
     k_loss<<<nblocks, 256, 0, st>>>(y, t, m, denom, gy, part, npix_per, nb);
     k_block_sum<<<1, 256, 0, st>>>(part, nblocks, 1, 0, loss_out, 1);
 }
-void adam(hipStream_t st, int64_t n, float* p, const float* g, float* m, float* v, bf16* pb,
+void adam(hipStream_t st, const WeightList& l, int64_t n, float* p, const float* g, float* m, float* v, bf16* pb,
           float lr, float b1, float b2, float eps, int step, float clip) {
     const float c1 = 1.f - powf(b1, (float)step), c2 = 1.f - powf(b2, (float)step);
-    k_adam<<<nblk(n), 256, 0, st>>>(n, p, g, m, v, pb, lr, b1, b2, eps, c1, c2, clip);
+    k_adam<<<nblk(n / 4), 256, 0, st>>>(l, n, p, g, m, v, pb, lr, b1, b2, eps, c1, c2, clip);
 }
-void to_bf16(hipStream_t st, int64_t n, const float* x, bf16* y) {
-    k_to_bf16<<<nblk(n), 256, 0, st>>>(n, x, y);
+void to_bf16(hipStream_t st, const WeightList& l, int64_t n, const float* x, bf16* y) {
+    k_to_bf16<<<nblk(n / 4), 256, 0, st>>>(l, n, x, y);
 }
 
 }  // namespace nn

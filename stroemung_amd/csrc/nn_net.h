@@ -50,7 +50,8 @@ struct Net {
     std::vector<Act> acts;
     int64_t nparam = 0, head_w = 0, head_b = 0;
     float *p32 = nullptr, *g32 = nullptr, *m32 = nullptr, *v32 = nullptr;
-    nn::bf16* pb = nullptr;      // bf16 copy of the parameters
+    nn::bf16* pb = nullptr;      // bf16 copy of the parameters (weights packed)
+    nn::WeightList weights;      // where the layers' weights are
     nn::bf16* wflip = nullptr;   // the backward-input weights of every layer, as pb
     // partial sums of the layers' gradients (weights, bias), each at its layer's offset
     float *gpart = nullptr, *bpart = nullptr;

@@ -85,6 +85,11 @@ int Net::init(stm_ctx* c, int H_, int W_, int cap_, uint64_t seed) {
         off = (off + 7) / 8 * 8;   // keep every weight block 16-byte aligned in bf16
         convs.push_back(cv);
     }
+    for (const Conv& cv : convs) {
+        weights.cin[weights.n] = cv.cin;
+        weights.cout[weights.n] = cv.cout;
+        weights.off[weights.n++] = cv.woff;
+    }
     head_w = off;
     off += 32;
     head_b = off;
@@ -149,7 +154,7 @@ int Net::init(stm_ctx* c, int H_, int W_, int cap_, uint64_t seed) {
     }
     for (int i = 0; i < 32; i++) p[head_w + i] = (float)(0.1 * std::sqrt(1.0 / 32) * normal(s));
     NCHK(hipMemcpy(p32, p.data(), pbytes, hipMemcpyHostToDevice));
-    nn::to_bf16(stream, nparam, p32, pb);
+    nn::to_bf16(stream, weights, nparam, p32, pb);
     NCHK(hipStreamSynchronize(stream));
     return STM_OK;
 }
@@ -335,7 +340,7 @@ int Net::train_step(int nb, float lr) {
     nn::loss(stream, y, target, mask, denom, gy, loss, (int64_t)H * W, nb, splitk);
     backward(nb);
     adam_step++;
-    nn::adam(stream, nparam, p32, g32, m32, v32, pb, lr, 0.9f, 0.999f, 1e-8f, adam_step, 1.0f);
+    nn::adam(stream, weights, nparam, p32, g32, m32, v32, pb, lr, 0.9f, 0.999f, 1e-8f, adam_step, 1.0f);
     return STM_OK;
 }
 
@@ -439,7 +444,7 @@ int stm_net_set_params(stm_net* n, const float* in) {
     std::string& err = n->net.err;
     Net& net = n->net;
     NCHK(hipMemcpyAsync(net.p32, in, sizeof(float) * net.nparam, hipMemcpyHostToDevice, net.stream));
-    nn::to_bf16(net.stream, net.nparam, net.p32, net.pb);
+    nn::to_bf16(net.stream, net.weights, net.nparam, net.p32, net.pb);
     NCHK(hipStreamSynchronize(net.stream));
     return STM_OK;
 }
