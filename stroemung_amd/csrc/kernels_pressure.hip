@@ -8,6 +8,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "kernels.h"
 #include "stm_internal.h"
@@ -395,12 +396,13 @@ constexpr int LEX_FEW = 2;
 // anti-diagonals x + y = const in increasing order, with a barrier between
 // them, reproduces exactly those reads, so the result is bit-identical.
 //
-// A channel that fits LEX_LDS_CELLS (it has at most 8 columns then) is staged
-// in LDS once, iterated there and written back: the same operations on the
-// same values in the same order.  The first wave sweeps alone, a lane per cell
-// of a diagonal: a wave's LDS accesses complete in order, so it needs no
-// workgroup barrier between diagonals (the wavefront-scope fence keeps the
-// compiler from reordering).
+// A channel that fits LEX_LDS_CELLS is staged in LDS once, iterated there and
+// written back: the same operations on the same values in the same order.  The
+// first wave sweeps alone, a lane per cell of a diagonal: a wave's LDS accesses
+// complete in order, so it needs no workgroup barrier between diagonals (the
+// wavefront-scope fence keeps the compiler from reordering).  Three sizes (67 x
+// 67, 67 x 68, 68 x 67) have a diagonal of 65 cells and a loop over it, which in
+// the others' sweeps cost 7% of a solve of one sweep (102 x 22 cells).
 __global__ void __launch_bounds__(1024)
 k_lex_solve(const ChanDesc* __restrict__ cd, ChanState* __restrict__ cs,
             const BEntry* __restrict__ be, const uint8_t* __restrict__ flags,
@@ -443,22 +445,30 @@ k_lex_solve(const ChanDesc* __restrict__ cd, ChanState* __restrict__ cs,
             }
             __syncthreads();
             if (tid < 64) {
-                for (int dd = 2; dd <= nxi + nyi; dd++) {
-                    const int xlo = dd - nyi > 1 ? dd - nyi : 1;
-                    const int xhi = dd - 1 < nxi ? dd - 1 : nxi;
-                    const int x = xlo + tid;
-                    if (x <= xhi) {
-                        // the flag and the values are read together (an
-                        // interior cell's neighbours are all in the
-                        // channel); only a fluid cell stores its update
-                        const int l = x * ny + (dd - x);
-                        const uint8_t f = sfl[l];
-                        const double nv = lex_update(d, sp[l], sp[l + ny], sp[l - ny],
-                                                     sp[l + 1], sp[l - 1], srhs[l]);
-                        if (flag_fluid(f)) sp[l] = nv;
+                // the flag and the values are read together (an interior
+                // cell's neighbours are all in the channel); only a fluid
+                // cell stores its update
+                auto cell = [&](int x, int dd) {
+                    const int l = x * ny + (dd - x);
+                    const uint8_t f = sfl[l];
+                    const double nv = lex_update(d, sp[l], sp[l + ny], sp[l - ny],
+                                                 sp[l + 1], sp[l - 1], srhs[l]);
+                    if (flag_fluid(f)) sp[l] = nv;
+                };
+                auto diagonals = [&](auto wide) {
+                    for (int dd = 2; dd <= nxi + nyi; dd++) {
+                        const int xlo = dd - nyi > 1 ? dd - nyi : 1;
+                        const int xhi = dd - 1 < nxi ? dd - 1 : nxi;
+                        if constexpr (wide.value) {
+                            for (int x = xlo + tid; x <= xhi; x += 64) cell(x, dd);
+                        } else if (xlo + tid <= xhi) {
+                            cell(xlo + tid, dd);
+                        }
+                        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
                     }
-                    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-                }
+                };
+                if (min(nxi, nyi) <= 64) diagonals(std::false_type{});
+                else diagonals(std::true_type{});
             }
             __syncthreads();
             // src/simulation.rs:216-227, as ref_norm_squared, on the LDS copy:
