@@ -54,6 +54,8 @@
 // slower).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "kernels.h"
 #include "stm_internal.h"
 
@@ -567,14 +569,15 @@ constexpr int LIGHT_MOST = 256;   // sweeps of a LIGHT batch
 template <int CLASS, int LW, int RPL, int NSLOT, int TS>
 __global__ void __launch_bounds__(256)
 k_lex_init(const ChanDesc* __restrict__ cd, const int64_t* __restrict__ work_off,
-           double* __restrict__ work)
+           double* __restrict__ work, uint32_t per)   // per: workgroups of a channel
 {
     using P = Pipe<LW, RPL, NSLOT, TS>;
-    const ChanDesc& d = cd[blockIdx.y];
+    const uint32_t c = blockIdx.x / per, part = blockIdx.x - c * per;
+    const ChanDesc& d = cd[c];
     if (d.lex_class != CLASS) return;
     const uint32_t cells = (uint32_t)(d.nx + d.ny - 1 + 2 * LEX_PAD) * P::ROW;
-    char* codes = reinterpret_cast<char*>(work + work_off[blockIdx.y]) + (4 + TS) * (uint64_t)cells * 8;
-    for (uint32_t k = blockIdx.x * 256 + threadIdx.x; k < cells; k += gridDim.x * 256)
+    char* codes = reinterpret_cast<char*>(work + work_off[c]) + (4 + TS) * (uint64_t)cells * 8;
+    for (uint32_t k = part * 256 + threadIdx.x; k < cells; k += per * 256)
         *P::code_place(codes, k / P::ROW, k % P::ROW) =
             (uint16_t)P::code(make_flag(T_NOSLIP, E_NONE), (int)(k % P::ROW), false);
 }
@@ -739,8 +742,12 @@ const int N_LEX_CLASSES = sizeof(LEX_CLASSES) / sizeof(LEX_CLASSES[0]);
 
 void launch_lex_init(hipStream_t st, int cls, int nchan, const ChanDesc* cd,
                      const int64_t* work_off, double* work) {
+    const uint32_t per = (uint32_t)std::max(1, std::min(16, 65536 / nchan));
 #define L_CASE(c, LW, RPL, NSLOT, TS)                                                          \
-    case c: k_lex_init<c, LW, RPL, NSLOT, TS><<<dim3(16, nchan), 256, 0, st>>>(cd, work_off, work); break;
+    case c:                                                                                   \
+        k_lex_init<c, LW, RPL, NSLOT, TS><<<per * (uint32_t)nchan, 256, 0, st>>>(cd, work_off, work, \
+                                                                              per);           \
+        break;
     switch (cls) {
         STM_LEX_CLASSES(L_CASE)
     default: break;

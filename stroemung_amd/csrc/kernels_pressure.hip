@@ -289,13 +289,14 @@ __device__ double ref_norm_squared(const ChanDesc& d, const double* __restrict__
 __global__ void __launch_bounds__(256)
 k_norm_squares(const ChanDesc* __restrict__ cd, const ChanState* __restrict__ cs,
                const double* __restrict__ rhs, const double* __restrict__ p,
-               double* __restrict__ sq)
+               double* __restrict__ sq, uint32_t per)   // per: workgroups of a channel
 {
-    if (cs[blockIdx.y].has_init) return;
-    const ChanDesc& d = cd[blockIdx.y];
+    const uint32_t c = blockIdx.x / per, part = blockIdx.x - c * per;
+    if (cs[c].has_init) return;
+    const ChanDesc& d = cd[c];
     const int nxi = d.nx - 2, nyi = d.ny - 2;
     const int64_t n = (int64_t)nxi * nyi, P = d.pitch;
-    for (int64_t k = blockIdx.x * 256 + threadIdx.x; k < n; k += (int64_t)gridDim.x * 256) {
+    for (int64_t k = part * 256 + threadIdx.x; k < n; k += (int64_t)per * 256) {
         const int64_t i = d.off + (1 + k / nyi) * P + 1 + k % nyi;
         sq[d.off + k] = ref_residual_sq(p, rhs, i, P, d.delx2, d.dely2);
     }
@@ -572,8 +573,9 @@ void launch_solve_begin(hipStream_t st, int nchan, const ChanDesc* cd, ChanState
 void launch_initial_norm(hipStream_t st, int nchan, const ChanDesc* cd, ChanState* cs,
                          const double* rhs, const double* p, double* scratch) {
     // four workgroups a CU over all channels, each with a few cells a thread
-    k_norm_squares<<<dim3((unsigned)std::max(1, 1024 / nchan), nchan), 256, 0, st>>>(cd, cs, rhs, p,
-                                                                                scratch);
+    // (in x, whose grids are not limited to 65536)
+    const uint32_t per = (uint32_t)std::max(1, 1024 / nchan);
+    k_norm_squares<<<per * (uint32_t)nchan, 256, 0, st>>>(cd, cs, rhs, p, scratch, per);
     k_initial_norm<<<nchan, 64 * NORM_WAVES, 0, st>>>(cd, cs, scratch);
 }
 void launch_lex_solve(hipStream_t st, int nchan, const ChanDesc* cd, ChanState* cs,
