@@ -49,6 +49,7 @@ struct HostChan {
     int32_t tile0 = 0, ntiles = 0, boff = 0;
     int32_t tb0 = 0, ntb = 0;      // blocked-solver tiles of the current variant
     int32_t lex = -1;              // instance of the pipelined lexicographic solve, -1: none
+    bool lex_part = false;         // has its part of that solve's scratch
 };
 
 struct KStat {
@@ -77,6 +78,7 @@ struct stm_ctx {
     double* scratch = nullptr;
     bool lex_few = false;          // see stage_lex
     double* lexwork = nullptr;     // pipelined lexicographic solve: its channels' scratch
+    bool lex_ready = false;        // every lexicographic channel has its part, or none is to be had
     int64_t* d_lexoff = nullptr;   // ... and each channel's offset in it
     double* p2 = nullptr;          // second pressure buffer of the blocked solver
     uint8_t* flags = nullptr;
@@ -1100,32 +1102,45 @@ int check_net(stm_ctx* ctx, stm_net* net, uint32_t f) {
     return STM_OK;
 }
 
-// Scratch of the pipelined lexicographic solve, made at the first solve that
-// has a lexicographic channel: every channel that fits an instance has its
-// part (a channel may switch solvers later).
+// Scratch of the pipelined lexicographic solve: a part for every channel that
+// fits an instance and is lexicographic (or has been).  Made at the first solve
+// that has one, and anew after another channel has become lexicographic.  It can be
+// many times the fields (18 MB for a channel of 3 x 512 cells), so it takes at
+// most half of the memory that is free: the rest is other contexts' and the
+// networks'.
 int lex_buffers(stm_ctx* ctx) {
-    if (ctx->lexwork) return STM_OK;
+    if (ctx->lex_ready) return STM_OK;
     std::vector<int64_t> off;
     int64_t n = 0;
-    for (const HostChan& c : ctx->chans) {
+    for (HostChan& c : ctx->chans) {
         off.push_back(n);
-        n += round_up(lex_work_doubles(c.lex, (int)c.nx, (int)c.ny), 16);
+        c.lex_part = c.lex_part || c.prm.solver == STM_SOLVER_LEX;
+        if (c.lex_part) n += round_up(lex_work_doubles(c.lex, (int)c.nx, (int)c.ny), 16);
     }
-    if (n == 0) return STM_OK;
-    if (!ctx->d_lexoff) HIPCHK(ctx, hipMalloc(&ctx->d_lexoff, sizeof(int64_t) * off.size()));
-    HIPCHK(ctx, hipMemcpyAsync(ctx->d_lexoff, off.data(), sizeof(int64_t) * off.size(),
-                               hipMemcpyHostToDevice, ctx->stream));
-    HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
-    if (hipMalloc(&ctx->lexwork, sizeof(double) * (size_t)n) != hipSuccess) {
-        // no memory for it: k_lex_solve takes every channel, in the fields alone
-        (void)hipGetLastError();
-        ctx->lexwork = nullptr;
-        for (HostChan& c : ctx->chans) c.lex = -1;
-        return upload_descs(ctx);
+    if (ctx->lexwork) HIPCHK(ctx, hipFree(ctx->lexwork));
+    ctx->lexwork = nullptr;
+    if (n > 0) {
+        const size_t bytes = sizeof(double) * (size_t)n;
+        if (!ctx->d_lexoff) HIPCHK(ctx, hipMalloc(&ctx->d_lexoff, sizeof(int64_t) * off.size()));
+        HIPCHK(ctx, hipMemcpyAsync(ctx->d_lexoff, off.data(), sizeof(int64_t) * off.size(),
+                                   hipMemcpyHostToDevice, ctx->stream));
+        HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
+        size_t free_bytes = 0, all_bytes = 0;
+        HIPCHK(ctx, hipMemGetInfo(&free_bytes, &all_bytes));
+        if (bytes > free_bytes / 2 || hipMalloc(&ctx->lexwork, bytes) != hipSuccess) {
+            // no memory for it: k_lex_solve takes every channel, in the fields alone
+            (void)hipGetLastError();
+            ctx->lexwork = nullptr;
+            for (HostChan& c : ctx->chans) c.lex = -1;
+            const int rc = upload_descs(ctx);
+            if (rc) return rc;
+        } else {
+            launch_fill(ctx->stream, n, ctx->lexwork, 0.0);
+            for (int k = 0; k < N_LEX_CLASSES; k++)
+                launch_lex_init(ctx->stream, k, nch(ctx), ctx->d_cd, ctx->d_lexoff, ctx->lexwork);
+        }
     }
-    launch_fill(ctx->stream, n, ctx->lexwork, 0.0);
-    for (int k = 0; k < N_LEX_CLASSES; k++)
-        launch_lex_init(ctx->stream, k, nch(ctx), ctx->d_cd, ctx->d_lexoff, ctx->lexwork);
+    ctx->lex_ready = true;
     return check_launch(ctx);
 }
 
@@ -1615,6 +1630,7 @@ int stm_set_params(stm_ctx* ctx, uint32_t ch, const stm_params* params) {
     if (params->check_every != ctx->chans[0].prm.check_every && ctx->chans.size() > 1)
         return fail(ctx, STM_ERR_INVALID_ARG, "all channels must share check_every");
     const bool new_k = params->check_every != ctx->chans[ch].prm.check_every;
+    if (params->solver == STM_SOLVER_LEX && !ctx->chans[ch].lex_part) ctx->lex_ready = false;
     ctx->chans[ch].prm = *params;
     update_solvers(ctx);
     if (!ctx->finalized) return STM_OK;

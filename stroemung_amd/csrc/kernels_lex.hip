@@ -574,7 +574,7 @@ k_lex_init(const ChanDesc* __restrict__ cd, const int64_t* __restrict__ work_off
     using P = Pipe<LW, RPL, NSLOT, TS>;
     const uint32_t c = blockIdx.x / per, part = blockIdx.x - c * per;
     const ChanDesc& d = cd[c];
-    if (d.lex_class != CLASS) return;
+    if (d.solver != SOLVER_LEX || d.lex_class != CLASS) return;
     const uint32_t cells = (uint32_t)(d.nx + d.ny - 1 + 2 * LEX_PAD) * P::ROW;
     char* codes = reinterpret_cast<char*>(work + work_off[c]) + (4 + TS) * (uint64_t)cells * 8;
     for (uint32_t k = part * 256 + threadIdx.x; k < cells; k += per * 256)
