@@ -53,7 +53,9 @@ struct Net {
     nn::bf16* pb = nullptr;      // bf16 copy of the parameters (weights packed)
     nn::WeightList weights;      // where the layers' weights are
     nn::bf16* wflip = nullptr;   // the backward-input weights of every layer, as pb
-    // partial sums of the layers' gradients (weights, bias), each at its layer's offset
+    // partial sums of the layers' gradients (weights, bias; one allocation), each at
+    // its layer's offset: 87 MB for 32 frames of 64 x 64 (made by train_buffers, so
+    // that a network that only infers does without)
     float *gpart = nullptr, *bpart = nullptr;
     // FP32 partial sums: one slice per split of a split-K convolution in the
     // forward pass, the per-block sums of the head's and the loss' reductions in
@@ -94,6 +96,7 @@ struct Net {
     void forward_infer(int nb, const int* live = nullptr);
     void backward(int nb);
     int train_step(int nb, float lr);
+    int train_buffers();           // what the backward pass needs, before the first one
 };
 
 }  // namespace stm

@@ -108,16 +108,6 @@ int Net::init(stm_ctx* c, int H_, int W_, int cap_, uint64_t seed) {
     NCHK(hipMemset(v32, 0, pbytes));
     NCHK(hipMemset(g32, 0, pbytes));
     NCHK(hipMalloc(&wflip, sizeof(bf16) * nparam));
-    int64_t ngrad = 0, nbias = 0;
-    for (auto& cv : convs) {
-        const int64_t np = (int64_t)cap * h(cv.level) * w(cv.level);
-        cv.poff = ngrad;
-        cv.bpoff = nbias;
-        ngrad += nn::dw_partials(cv.cin, cv.cout, np);
-        nbias += nn::bias_partials(cv.cout, np);
-    }
-    NCHK(hipMalloc(&gpart, sizeof(float) * (size_t)std::max<int64_t>(ngrad, 1)));
-    NCHK(hipMalloc(&bpart, sizeof(float) * (size_t)nbias));
     // the largest conv output is level 0's: cap x H x W x 32 (levels below have
     // a quarter of the pixels and twice the channels)
     scratch_floats = std::max(splitk_cap(), nn::loss_partials((int64_t)H * W, cap, 32));
@@ -159,8 +149,26 @@ int Net::init(stm_ctx* c, int H_, int W_, int cap_, uint64_t seed) {
     return STM_OK;
 }
 
+int Net::train_buffers() {
+    if (gpart) return STM_OK;
+    int64_t ngrad = 0, nbias = 0;
+    for (auto& cv : convs) {
+        const int64_t np = (int64_t)cap * h(cv.level) * w(cv.level);
+        cv.poff = ngrad;
+        cv.bpoff = nbias;
+        ngrad += nn::dw_partials(cv.cin, cv.cout, np);
+        nbias += nn::bias_partials(cv.cout, np);
+    }
+    ngrad = (ngrad + 3) / 4 * 4;   // the bias' follow, 16-byte aligned
+    float* both = nullptr;
+    NCHK(hipMalloc(&both, sizeof(float) * (size_t)(ngrad + nbias)));
+    gpart = both;
+    bpart = both + ngrad;
+    return STM_OK;
+}
+
 void Net::release() {
-    void* bufs[] = {p32, g32, m32, v32, pb, wflip, gpart, bpart, splitk, y, gy, target, mask, denom, loss,
+    void* bufs[] = {p32, g32, m32, v32, pb, wflip, gpart, splitk, y, gy, target, mask, denom, loss,
                     d_idx, dx, dt, host_in};
     for (void* b : bufs)
         if (b) hipFree(b);
@@ -333,7 +341,8 @@ void Net::backward(int nb) {
     nn::grad_finish(stream, grads, gpart, bpart, g32);
 }
 
-// One Adam step on the batch already in acts[0].v / target / mask.
+// One Adam step on the batch already in acts[0].v / target / mask (train_buffers
+// has been called).
 int Net::train_step(int nb, float lr) {
     NCHK(hipMemsetAsync(g32, 0, sizeof(float) * nparam, stream));
     forward(nb);
@@ -486,6 +495,10 @@ int stm_net_gradients(stm_net* n, uint32_t nb, const float* x, const float* t, f
     net.forward((int)nb);
     nn::loss(net.stream, net.y, net.target, net.mask, net.denom, net.gy, net.loss,
              (int64_t)net.H * net.W, (int)nb, net.splitk);
+    if (int rc = net.train_buffers()) {   // (here: a first allocation while the forward pass runs)
+        hipStreamSynchronize(net.stream);
+        return rc;
+    }
     net.backward((int)nb);
     hipMemcpyAsync(loss, net.loss, sizeof(float), hipMemcpyDeviceToHost, net.stream);
     return ctx_download(net.ctx, grads, net.g32, sizeof(float) * net.nparam)
@@ -506,7 +519,7 @@ int stm_net_dataset_reserve(stm_net* n, uint32_t capacity) {
     net.dcap = (int)capacity;
     net.dsize = 0;
     net.dwrite = 0;
-    return STM_OK;
+    return net.train_buffers();   // (the samples are there to be trained on)
 }
 
 int stm_net_dataset_size(stm_net* n, uint32_t* size) {
@@ -538,6 +551,7 @@ int stm_net_train(stm_net* n, uint32_t steps, uint32_t batch, float lr, uint64_t
     std::string& err = net.err;
     if ((int)batch > net.cap) return fail_net(n, STM_ERR_INVALID_ARG, "batch larger than capacity");
     if (net.dsize < (int)batch) return fail_net(n, STM_ERR_STATE, "dataset smaller than a batch");
+    if (int rc = net.train_buffers()) return rc;
     const int64_t hw = (int64_t)net.H * net.W;
     uint64_t s = seed;
     std::vector<int32_t> idx(batch);
@@ -582,6 +596,8 @@ int stm_net_benchmark(stm_net* n, uint32_t nb, uint32_t reps, double* fwd_ms, do
     Net& net = n->net;
     std::string& err = net.err;
     if ((int)nb > net.cap) return fail_net(n, STM_ERR_INVALID_ARG, "batch larger than capacity");
+    if (train_ms)
+        if (int rc = net.train_buffers()) return rc;
     hipEvent_t e0, e1, e2;
     NCHK(hipEventCreate(&e0));
     NCHK(hipEventCreate(&e1));
