@@ -501,8 +501,13 @@ int stm_net_gradients(stm_net* n, uint32_t nb, const float* x, const float* t, f
     }
     net.backward((int)nb);
     hipMemcpyAsync(loss, net.loss, sizeof(float), hipMemcpyDeviceToHost, net.stream);
-    return ctx_download(net.ctx, grads, net.g32, sizeof(float) * net.nparam)
-               ? fail_net(n, STM_ERR_HIP, stm_last_error(net.ctx)) : STM_OK;
+    if (net.ctx)
+        return ctx_download(net.ctx, grads, net.g32, sizeof(float) * net.nparam)
+                   ? fail_net(n, STM_ERR_HIP, stm_last_error(net.ctx)) : STM_OK;
+    // (its context is gone, and the staging buffer with it)
+    NCHK(hipMemcpyAsync(grads, net.g32, sizeof(float) * net.nparam, hipMemcpyDeviceToHost, net.stream));
+    NCHK(hipStreamSynchronize(net.stream));
+    return STM_OK;
 }
 
 int stm_net_dataset_reserve(stm_net* n, uint32_t capacity) {
