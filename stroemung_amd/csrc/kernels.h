@@ -48,8 +48,11 @@ void launch_ghost(hipStream_t, int nbtot, const BEntry*, const ChanState*, doubl
 void launch_rhs_stats(hipStream_t, int ntiles, int nchan, const ChanDesc*, ChanState*,
                       const Tile*, const uint8_t* flags, const double* rhs, double* part);
 // The same and launch_solve_begin in one launch, for channels of at most
-// STATS_TILES tiles each.
-constexpr int STATS_TILES = 256;
+// STATS_TILES tiles each: four for each of a workgroup's waves.  The four launches
+// take 66 or 88 us of a solve without sweeps, as the host is quick or slow to
+// launch, whatever the size; the one takes 58 to 79 (16 tiles), 65 to 77 (64), 78 to
+// 80 (120), 83 to 86 (144) and 108 to 110 (256).
+constexpr int STATS_TILES = 64;
 void launch_solve_stats(hipStream_t, int nchan, const ChanDesc*, ChanState*, const Tile*,
                         const uint8_t* flags, const double* rhs, int32_t* active);
 void launch_solve_begin(hipStream_t, int nchan, const ChanDesc*, ChanState*, const double* part,

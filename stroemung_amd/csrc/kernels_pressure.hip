@@ -152,6 +152,7 @@ k_solve_stats(const ChanDesc* __restrict__ cd, ChanState* __restrict__ cs,
               const double* __restrict__ rhs, int32_t* __restrict__ active_out)
 {
     static_assert(TILE_X == 4 && TILE_Y == 64, "a lane's four cells");
+    static_assert(STATS_TILES <= 64, "a tile a lane in the fold");
     __shared__ double part[STATS_TILES], total;
     const ChanDesc& d = cd[blockIdx.x];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -175,7 +176,7 @@ k_solve_stats(const ChanDesc* __restrict__ cd, ChanState* __restrict__ cs,
         __syncthreads();
         if (wave == 0) {
             auto at = [&](int k) { return k < d.ntiles ? 0.0 + part[k] : 0.0; };
-            const double s = wave_tree((at(lane) + at(lane + 128)) + (at(lane + 64) + at(lane + 192)));
+            const double s = wave_tree(at(lane));
             if (lane == 0) total = s;
         }
         __syncthreads();
