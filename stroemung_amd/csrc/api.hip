@@ -283,6 +283,7 @@ ChanDesc make_desc(const HostChan& c) {
     d.tb0 = c.tb0;
     d.ntb = c.ntb;
     d.lex_class = c.lex;
+    d.lex_begin = lex_begin(c.lex, (int)c.nx, (int)c.ny);
     d.delx = q.delx;
     d.dely = q.dely;
     d.gamma = q.gamma;
@@ -1145,8 +1146,8 @@ int lex_buffers(stm_ctx* ctx) {
 }
 
 // The lexicographic channels: a launch per class in use.  The kernel in front of
-// them is launched if it has channels of its own or if, when the states were last
-// read, some channel's solve was one that it begins (it decides on the present
+// them is launched if it has channels of its own or if, by the states as they were
+// last read, some channel's solve is one that it begins (it decides on the present
 // state; without it the pipelined solve takes them all).
 int stage_lex(stm_ctx* ctx) {
     int rc = lex_buffers(ctx);
@@ -1223,9 +1224,10 @@ int read_states(stm_ctx* ctx) {
     ctx->lex_few = false;
     for (int k = 0; k < nch(ctx); k++) {
         const HostChan& c = ctx->chans[k];
-        ctx->lex_few = ctx->lex_few || (c.prm.solver == STM_SOLVER_LEX &&
-                                        lex_few((int)(c.nx * c.ny), ctx->h_cs[k].sor_iters,
-                                                ctx->h_cs[k].exhausted));
+        ctx->lex_few = ctx->lex_few ||
+                       (c.prm.solver == STM_SOLVER_LEX &&
+                        lex_few(lex_begin(c.lex, (int)c.nx, (int)c.ny), (int)c.prm.max_iterations,
+                                ctx->h_cs[k]));
     }
     return check_launch(ctx);
 }

@@ -59,12 +59,19 @@ void launch_solve_begin(hipStream_t, int nchan, const ChanDesc*, ChanState*, con
                         int32_t* active);
 void launch_initial_norm(hipStream_t, int nchan, const ChanDesc*, ChanState*, const double* rhs,
                          const double* p, double* scratch);
-// Does launch_lex_solve begin the solve of a channel that the pipelined solve
-// takes too?  (cells, ring included; how its last solve ended)
-constexpr int LEX_LDS_CELLS = 4608;
-__host__ __device__ inline bool lex_few(int cells, uint32_t last_sweeps, int32_t exhausted) {
-    return cells <= LEX_LDS_CELLS && last_sweeps == 1 && !exhausted;
+// Does launch_lex_solve begin a solve that the pipelined one takes too?  If it is
+// expected to take at most `begin` sweeps (lex_begin): its limit, or what the channel's
+// last solve took if that met the stopping rule.  Two for the LEX_EXACT solves after
+// one in which the pipeline found values that its quotient is not right for, and did
+// its sweeps twice (a pressure that falls off to nothing in a long channel: ticks of
+// one sweep of 768 x 64 cells 1.6 times as long, of 768 x 256 2.1 times).
+constexpr int LEX_EXACT = 16;
+__host__ __device__ inline bool lex_few(int begin, int itermax, const ChanState& s) {
+    const int e = s.sor_iters == 0 || s.exhausted || s.sor_iters > (uint32_t)itermax
+                      ? itermax : (int)s.sor_iters;
+    return e > 0 && e <= (s.lex_exact > 0 ? 2 : begin);
 }
+constexpr int LEX_LDS_CELLS = 4608;   // channels of up to so many cells are solved in LDS there
 void launch_lex_solve(hipStream_t, int nchan, const ChanDesc*, ChanState*, const BEntry*,
                       const uint8_t* flags, const double* rhs, double* p, double* scratch);
 
@@ -73,10 +80,12 @@ struct LexClass {
     int row;        // most rows (ring included) a channel of the class has
     int full;       // sweeps whose squares are kept at once
     int codes;      // bytes of a diagonal's codes
+    int rows_lane;  // rows of a lane
 };
 extern const LexClass LEX_CLASSES[];
 extern const int N_LEX_CLASSES;
 int lex_class(int nx, int ny);
+int lex_begin(int cls, int nx, int ny);
 int64_t lex_work_doubles(int cls, int nx, int ny);   // scratch of one channel
 // What the scratch of class `cls` holds where there is no cell (the rest zeroed before).
 void launch_lex_init(hipStream_t, int cls, int nchan, const ChanDesc*, const int64_t* work_off,

@@ -555,6 +555,22 @@ int lex_class(int nx, int ny) {
     return -1;
 }
 
+// The most sweeps of a solve that k_lex_solve begins (0: none), which has no fields
+// to set up and goes through a diagonal with the whole workgroup.  One sweep in LDS is
+// always the faster there.  In the fields it is while they are small where a lane here
+// has four rows, whose step is the longer one: a tick of one sweep there over here, 64
+// rows of 96, 192 and 384 cells 0.88, 0.91 and 1.00, 128 of 48, 96 and 192 0.87, 0.93
+// and 1.01, 256 of 24, 48 and 192 0.82, 0.85 and 0.96 (224 rows 1.06); with three rows
+// 0.97 to 1.25.  With eight rows it is for two sweeps as well: ticks of one 0.28 to
+// 0.70; solves of 502 x 62 cells in one sweep 585 and 1055 us, in two 1049 and 1451,
+// in three 1569 and 1548.
+int lex_begin(int cls, int nx, int ny) {
+    if (cls < 0) return 0;
+    const int rows = LEX_CLASSES[cls].rows_lane;
+    if (rows >= 8) return 2;
+    return (int64_t)nx * ny <= (rows == 4 ? 3 : 1) * LEX_LDS_CELLS ? 1 : 0;
+}
+
 // A, B, C, rhs, the squares of the FULL sweeps, the codes.
 int64_t lex_work_doubles(int cls, int nx, int ny) {
     if (cls < 0) return 0;
@@ -714,6 +730,7 @@ k_lex_pipe(const ChanDesc* __restrict__ cd, ChanState* __restrict__ cs,
         s.sor_iters = (uint32_t)iters;
         s.norm2 = norm2;
         s.exhausted = exhausted;
+        s.lex_exact = exact ? LEX_EXACT : 0;
         s.active = 0;
     }
 }
@@ -735,7 +752,7 @@ k_lex_pipe(const ChanDesc* __restrict__ cd, ChanState* __restrict__ cs,
     V(6, 64, 4, 8, 8)      \
     V(7, 64, 8, 4, 4)
 
-#define L_ENTRY(c, LW, RPL, NSLOT, TS) {LW * RPL, TS, LW * 4 * code_words(RPL)},
+#define L_ENTRY(c, LW, RPL, NSLOT, TS) {LW * RPL, TS, LW * 4 * code_words(RPL), RPL},
 const LexClass LEX_CLASSES[] = {STM_LEX_CLASSES(L_ENTRY)};
 #undef L_ENTRY
 const int N_LEX_CLASSES = sizeof(LEX_CLASSES) / sizeof(LEX_CLASSES[0]);

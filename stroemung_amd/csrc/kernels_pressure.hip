@@ -383,23 +383,23 @@ __device__ __forceinline__ double lex_update(const ChanDesc& d, double pc, doubl
     return (d.omw * pc) + (d.mid * ((((pxp + pxm) / d.delx2) + ((pyp + pym) / d.dely2)) - r));
 }
 
-// Channels of at most LEX_LDS_CELLS cells (ring included) solve with p, rhs, the
-// flags and the norm's terms in LDS (115 KB).
+// The most sweeps that k_lex_solve does of a solve that the pipeline can go on with.
 constexpr int LEX_FEW = 2;
 
 // src/simulation.rs:239-285 for the channels with solver == SOLVER_LEX that no
-// instance of the pipelined solve takes (kernels_lex.hip: more than 512 rows), and
-// the first LEX_FEW sweeps of channels in LDS whose last solve took one: the
-// pipeline's set-up (its diagonal-major copies) and its longer step pay from the
-// second or third sweep on.  A solve (statistics included) of 102 x 22 cells in
-// one sweep: 73 us here, 87 there; in two 113 and 88, in four 196 and 90.
+// instance of the pipelined solve takes (kernels_lex.hip: more than 512 rows, or no
+// scratch for them), and the first LEX_FEW sweeps of solves that are expected to be
+// short (lex_few, lex_begin): the pipeline's set-up (its diagonal-major copies) and
+// its longer step pay from the second or third sweep on.  A solve (statistics
+// included) of 102 x 22 cells in one sweep: 73 us here, 87 there; in two 113 and 88,
+// in four 196 and 90.
 // Lexicographic Gauss-Seidel order (x outer, y inner, in place) makes cell
 // (x, y) read the new W and N values and the old E and S values; sweeping the
 // anti-diagonals x + y = const in increasing order, with a barrier between
 // them, reproduces exactly those reads, so the result is bit-identical.
 //
-// A channel that fits LEX_LDS_CELLS is staged in LDS once, iterated there and
-// written back: the same operations on the same values in the same order.  The
+// A channel that fits LEX_LDS_CELLS is staged in LDS once (p, rhs, the flags and the
+// norm's terms, 115 KB), iterated there and written back: the same operations on the same values in the same order.  The
 // first wave sweeps alone, a lane per cell of a diagonal: a wave's LDS accesses
 // complete in order, so it needs no workgroup barrier between diagonals (the
 // wavefront-scope fence keeps the compiler from reordering).  Three sizes (67 x
@@ -417,7 +417,7 @@ k_lex_solve(const ChanDesc* __restrict__ cd, ChanState* __restrict__ cs,
     if (d.solver != SOLVER_LEX) return;
     ChanState& s = cs[blockIdx.x];
     const bool few = d.lex_class >= 0;
-    if (few && !lex_few(d.nx * d.ny, s.sor_iters, s.exhausted)) return;
+    if (few && !lex_few(d.lex_begin, d.itermax, s)) return;
     const int limit = few ? min(d.itermax, LEX_FEW) : d.itermax;
     const int nxi = d.nx - 2, nyi = d.ny - 2;
     const int64_t P = d.pitch;
@@ -503,6 +503,7 @@ k_lex_solve(const ChanDesc* __restrict__ cd, ChanState* __restrict__ cs,
         }
         if (tid == 0) {
             s.budget = -1;
+            s.lex_exact -= s.lex_exact > 0;
             s.sor_iters = (uint32_t)iters;
             s.norm2 = norm2;
             s.exhausted = exhausted;
@@ -510,7 +511,7 @@ k_lex_solve(const ChanDesc* __restrict__ cd, ChanState* __restrict__ cs,
         }
         return;
     }
-    for (int it = 0; it < d.itermax; it++) {
+    for (int it = 0; it < limit; it++) {
         // copy_pressure_to_boundaries, src/grid/mod.rs:343-412
         for (int k = threadIdx.x; k < d.nb; k += blockDim.x) {
             const BEntry e = be[d.boff + k];
@@ -539,7 +540,13 @@ k_lex_solve(const ChanDesc* __restrict__ cd, ChanState* __restrict__ cs,
             break;
         }
     }
+    if (few && exhausted && limit < d.itermax) {
+        if (threadIdx.x == 0) s.budget = limit;
+        return;
+    }
     if (threadIdx.x == 0) {
+        s.budget = -1;
+        s.lex_exact -= s.lex_exact > 0;
         s.sor_iters = (uint32_t)iters;
         s.norm2 = norm2;
         s.exhausted = exhausted;

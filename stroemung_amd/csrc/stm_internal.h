@@ -33,7 +33,8 @@ struct ChanDesc {
     int32_t tile0, ntiles;       // slice of the tile list
     int32_t itermax, check_every;
     int32_t tb0, ntb;            // slice of the blocked-solver tile list
-    int32_t lex_class, pad;      // instance of the pipelined lexicographic solve, -1: none
+    int32_t lex_class;           // instance of the pipelined lexicographic solve, -1: none
+    int32_t lex_begin;           // see lex_few
     double delx, dely, gamma, reynolds, omega, eps, tau;
     double fluid_cells;
     double n_inner;              // interior fluid cells, x in [1, nx-2], y in [1, ny-2]
@@ -62,6 +63,7 @@ struct ChanState {
     int32_t pbuf;                // blocked solver: latest p is in the second buffer
     int32_t stop_launch;         // blocked solver: launch whose result ended the solve, -1 running
     int32_t budget;              // blocked solver: sweep limit below itermax, 0 = none
+    int32_t lex_exact;           // see lex_few
 };
 
 // Per-channel state of the learned correction (device copy in LearnChan[]).
