@@ -614,6 +614,15 @@ k_lex_pipe(const ChanDesc* __restrict__ cd, ChanState* __restrict__ cs,
     const int begun = s.budget;    // sweeps that k_lex_solve has done
     if (begun < 0) return;         // it has ended the solve
     const int tid = threadIdx.x;
+    if (d.itermax <= 0) {          // nothing to sweep: no need of the fields' copies
+        if (tid == 0) {
+            s.sor_iters = (uint32_t)d.itermax;
+            s.norm2 = 0.0;
+            s.exhausted = 1;
+            s.active = 0;
+        }
+        return;
+    }
     const int nxi = d.nx - 2, nyi = d.ny - 2;
     LexWork w;
     w.dmax = d.nx + d.ny - 2;
