@@ -7,7 +7,7 @@
 namespace stm {
 
 // Output parts of one axis of n cells for the blocked solver: region E
-// cells, halo H, part starts and region origins multiples of q (1 in x, 2 in
+// cells, halo H, part starts and region origins multiples of q (2 in x and
 // y).  A middle part has H cells of halo on both sides (at most E - 2H
 // cells).  The first part's region starts q cells before the channel and the
 // last part's region reaches past its end, where nothing feeds the tile, so
