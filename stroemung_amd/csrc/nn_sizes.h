@@ -45,13 +45,13 @@ inline int64_t bias_partials(int cout, int64_t npix) {
 
 // Partials (floats) of the weight gradient of a layer for any pixel count up to
 // npix.  The chunk counts are not monotone in the pixel count: at most 257
-// chunks until the chunk size stops growing, at most 257 bias blocks.
+// chunks until the chunk size stops growing.
 inline int64_t dw_partials(int cin, int cout, int64_t npix) {
     const int64_t chunks =
         std::min((npix + 1023) / 1024, std::max<int64_t>(257, (npix + (1 << 20) - 1) >> 20));
     return chunks > 1 ? chunks * cout * 9 * cin : 0;
 }
-// The larger of a layer's two kinds of partials.
+// The larger of a layer's two kinds of partials (no buffer is sized by it).
 inline int64_t grad_partials(int cin, int cout, int64_t npix) {
     return std::max(dw_partials(cin, cout, npix), bias_partials(cout, npix));
 }
