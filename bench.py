@@ -275,7 +275,7 @@ def sweeps_run(a):
     unique, loaded = ctx.solver_bytes()
     achieved = unique / avg_s / 1e9
     effective = SWEEP_BYTES_PER_CELL * k * n * n / avg_s / 1e9
-    working_set = (3 * 8 + 1) * (n + 2) * (n + 2)
+    working_set = 3 * 8 * (n + 2) * (n + 2)
     ctx.close()
     out = {
         "metric": "blocked red-black SOR launch, algorithmic bytes per second",
@@ -842,10 +842,11 @@ def main():
 
     kname = "rb_tb"
     kernel_id = "k_rb_strip<%s>, %d sweeps" % (VARIANT_SHAPES.get(variant, "?"), ksweeps)
-    traffic = None
+    traffic, counted = None, {}
     try:
         with open(os.path.join(ROOT, "profiles", "traffic.json")) as fh:
-            traffic = json.load(fh).get(kernel_id, {}).get("traffic_bytes_per_launch")
+            counted = json.load(fh).get(kernel_id, {})
+            traffic = counted.get("traffic_bytes_per_launch")
     except OSError:
         pass
     # batches of 8 to 64 launches queued back to back between host polls,
@@ -864,10 +865,10 @@ def main():
     unique, loaded = ctx.solver_bytes()
     achieved = unique / avg_s / 1e9 if timed else None
     effective = SWEEP_BYTES_PER_CELL * ksweeps * cells / avg_s / 1e9 if timed else None
-    working_set = (3 * 8 + 1) * (n + 2) * (n + 2)
+    working_set = 3 * 8 * (n + 2) * (n + 2)
     kernels = {}
     for k in ("rb_tb", "pbuf_fix", "solve_begin", "rhs_stats", "fg_rhs", "fg", "rhs",
-              "adap_ranges", "restore", "bc_velocity", "delt"):
+              "adap_ranges", "restore", "bc_velocity"):
         kms, kt, kl = ctx.kernel_stats(k)
         if kl:
             kernels[k] = {"launches": kl, "timed": kt,
@@ -912,9 +913,10 @@ def main():
             "frac": achieved / HBM_PEAK_GBS if achieved else None,
             "traffic": traffic,
             "traffic_source": ("FETCH_SIZE and WRITE_SIZE per working dispatch from two "
-                               "rocprofv3 --pmc runs of `bench.py --profile --variant 9`, "
-                               "scaled by a 256 MiB copy (profiles/traffic.json); not "
-                               "measured in this run" if traffic else None),
+                               "rocprofv3 --pmc runs, scaled by a 256 MiB copy "
+                               "(profiles/traffic.json: %s); not measured in this run"
+                               % counted.get("dispatches", "no dispatches named")
+                               if traffic else None),
             "bytes_per_launch": unique,
             "model": "24 B per cell per launch: p read, rhs read, p written",
             "loaded_bytes_per_launch": loaded,
@@ -926,7 +928,7 @@ def main():
             "timing": "HIP events around queued batches of 8-64 launches",
             "single_launch_event_us": sms * 1e3 / stimed if stimed else None,
             "measured_copy_gbs": copy_gbs,
-            # p, the second p buffer, rhs and flags: under the 256 MB Infinity Cache
+            # p, the second p buffer and rhs: under the 256 MB Infinity Cache
             # on this grid, so the kernel's data may stay in the MALL between launches
             "working_set_bytes": working_set,
             "cache_resident": working_set < MALL_BYTES,
