@@ -45,6 +45,7 @@ struct Net {
     stm_ctx* ctx = nullptr;
     uint64_t serial = 0;         // unique per net in the process (graph keys)
     hipStream_t stream = nullptr;
+    int device = 0;
     int H = 0, W = 0, cap = 0;   // spatial size and batch capacity
     std::vector<Conv> convs;
     std::vector<Act> acts;

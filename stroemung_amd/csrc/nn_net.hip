@@ -96,7 +96,8 @@ int Net::init(stm_ctx* c, int H_, int W_, int cap_, uint64_t seed) {
     off += 8;
     nparam = off;
 
-    NCHK(hipSetDevice(ctx_device(c)));
+    device = ctx_device(c);
+    NCHK(hipSetDevice(device));
     const size_t pbytes = sizeof(float) * nparam;
     ctx_stage(c, pbytes);   // the gradients' way out
     NCHK(hipMalloc(&p32, pbytes));
@@ -161,6 +162,7 @@ int Net::train_buffers() {
     }
     ngrad = (ngrad + 3) / 4 * 4;   // the bias' follow, 16-byte aligned
     float* both = nullptr;
+    NCHK(hipSetDevice(device));
     NCHK(hipMalloc(&both, sizeof(float) * (size_t)(ngrad + nbias)));
     gpart = both;
     bpart = both + ngrad;
