@@ -109,7 +109,7 @@ struct stm_ctx {
     int tbc_capacity = 0;
     int variant = -1;              // blocked-solver variant in use
     ChanState* h_cs = nullptr;     // pinned
-    char* h_stage = nullptr;       // pinned: field transfers, images
+    char* h_stage = nullptr;       // pinned: field transfers, a network's gradients
     size_t stage_bytes = 0;
     int be_capacity = 0;
     // learned correction and capture of training pairs

@@ -29,7 +29,7 @@
 //   LIGHT  The squares of the residual are added in order, so the sum is at
 //          least as large as any one of them (rounding is monotone): a sweep
 //          in which one square alone reaches the bound has not met the rule.
-//          A quarter of the diagonals are looked at; when every sweep of the
+//          A third of the diagonals are looked at; when every sweep of the
 //          batch shows such a square, all of them count.  The norm the solve
 //          returns, its last sweep's, is formed from the final field.
 //   FULL   Every sweep leaves all its squares (T), the norms are summed in the
@@ -49,9 +49,11 @@
 // dependent FP64 addition takes 4.6 cycles), the LDS round trip to the next slot
 // and the barrier; no memory and no unit is busy.  With up to 32 sweeps in
 // flight, three diagonals apart, a sweep costs a few steps instead of nx + ny.
-// A hundred sweeps and their norms: 102 x 22 cells 3.65 ms with one sweep at a
-// time, 0.30 now; 402 x 82 cells 54.2 ms and 2.5 (a lag of four diagonals: 8%
-// slower).
+// A solve of a hundred sweeps to its limit (LIGHT: a hundred tests, one norm
+// formed): 102 x 22 cells 3.58 ms with one sweep at a time, 0.30 now; 402 x 82 cells
+// 53.9 ms and 2.44 (a lag of four diagonals: 8% slower).  One that meets the rule at
+// the hundredth (FULL, after another such solve: a hundred norms, and what was swept
+// beyond it again): 202 x 62 cells 19.8 and 2.67 (LIGHT 1.00), 402 x 82 54.5 and 8.4.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
